@@ -395,9 +395,9 @@ int tcs_split(const void* x, int x_elem_bytes, const int8_t* mask, const int32_t
  * Radix sort
  * --------------------------------------------------------------------- */
 
-/* Workspace of tcs_sort (look-back descriptors and digit counts: zeroed
- * once, reusable like every workspace) and its scratch (one temporary copy
- * of keys and positions, any contents); 0 for an unsupported dtype. */
+/* Workspace of tcs_sort (its header: zeroed once, reusable like every
+ * workspace) and its scratch (one temporary copy of keys and positions and
+ * the digit counts, any contents); 0 for an unsupported dtype. */
 size_t tcs_sort_workspace_bytes(int64_t n, int dtype);
 size_t tcs_sort_scratch_bytes(int64_t n, int dtype);
 

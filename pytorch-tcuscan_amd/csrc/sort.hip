@@ -9,60 +9,140 @@
 // output holds the input's exact bits; the order key is recomputed from
 // them in every pass.
 //
-// Launches: one histogram pass over the keys counts the digits of every
-// digit position at once; a small kernel turns the counts into the
-// first index of each digit's bucket; then one kernel per digit position.
-// A pass kernel ranks each tile's keys by digit (per wave: one ballot per
-// digit bit gives each lane the lanes holding the same digit, so ranks are
-// stable without atomics), publishes the tile's 256 digit counts, finds
-// how many keys of each digit the tiles before it hold through a per-digit
-// decoupled look-back, reorders the tile in LDS by digit and writes each
-// digit's run contiguously.
+// The keys are cut into at most kSortMaxChunks contiguous chunks, one
+// resident workgroup each.  Every digit position is a count kernel (the 256
+// digit counts of each chunk, or of each of a chunk's parts), for many counts
+// a kernel that sums them up to each part's first output index per digit,
+// and a scatter kernel: a workgroup walks its chunk tile by tile with the
+// 256 output indices in registers, ranks a tile's keys by digit, reorders
+// the tile in LDS and writes each digit's run contiguously.  There is no
+// look-back: no tile waits for another.  At most kSortBlockMax keys are
+// sorted by one workgroup in one launch.
 #include "tcs_common.hpp"
 #include "tcs_device.hpp"
 #include "tcs_sortkey.hpp"
 
 namespace tcs {
 
-constexpr int kSortNW = 8, kSortItems = 16;
-constexpr int64_t kSortTile = (int64_t)kSortNW * kWave * kSortItems;  // 8192
-constexpr int kHistThreads = 512, kHistMaxGroups = 1024;
-constexpr int kMaxPasses = 4;
+constexpr int kSortThreads = 512;     // of a count workgroup
+constexpr int kSortNW = kSortThreads / kWave;
+constexpr int kSortMaxChunks = 512;   // scatter workgroups
+constexpr int kSortMaxRows = 1024;    // count workgroups
+constexpr int kSortFusedRows = 64;    // up to here the scatter kernel sums the counts itself
+
+// Digit of an order key (or of the order key in the low or high half of a
+// pair, with 16 added to the shift).
+__device__ __forceinline__ uint32_t sort_digit(uint32_t key, uint32_t shift) {
+  return __builtin_amdgcn_ubfe(key, shift, 8);
+}
+
+// Order keys of two consecutive rows: the pair of a 16-bit type in one word
+// (row 0 in the low half), or the two keys.  Descending order inverts every
+// key bit (flip = ~0).
+template <int DT>
+struct KeyPair {
+  using KT = SortKey<DT>;
+  static constexpr bool kPacked = KT::kBits == 16;
+  uint32_t k[kPacked ? 1 : 2];
+  __device__ __forceinline__ void set(uint32_t r0, uint32_t r1, uint32_t flip) {
+    if constexpr (kPacked) {
+      k[0] = KT::pair(r0 | (r1 << 16)) ^ flip;
+    } else {
+      k[0] = KT::key((typename KT::Raw)r0) ^ flip;
+      k[1] = KT::key((typename KT::Raw)r1) ^ flip;
+    }
+  }
+  __device__ __forceinline__ uint32_t word(int h) const { return kPacked ? k[0] : k[h]; }
+  __device__ __forceinline__ uint32_t shift(uint32_t s, int h) const { return kPacked ? s + 16u * (uint32_t)h : s; }
+};
+
+// N values of `BITS` bits, 16-bit ones two to a register.
+template <int N, int BITS>
+struct RowRegs {
+  static constexpr bool kPacked = BITS <= 16;
+  uint32_t w[kPacked ? N / 2 : N];
+  // Sets rows i and i + 1 (i even).
+  __device__ __forceinline__ void set2(int i, uint32_t a, uint32_t b) {
+    if constexpr (kPacked) {
+      w[i / 2] = a | (b << 16);
+    } else {
+      w[i] = a;
+      w[i + 1] = b;
+    }
+  }
+  __device__ __forceinline__ uint32_t get(int i) const {
+    if constexpr (kPacked) return i % 2 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu;
+    else return w[i];
+  }
+};
+
+// Counts one row into the wave's `hist` and returns the number of keys of
+// this lane's digit d that the wave has met before this key (earlier rows,
+// then lower lanes).  Eight ballots, one per digit bit from bit `at` of
+// `word`, leave in (lo, hi) the lanes of `vmask` with the same digit: a
+// sign-extended bit, its ballot and two three-input logic operations a bit.
+// A wave's LDS operations execute in order, so the rows' reads and the adds
+// of the first lane of each digit follow one another without a wait.
+__device__ __forceinline__ uint32_t sort_rank_row(uint32_t* hist, uint32_t word, uint32_t at, uint32_t d,
+                                                  bool valid, uint64_t vmask) {
+  uint32_t lo = (uint32_t)vmask, hi = (uint32_t)(vmask >> 32);
+#pragma unroll
+  for (uint32_t b = 0; b < 8; ++b) {
+    const int s = __builtin_amdgcn_sbfe((int)word, at + b, 1);
+    const uint64_t m = __ballot(s != 0);
+    lo = __builtin_amdgcn_bitop3_b32(lo, (uint32_t)m, (uint32_t)s, 0x90);          // lo & ~(m ^ s)
+    hi = __builtin_amdgcn_bitop3_b32(hi, (uint32_t)(m >> 32), (uint32_t)s, 0x90);
+  }
+  const uint32_t rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
+  uint32_t base = 0;
+  if (valid) {
+    base = __hip_atomic_load(&hist[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    if (rank == 0)
+      (void)__hip_atomic_fetch_add(&hist[d], (uint32_t)(__builtin_popcount(lo) + __builtin_popcount(hi)),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  }
+  return base + rank;
+}
 
 // ---------------------------------------------------------------------------
-// Digit counts of every pass: per-workgroup partials (no atomics in HBM),
-// then one workgroup per pass sums them in a fixed order and scans them.
+// Digit counts: counts[r * 256 + d] = keys of digit d among the `part` keys
+// from r * part.  Per
+// wave C copies of the 256 bins, lane l adding into copy l % C: lanes whose
+// keys share a digit (skewed data) then contend C times less.  Bound by the
+// read: 2^26 int32 keys 45 us (5.9 TB/s) in the first pass; the later passes'
+// counts take about 95 us, since reading what the scatter before them wrote
+// makes room in the last-level cache for which that write has to drain.
 // ---------------------------------------------------------------------------
-template <int DT>
-__global__ __launch_bounds__(kHistThreads) void sort_hist_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
-                                                                 int64_t n, int64_t chunk, uint32_t flip,
-                                                                 uint64_t* __restrict__ partial) {
-  using KT = SortKey<DT>;
-  using Raw = typename KT::Raw;
-  constexpr int P = KT::kBits / 8;
-  constexpr int NWV = kHistThreads / kWave;
+template <int DT, int C>
+__global__ __launch_bounds__(kSortThreads) void sort_count_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
+                                                                  int64_t n, int64_t part, uint32_t shift,
+                                                                  uint32_t flip, uint32_t* __restrict__ counts) {
+  using Raw = typename SortKey<DT>::Raw;
   constexpr int V = 16 / (int)sizeof(Raw);
-  // C copies of the counts per wave, lane l adding into copy l % C: lanes
-  // whose keys share a digit (skewed data) then contend C times less.
-  constexpr int C = 4 / P > 0 ? 4 / P : 1;
-  constexpr int NH = NWV * C;
+  constexpr int NH = kSortNW * C;
   // One word of padding per copy: the copies of one bin fall in different
   // LDS banks.
-  __shared__ uint32_t h[NH][P * 256 + 1];
+  __shared__ uint32_t h[NH][257];
   const int tid = threadIdx.x, wid = tid / kWave;
-  const int hc = wid * C + (__lane_id() % C);
-  for (int k = tid; k < NH * (P * 256 + 1); k += kHistThreads) (&h[0][0])[k] = 0;
+  for (int k = tid; k < NH * 257; k += kSortThreads) (&h[0][0])[k] = 0;
+  uint32_t* hc = h[wid * C + (__lane_id() % C)];
   __syncthreads();
-  const int64_t c0 = (int64_t)blockIdx.x * chunk;
-  const int64_t c1 = c0 + chunk < n ? c0 + chunk : n;
+  const int64_t c0 = (int64_t)blockIdx.x * part;
+  const int64_t c1 = c0 + part < n ? c0 + part : n;
   // Four 16-byte loads in flight per thread per step; steps that lie wholly
   // inside the chunk skip the per-element bounds checks.
   constexpr int U = 4;
-  constexpr int64_t STEP = (int64_t)kHistThreads * V;
-  auto add = [&](Raw r) {
-    const uint32_t k = KT::key(r) ^ flip;
+  constexpr int64_t STEP = (int64_t)kSortThreads * V;
+  auto add = [&](const Raw(&r)[V], auto all, int64_t left) {
+    constexpr bool ALL = decltype(all)::value;
 #pragma unroll
-    for (int p = 0; p < P; ++p) atomicAdd(&h[hc][p * 256 + ((k >> (8 * p)) & 0xffu)], 1u);
+    for (int i = 0; i < V; i += 2) {
+      KeyPair<DT> kp;
+      kp.set(r[i], r[i + 1], flip);
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        if (ALL || i + e < left) atomicAdd(&hc[sort_digit(kp.word(e), kp.shift(shift, e))], 1u);
+    }
   };
   int64_t b0 = c0 + (int64_t)tid * V;
   const int64_t full_end = c0 + ((c1 - c0) / (U * STEP)) * (U * STEP);  // steps [c0, full_end) are whole
@@ -71,257 +151,398 @@ __global__ __launch_bounds__(kHistThreads) void sort_hist_kernel(const typename 
 #pragma unroll
     for (int u = 0; u < U; ++u) load_items<Raw, V, true>(x, b0 + u * STEP, c1, r[u]);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int i = 0; i < V; ++i) add(r[u][i]);
-    }
+    for (int u = 0; u < U; ++u) add(r[u], std::integral_constant<bool, true>{}, V);
   }
   for (; b0 < c1; b0 += STEP) {
     Raw r[V];
     load_items<Raw, V, false>(x, b0, c1, r);
-#pragma unroll
-    for (int i = 0; i < V; ++i) {
-      if (b0 + i < c1) add(r[i]);
-    }
+    add(r, std::integral_constant<bool, false>{}, c1 - b0);
   }
   __syncthreads();
-  for (int e = tid; e < P * 256; e += kHistThreads) {
+  if (tid < 256) {
     uint32_t s = 0;
 #pragma unroll
-    for (int w = 0; w < NH; ++w) s += h[w][e];
-    partial[(size_t)blockIdx.x * P * 256 + e] = s;  // 64-bit: high half zero
+    for (int w = 0; w < NH; ++w) s += h[w][tid];
+    counts[(size_t)blockIdx.x * 256 + tid] = s;
   }
 }
 
-// First level of the digit-count sum: workgroup (q, p) adds pass p's
-// partials of groups [q * per, (q + 1) * per) into psum (same layout as the
-// partials, kSortSumGroups rows; 64-bit words, high half zero).
-constexpr int kSortSumGroups = 32;
-__global__ __launch_bounds__(256) void sort_sum_kernel(const uint64_t* __restrict__ partial, int groups, int per,
-                                                       int passes, uint64_t* __restrict__ psum) {
-  const int d = threadIdx.x, q = blockIdx.x, p = blockIdx.y;
-  const int g0 = q * per;
-  const int g1 = g0 + per < groups ? g0 + per : groups;
-  uint32_t s = 0;
-  int g = g0;
-  for (; g + 8 <= g1; g += 8) {  // eight loads in flight
-    uint64_t v[8];
+// In place: counts[r * 256 + d] = keys of digit d in the rows before r, and
+// totals[d] = keys of digit d.  A workgroup takes 16 digits; its threads are
+// 64 groups of kSortMaxRows / 64 consecutive rows.
+constexpr int kSortScanThreads = 1024, kSortScanDigits = 16;
+__global__ __launch_bounds__(kSortScanThreads) void sort_row_scan_kernel(uint32_t* __restrict__ counts, int rows,
+                                                                           uint32_t* __restrict__ totals) {
+  constexpr int NG = kSortScanThreads / kSortScanDigits, PER = kSortMaxRows / NG;
+  __shared__ uint32_t s_sum[kSortScanDigits][NG + 1];
+  const int q = threadIdx.x % kSortScanDigits, g = threadIdx.x / kSortScanDigits;
+  const int d = blockIdx.x * kSortScanDigits + q;
+  uint32_t v[PER], sum = 0;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = partial[((size_t)(g + u) * passes + p) * 256 + d];
+  for (int i = 0; i < PER; ++i) v[i] = g * PER + i < rows ? counts[(size_t)(g * PER + i) * 256 + d] : 0u;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) s += (uint32_t)v[u];
-  }
-  for (; g < g1; ++g) s += (uint32_t)partial[((size_t)g * passes + p) * 256 + d];
-  psum[((size_t)q * passes + p) * 256 + d] = s;
-}
-
-// gbase[p * 256 + d] = number of keys whose digit p is below d.  One
-// workgroup per pass: four threads per digit sum interleaved groups (eight
-// loads in flight each), then the 256 totals are scanned.
-constexpr int kBucketThreads = 1024;
-__global__ __launch_bounds__(kBucketThreads) void sort_bucket_kernel(const uint64_t* __restrict__ partial,
-                                                                     int groups, int passes,
-                                                                     uint64_t* __restrict__ gbase) {
-  const int p = blockIdx.x, tid = threadIdx.x, d = tid & 255, r = tid >> 8;
-  uint32_t s = 0;
-  int g = r;
-  for (; g + 28 < groups; g += 32) {
-    uint64_t v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = partial[((size_t)(g + 4 * u) * passes + p) * 256 + d];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += (uint32_t)v[u];
-  }
-  for (; g < groups; g += 4) s += (uint32_t)partial[((size_t)g * passes + p) * 256 + d];
-  __shared__ uint32_t sr[4][256];
-  __shared__ uint32_t ws[4];
-  sr[r][d] = s;
+  for (int i = 0; i < PER; ++i) sum += v[i];
+  s_sum[q][g] = sum;
   __syncthreads();
-  uint32_t t = 0, incl = 0;
-  if (tid < 256) {
-    t = sr[0][d] + sr[1][d] + sr[2][d] + sr[3][d];
-    incl = wave_incl_scan(t);
-    if (__lane_id() == kWave - 1) ws[tid / kWave] = incl;
-  }
+  // Wave w scans digit w's 64 group sums.
+  const int w = threadIdx.x / kWave, lane = __lane_id();
+  const uint32_t mine = s_sum[w][lane];
+  const uint32_t incl = wave_incl_scan(mine);
+  s_sum[w][lane] = incl - mine;
+  if (lane == kWave - 1) totals[blockIdx.x * kSortScanDigits + w] = incl;
   __syncthreads();
-  if (tid < 256) {
-    uint32_t before = 0;
-    for (int w = 0; w < tid / kWave; ++w) before += ws[w];
-    gbase[p * 256 + d] = (uint64_t)(before + incl - t);
+  uint32_t run = s_sum[q][g];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    if (g * PER + i < rows) counts[(size_t)(g * PER + i) * 256 + d] = run;
+    run += v[i];
   }
 }
 
 // ---------------------------------------------------------------------------
-// One digit position.  Tile t holds elements [t * 8192, t * 8192 + 8192):
-// wave w, item i, lane l is element t * 8192 + w * 1024 + i * 64 + l, so the
-// (item, lane) order of a wave is the input order.
+// One digit position.  Workgroup c walks its chunk in tiles of 64 NW IT keys:
+// wave w, row i, lane l is tile element w * 64 IT + i * 64 + l, so the
+// (row, lane) order of a wave is the input order (the chunk's last tile
+// takes the fewest rows a wave that hold it).  Each wave ranks its rows
+// with its own 256 counters; 256 threads turn the counters into tile
+// positions and advance the chunk's output indices, which thread d keeps in
+// a register; the tile is reordered in LDS and each digit's run written
+// contiguously, while the next tile's keys are already being loaded.
+//
+// GEN: positions are generated (the first pass without given indices); a
+// 16-bit key then shares a word with its tile-local position, and the tile
+// takes half the LDS.  BIG: 2^30 keys or more, whose outputs 32-bit byte
+// offsets do not reach.
+//
+// Bound by the write requests of the runs and by the ranking: 2^28 fp16
+// normals, first pass 0.73 ms and second 0.79 (8-wave workgroups with
+// 8192-key tiles 1.07 and 0.92; with their writes made linear 0.66 and 0.70;
+// without any write 0.50).  The look-back passes before took 1.34 and 1.25 ms.
+// Plain loads: nontemporal ones measured the same.
 // ---------------------------------------------------------------------------
-template <int DT, bool GEN_IDX>
-__global__ __launch_bounds__(kSortNW * kWave) void sort_pass_kernel(
+template <int DT, bool GEN, int NW, int IT, bool BIG>
+__global__ __launch_bounds__(NW * kWave, 4) void sort_scatter_kernel(
     const typename SortKey<DT>::Raw* __restrict__ kin, const int32_t* __restrict__ vin,
-    typename SortKey<DT>::Raw* __restrict__ kout, int32_t* __restrict__ vout, const uint64_t* __restrict__ gbase,
-    int shift, uint32_t flip, int64_t n, void* ws, uint32_t num_tiles) {
+    typename SortKey<DT>::Raw* __restrict__ kout, int32_t* __restrict__ vout, const uint32_t* __restrict__ counts,
+    const uint32_t* __restrict__ totals, int rows, int parts, uint32_t shift, uint32_t flip, int64_t n,
+    int64_t chunk) {
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
-  constexpr int NW = kSortNW, IT = kSortItems;
-  __shared__ uint32_t s_whist[NW][256];  // per wave: digit counts, then their exclusive prefix over waves
-  __shared__ uint32_t s_excl[256];       // first tile-local position of each digit
-  __shared__ int32_t s_gofs[256];        // output index of tile-local position 0 for each digit
+  constexpr int NT = NW * kWave, TILE = NT * IT;
+  constexpr bool kNarrow = KT::kBits <= 16;
+  constexpr bool kWord = GEN && kNarrow;  // key and tile-local position in one word
+  static_assert(TILE <= 65536 && IT % 2 == 0, "16-bit tile positions, rows in pairs");
+  using Item = typename std::conditional<kWord, uint32_t, uint64_t>::type;
+  __shared__ uint32_t s_whist[NW][256];  // per wave: digit counts, then the tile position of its first key per digit
+  __shared__ uint32_t s_gofs[256];       // output index of tile position 0 for each digit
   __shared__ uint32_t s_wsum[4];
-  __shared__ LaunchTag s_tag;
-  __shared__ Raw s_keys[kSortTile];
-  __shared__ int32_t s_vals[kSortTile];
-  // Digits beside the reordered keys for keys of up to 2 bytes; 4-byte keys
-  // recompute them (the extra 8 KiB would leave one workgroup per CU).
-  constexpr bool kDigLds = sizeof(Raw) <= 2;
-  __shared__ uint8_t s_dig[kDigLds ? kSortTile : 1];
+  __shared__ Item s_item[TILE];
+  // A word holds no digit beside key and position: the digits beside it, read
+  // back instead of the key's order computed again.
+  constexpr bool kDig = kWord && TILE < 32768;
+  __shared__ uint8_t s_dig[kDig ? TILE : 1];
 
   const int tid = threadIdx.x, lane = __lane_id(), wid = tid / kWave;
-  if (tid == 0) s_tag = launch_arrive(ws);
-  for (int k = tid; k < NW * 256; k += NW * kWave) (&s_whist[0][0])[k] = 0;
-  const uint32_t tile = blockIdx.x;
-  const int64_t t0 = (int64_t)tile * kSortTile;
-  const int64_t wb = t0 + (int64_t)wid * (kWave * IT);
-  auto digit_of = [&](Raw r) { return (int)(((KT::key(r) ^ flip) >> shift) & 0xffu); };
+  const int64_t c0 = (int64_t)blockIdx.x * chunk;
+  const int64_t c1 = c0 + chunk < n ? c0 + chunk : n;
+  uint32_t* whist = s_whist[wid];
 
-  // A tile wholly inside [0, n) takes the unchecked path (every tile but
-  // the last).
-  const bool full = t0 + kSortTile <= n;
-  Raw kr[IT];
-  int32_t vv[IT];
-  uint32_t dp[IT];  // digit << 16 | position within the wave's digit bucket
-  auto load_rank = [&](auto full_c) {
-    constexpr bool FULL = decltype(full_c)::value;
+  uint32_t kr[IT];
+  int32_t vv[GEN ? 1 : IT];
+  const uint32_t len = (uint32_t)(c1 - c0);
+  const Raw* kc = kin + c0;
+  const int32_t* vc = GEN ? nullptr : vin + c0;
+  const uint32_t wl = (uint32_t)(wid * (kWave * IT) + lane);  // whole tile: position of the lane's row 0
+  // A whole tile's loads share one uniform base and one lane offset.
+  auto load = [&](uint32_t t) {
+    const char* kt = reinterpret_cast<const char*>(kc + t);
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+      kr[i] = *reinterpret_cast<const Raw*>(kt + wl * (uint32_t)sizeof(Raw) + i * kWave * sizeof(Raw));
+    if constexpr (!GEN) {
+      const char* vt = reinterpret_cast<const char*>(vc + t);
+#pragma unroll
+      for (int i = 0; i < IT; ++i) vv[i] = *reinterpret_cast<const int32_t*>(vt + wl * 4u + i * kWave * 4);
+    }
+  };
+  // The chunk's last tile, when it is not whole, has `part_rows` rows a wave.
+  // Loads past the chunk's end take its last key, so that none waits behind
+  // a branch.
+  auto load_part = [&](uint32_t t, uint32_t part_rows) {
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-      const int64_t p = wb + i * kWave + lane;
-      const bool valid = FULL || p < n;
-      kr[i] = valid ? kin[p] : Raw(0);
-      if constexpr (GEN_IDX) {
-        vv[i] = (int32_t)p;
+      const uint32_t p = t + (uint32_t)wid * kWave * part_rows + lane + i * kWave;
+      const uint32_t q = p < len ? p : len - 1;
+      kr[i] = kc[q];
+      if constexpr (!GEN) vv[i] = vc[q];
+    }
+  };
+  if (len >= (uint32_t)TILE) load(0);
+
+  // Output index of the chunk's first key of digit tid.
+  uint32_t ofs = 0;
+  {
+    uint32_t total = 0, incl = 0;
+    if (tid < 256) {
+      if (totals) {
+        ofs = counts[(size_t)blockIdx.x * parts * 256 + tid];
+        total = totals[tid];
       } else {
-        vv[i] = valid ? vin[p] : 0;
+        constexpr int U = 16;  // loads in flight
+        for (int g0 = 0; g0 < rows; g0 += U) {
+          uint32_t v[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[u] = counts[(size_t)(g0 + u < rows ? g0 + u : 0) * 256 + tid];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            ofs += g0 + u < (int)blockIdx.x * parts ? v[u] : 0u;
+            total += g0 + u < rows ? v[u] : 0u;
+          }
+        }
+      }
+      incl = wave_incl_scan(total);
+      if (lane == kWave - 1) s_wsum[wid] = incl;
+    }
+    __syncthreads();
+    if (tid < 256) {
+      for (int w = 0; w < wid; ++w) ofs += s_wsum[w];
+      ofs += incl - total;
+    }
+  }
+
+  auto do_tile = [&](uint32_t t, uint32_t part_rows, auto full_c) {
+    constexpr bool FULL = decltype(full_c)::value;
+    const int nrows = FULL ? IT : (int)part_rows;
+    const uint32_t wt = FULL ? wl : (uint32_t)wid * kWave * part_rows + lane;  // tile position of the lane's row 0
+    const int tvalid = FULL ? TILE : (int)(len - t);
+    const uint32_t first = (uint32_t)c0 + t;  // input position of the tile
+#pragma unroll
+    for (int k = 0; k < 256 / kWave; ++k) whist[k * kWave + lane] = 0;
+    KeyPair<DT> kp[IT / 2];
+    RowRegs<IT, KT::kBits> raw;
+    RowRegs<IT, 16> rk;
+    uint32_t pr[2];
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      if (i % 2 == 0) {
+        raw.set2(i, kr[i], kr[i + 1]);
+        kp[i / 2].set(kr[i], kr[i + 1], flip);
+      }
+      const uint32_t word = kp[i / 2].word(i % 2), at = kp[i / 2].shift(shift, i % 2);
+      if (FULL || i < nrows) {
+        const bool valid = FULL || wt + i * kWave < (uint32_t)tvalid;
+        pr[i % 2] = sort_rank_row(whist, word, at, sort_digit(word, at), valid, FULL ? ~0ull : __ballot(valid));
+      } else {
+        pr[i % 2] = 0;
+      }
+      if (i % 2 == 1) {
+        rk.set2(i - 1, pr[0], pr[1]);
+        asm volatile("" : "+v"(rk.w[i / 2]));
       }
     }
     __syncthreads();
 
-    // Stable rank of every item among the wave's items of the same digit.
-    const uint64_t lt = (1ull << lane) - 1ull;
+    // Thread d: its digit's keys per wave, their tile positions, and the
+    // output index that tile position 0 stands for.
+    uint32_t before[NW], cnt = 0, incl = 0;
+    if (tid < 256) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        before[w] = cnt;
+        cnt += s_whist[w][tid];
+      }
+      incl = wave_incl_scan(cnt);
+      if (lane == kWave - 1) s_wsum[wid] = incl;
+    }
+    __syncthreads();
+    if (tid < 256) {
+      uint32_t excl = incl - cnt;
+      for (int w = 0; w < wid; ++w) excl += s_wsum[w];
+#pragma unroll
+      for (int w = 0; w < NW; ++w) s_whist[w][tid] = excl + before[w];
+      s_gofs[tid] = ofs - excl;
+      ofs += cnt;
+    }
+    __syncthreads();
+
+    constexpr int RB = 16;  // rows whose tile positions are read at once
+    uint32_t pos[RB];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-      const bool valid = FULL || wb + i * kWave + lane < n;
-      const int d = digit_of(kr[i]);
-      uint64_t peers = FULL ? ~0ull : __ballot(valid);
+      if (i % RB == 0) {
 #pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        const bool bit = (d >> b) & 1;
-        const uint64_t m = __ballot(bit);
-        peers &= bit ? m : ~m;
+        for (int j = 0; j < RB && j < IT; ++j)
+          pos[j] = whist[sort_digit(kp[(i + j) / 2].word(j % 2), kp[(i + j) / 2].shift(shift, j % 2))];
       }
-      const uint32_t rank = (uint32_t)__popcll(peers & lt);
-      uint32_t base = 0;
-      if (valid) {
-        base = s_whist[wid][d];
-        if (rank == 0) s_whist[wid][d] = base + (uint32_t)__popcll(peers);
+      const uint32_t local = wt + i * kWave;
+      if (FULL || (i < nrows && local < (uint32_t)tvalid)) {
+        const uint32_t d = sort_digit(kp[i / 2].word(i % 2), kp[i / 2].shift(shift, i % 2));
+        const uint32_t p = pos[i % RB] + rk.get(i);
+        if constexpr (kWord) {
+          s_item[p] = (raw.get(i) << 16) | local;
+          if constexpr (kDig) s_dig[p] = (uint8_t)d;
+        } else {
+          const uint32_t val = GEN ? first + local : (uint32_t)vv[i];
+          s_item[p] = ((uint64_t)val << 32) | (kNarrow ? (d << 16) | raw.get(i) : raw.get(i));
+        }
       }
-      dp[i] = ((uint32_t)d << 16) | (base + rank);
+    }
+    if (FULL && t + 2 * TILE <= len) load(t + TILE);
+    __syncthreads();
+
+    auto put = [&](int p, uint32_t d, uint32_t raw, uint32_t val) {
+      const uint32_t dst = s_gofs[d] + (uint32_t)p;
+      if constexpr (!BIG) {
+        *reinterpret_cast<Raw*>(reinterpret_cast<char*>(kout) + dst * (uint32_t)sizeof(Raw)) = (Raw)raw;
+        *reinterpret_cast<int32_t*>(reinterpret_cast<char*>(vout) + dst * 4u) = (int32_t)val;
+      } else {
+        kout[dst] = (Raw)raw;
+        vout[dst] = (int32_t)val;
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < IT; i += 2) {
+      Item e[2];
+      uint32_t d[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int p = (i + h) * NT + tid;
+        const bool in = FULL || (i < nrows && p < tvalid);
+        e[h] = in ? s_item[p] : Item(0);
+        if constexpr (kDig) d[h] = in ? s_dig[p] : 0u;
+      }
+      if constexpr (!kWord && kNarrow) {
+        d[0] = ((uint32_t)e[0] >> 16) & 0xffu;
+        d[1] = ((uint32_t)e[1] >> 16) & 0xffu;
+      } else if constexpr (!kDig) {
+        KeyPair<DT> q;
+        if constexpr (kWord) q.set((uint32_t)e[0] >> 16, (uint32_t)e[1] >> 16, flip);
+        else q.set((uint32_t)e[0], (uint32_t)e[1], flip);
+        d[0] = sort_digit(q.word(0), q.shift(shift, 0));
+        d[1] = sort_digit(q.word(1), q.shift(shift, 1));
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int p = (i + h) * NT + tid;
+        if (FULL || (i < nrows && p < tvalid)) {
+          if constexpr (kWord) {
+            put(p, d[h], (uint32_t)e[h] >> 16, first + ((uint32_t)e[h] & 0xffffu));
+          } else {
+            put(p, d[h], (uint32_t)e[h], (uint32_t)(e[h] >> 32));
+          }
+        }
+      }
     }
   };
-  if (full) {
-    load_rank(std::integral_constant<bool, true>{});
-  } else {
-    load_rank(std::integral_constant<bool, false>{});
-  }
-  __syncthreads();
-
-  uint64_t* desc = ws_desc(ws);
-  const uint32_t tag = s_tag.tag;
-  const int max_polls = s_tag.polls;
-  uint32_t cnt = 0, incl = 0;
-  if (tid < 256) {
-    const int d = tid;
-    uint32_t run = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const uint32_t c = s_whist[w][d];
-      s_whist[w][d] = run;
-      run += c;
-    }
-    cnt = run;
-    // Publish this tile's count of digit d at once (tile 0's is inclusive).
-    if (num_tiles > 1)
-      desc_publish<uint32_t>(desc, (uint64_t)tile * 256 + d, cnt, tag, tile == 0 ? kFlagIncl : kFlagAgg);
-    incl = wave_incl_scan(cnt);
-    if (lane == kWave - 1) s_wsum[wid] = incl;
-  }
-  __syncthreads();
-  if (tid < 256) {
-    const int d = tid;
-    uint32_t before = 0;
-    for (int w = 0; w < wid; ++w) before += s_wsum[w];
-    const uint32_t excl = before + incl - cnt;
-    s_excl[d] = excl;
-    // Keys of digit d in the tiles before this one: walk back to the
-    // nearest inclusive descriptor, one predecessor at a time (reading
-    // several at once measured slower: the extra device-scope loads cost
-    // more than the walk saves).  A predecessor that has not published
-    // after the poll limit (kFallbackPolls by default) is counted from its keys here.
-    uint32_t prefix = 0;
-    for (int64_t q = (int64_t)tile - 1; q >= 0; --q) {
-      uint32_t v = 0;
-      int flag = 0;
-      int polls = 0;
-      while (!desc_try_read<uint32_t>(desc, (uint64_t)q * 256 + d, tag, v, flag)) {
-        if (polls++ >= max_polls) {
-          const int64_t u0 = q * kSortTile;
-          const int64_t u1 = u0 + kSortTile < n ? u0 + kSortTile : n;
-          v = 0;
-          for (int64_t e = u0; e < u1; ++e) v += digit_of(kin[e]) == d ? 1u : 0u;
-          flag = q == 0 ? (int)kFlagIncl : (int)kFlagAgg;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
-      prefix += v;
-      if (flag == (int)kFlagIncl) break;
-    }
-    if (tile > 0 && tile + 1 < num_tiles) desc_publish<uint32_t>(desc, (uint64_t)tile * 256 + d, prefix + cnt, tag, kFlagIncl);
-    s_gofs[d] = (int32_t)((uint32_t)gbase[d] + prefix) - (int32_t)excl;
-  }
-  __syncthreads();
-
-  // Reorder the tile by digit in LDS (stable), then write each digit's run.
-#pragma unroll
-  for (int i = 0; i < IT; ++i) {
-    if (full || wb + i * kWave + lane < n) {
-      const int d = (int)(dp[i] >> 16);
-      const uint32_t pos = s_excl[d] + s_whist[wid][d] + (dp[i] & 0xffffu);
-      s_keys[pos] = kr[i];
-      s_vals[pos] = vv[i];
-      if constexpr (kDigLds) s_dig[pos] = (uint8_t)d;
-    }
-  }
-  __syncthreads();
-  const int tvalid = full ? (int)kSortTile : (int)(n - t0);
-  for (int pos = tid; pos < tvalid; pos += NW * kWave) {
-    const Raw r = s_keys[pos];
-    const int d = kDigLds ? (int)s_dig[pos] : digit_of(r);
-    const int64_t dst = (int64_t)s_gofs[d] + pos;
-    kout[dst] = r;
-    vout[dst] = s_vals[pos];
+  // Everything loaded so far has arrived when the loop starts (vmcnt 0), so
+  // that inside it a tile's first use waits for its own loads only, not for
+  // the stores issued after them.
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  uint32_t t = 0;
+  for (; t + TILE <= len; t += TILE) do_tile(t, IT, std::integral_constant<bool, true>{});
+  if (t < len) {
+    const uint32_t part_rows = (len - t + NT - 1) / NT;
+    load_part(t, part_rows);
+    do_tile(t, part_rows, std::integral_constant<bool, false>{});
   }
 }
 
-// Workspace: header, 256 descriptors per tile, bucket starts, histogram
-// partials and their first-level sums (zeroed once and reusable, like every
-// workspace; counts are kept in 64-bit words with a zero high half, which
-// never read as a valid descriptor when a later call uses the same bytes
-// for descriptors).
-// Scratch: one temporary copy of keys and positions (any contents).
+// ---------------------------------------------------------------------------
+// At most kSortBlockMax keys: every digit position in one workgroup, keys
+// and positions in LDS between passes: one launch (3000 fp16 keys 7.5 us, 8000
+// int32 keys 21 us; a histogram, two sums and a look-back pass per digit took
+// 29 and 53).  Twice as many keys in one workgroup are slower than the
+// chunked form (16000 fp16: 22 against 15 us).  Wave w holds elements
+// [64 w rows, 64 (w + 1) rows), rows = ceil(n / 1024).
+// ---------------------------------------------------------------------------
+constexpr int kSortBlockThreads = 1024, kSortBlockIT = 8;
+constexpr int64_t kSortBlockMax = (int64_t)kSortBlockThreads * kSortBlockIT;
+template <int DT>
+__global__ __launch_bounds__(kSortBlockThreads) void sort_block_kernel(
+    const typename SortKey<DT>::Raw* __restrict__ x, const int32_t* __restrict__ idx_in,
+    typename SortKey<DT>::Raw* __restrict__ out_x, int32_t* __restrict__ out_idx, int n, uint32_t flip) {
+  using KT = SortKey<DT>;
+  using Raw = typename KT::Raw;
+  constexpr int NW = kSortBlockThreads / kWave, IT = kSortBlockIT, P = KT::kBits / 8;
+  __shared__ uint32_t s_whist[NW][256];
+  __shared__ uint32_t s_wsum[4];
+  __shared__ uint64_t s_item[kSortBlockMax];
+  const int tid = threadIdx.x, lane = __lane_id(), wid = tid / kWave;
+  const int rows = (n + kSortBlockThreads - 1) / kSortBlockThreads;
+  const int wb = wid * rows * kWave + lane;
+  uint32_t* whist = s_whist[wid];
+  uint32_t kr[IT], vv[IT];
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int p = wb + i * kWave;
+    const bool valid = i < rows && p < n;
+    kr[i] = valid ? (uint32_t)x[p] : 0u;
+    vv[i] = valid && idx_in ? (uint32_t)idx_in[p] : (uint32_t)p;
+  }
+  for (int pass = 0; pass < P; ++pass) {
+    const uint32_t shift = 8u * (uint32_t)pass;
+#pragma unroll
+    for (int k = 0; k < 256 / kWave; ++k) whist[k * kWave + lane] = 0;
+    uint32_t dr[IT];  // digit << 16 | rank
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      if (i < rows) {
+        const bool valid = wb + i * kWave < n;
+        const uint32_t key = KT::key((Raw)kr[i]) ^ flip;
+        const uint32_t d = sort_digit(key, shift);
+        dr[i] = (d << 16) | sort_rank_row(whist, key, shift, d, valid, __ballot(valid));
+      }
+    }
+    __syncthreads();
+    uint32_t before[NW], cnt = 0, incl = 0;
+    if (tid < 256) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        before[w] = cnt;
+        cnt += s_whist[w][tid];
+      }
+      incl = wave_incl_scan(cnt);
+      if (lane == kWave - 1) s_wsum[wid] = incl;
+    }
+    __syncthreads();
+    if (tid < 256) {
+      uint32_t excl = incl - cnt;
+      for (int w = 0; w < wid; ++w) excl += s_wsum[w];
+#pragma unroll
+      for (int w = 0; w < NW; ++w) s_whist[w][tid] = excl + before[w];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      if (i < rows && wb + i * kWave < n)
+        s_item[whist[dr[i] >> 16] + (dr[i] & 0xffffu)] = ((uint64_t)vv[i] << 32) | kr[i];
+    }
+    __syncthreads();
+    if (pass + 1 < P) {
+#pragma unroll
+      for (int i = 0; i < IT; ++i) {
+        if (i < rows && wb + i * kWave < n) {
+          const uint64_t e = s_item[wb + i * kWave];
+          kr[i] = (uint32_t)e;
+          vv[i] = (uint32_t)(e >> 32);
+        }
+      }
+    }
+  }
+  for (int p = tid; p < n; p += kSortBlockThreads) {
+    const uint64_t e = s_item[p];
+    out_x[p] = (Raw)e;
+    out_idx[p] = (int32_t)(uint32_t)(e >> 32);
+  }
+}
+
+// Scratch: one temporary copy of keys and positions, the digit counts and
+// their totals (any contents).  The workspace is only its header: no pass
+// looks back.
 struct SortLayout {
-  size_t desc_off, gbase_off, part_off, psum_off, total;
-  size_t tmpv_off, scratch;
-  int groups;
+  size_t tmpv_off, counts_off, totals_off, scratch;
+  bool wide;            // 16-wave scatter workgroups, else 8-wave ones
+  int chunks, parts;    // scatter workgroups, count rows per chunk
   int64_t chunk;
 };
 
@@ -338,68 +559,117 @@ inline int sort_passes(int dt) {
 
 inline int sort_elem_bytes(int dt) { return dt == TCS_I8 ? 1 : (sort_passes(dt) == 2 ? 2 : 4); }
 
+// Above this many keys the scatter workgroups take 16 waves, and 16384 or
+// 32768 keys a tile (the LDS of a whole compute unit), one workgroup on each:
+// a tile's runs are then twice or four times as long, and fewer of the lines
+// that the 256 runs write are left partial between tiles.  Below it 8-wave
+// workgroups with 4096-key tiles, two to a compute unit, divide the keys more
+// evenly (fp16 keys, 4e6: 46 against 53 us, 5e6: 56 against 61, 8e6: 73
+// either way; int32, 4e6: 101 against 106, 8e6: 176 against 161).
+constexpr int64_t kSortWideMin = (int64_t)6 << 20;
 inline SortLayout sort_layout(int64_t n, int dt) {
   SortLayout L{};
-  const int P = sort_passes(dt);
-  const uint64_t tiles = (uint64_t)((n + kSortTile - 1) / kSortTile);
-  int64_t groups = (n + 65535) / 65536;
-  if (groups > kHistMaxGroups) groups = kHistMaxGroups;
-  if (groups < 1) groups = 1;
-  int64_t chunk = (n + groups - 1) / groups;
-  chunk = (chunk + 63) & ~(int64_t)63;  // 16-byte aligned chunk starts
-  L.groups = (int)groups;
-  L.chunk = chunk;
-  L.desc_off = kHeaderBytes;
-  L.gbase_off = align256(L.desc_off + (size_t)tiles * 256 * 8);
-  L.part_off = align256(L.gbase_off + (size_t)kMaxPasses * 256 * 8);
-  L.psum_off = align256(L.part_off + (size_t)groups * P * 256 * 8);
-  L.total = align256(L.psum_off + (size_t)kSortSumGroups * P * 256 * 8);
+  L.wide = n > kSortWideMin;
+  const int64_t least = 2048, most = L.wide ? kSortMaxChunks / 2 : kSortMaxChunks, unit = L.wide ? 4096 : 512;
+  int64_t chunks = (n + least - 1) / least;
+  if (chunks > most) chunks = most;
+  if (chunks < 1) chunks = 1;
+  L.chunk = ((n + chunks - 1) / chunks + unit - 1) / unit * unit;
+  if (L.chunk < unit) L.chunk = unit;
+  L.chunks = n > 0 ? (int)((n + L.chunk - 1) / L.chunk) : 1;
+  L.parts = 1;
+  while (L.wide && L.parts < 4 && L.chunk / L.parts > 16384) L.parts *= 2;
   L.tmpv_off = align256((size_t)n * sort_elem_bytes(dt));
-  L.scratch = align256(L.tmpv_off + (size_t)n * 4);
+  L.counts_off = align256(L.tmpv_off + (size_t)n * 4);
+  L.totals_off = align256(L.counts_off + (size_t)L.chunks * L.parts * 256 * 4);
+  L.scratch = align256(L.totals_off + 256 * 4);
   return L;
 }
 
 template <int DT>
+struct SortArgs {
+  using Raw = typename SortKey<DT>::Raw;
+  const Raw* kin;
+  const int32_t* vin;
+  Raw* kout;
+  int32_t* vout;
+  const uint32_t *counts, *totals;
+  uint32_t shift, flip;
+  int64_t n;
+};
+
+template <int DT, bool GEN, int NW, int IT, bool BIG = false>
+static void sort_scatter_launch(const SortLayout& L, const SortArgs<DT>& a, hipStream_t st) {
+  hipLaunchKernelGGL((sort_scatter_kernel<DT, GEN, NW, IT, BIG>), dim3(L.chunks), dim3(NW * kWave), 0, st, a.kin,
+                     a.vin, a.kout, a.vout, a.counts, a.totals, L.chunks * L.parts, L.parts, a.shift, a.flip, a.n,
+                     L.chunk);
+}
+
+// A tile as large as the LDS of a compute unit allows for the wide form:
+// 32768 16-bit keys whose positions are generated, 16384 others.
+template <int DT, bool GEN>
+static void sort_scatter(const SortLayout& L, const SortArgs<DT>& a, hipStream_t st) {
+  constexpr int IT = GEN && SortKey<DT>::kBits <= 16 ? 32 : 16;
+  if (!L.wide) {
+    sort_scatter_launch<DT, GEN, 8, 8>(L, a, st);
+  } else if (a.n < ((int64_t)1 << 30)) {
+    sort_scatter_launch<DT, GEN, 16, IT>(L, a, st);
+  } else {
+    sort_scatter_launch<DT, GEN, 16, IT, true>(L, a, st);
+  }
+}
+
+template <int DT>
 static int sort_run(const void* x, const int32_t* idx_in, void* out_x, int32_t* out_idx, int64_t n, bool desc,
-                    void* ws, void* scratch, hipStream_t st) {
+                    void* scratch, hipStream_t st) {
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
   constexpr int P = KT::kBits / 8;
+  SortArgs<DT> a{};
+  a.flip = desc ? ~0u : 0u;
+  a.n = n;
+  a.kin = static_cast<const Raw*>(x);
+  a.vin = idx_in;
+  if (n <= kSortBlockMax) {
+    hipLaunchKernelGGL((sort_block_kernel<DT>), dim3(1), dim3(kSortBlockThreads), 0, st, a.kin, idx_in,
+                       static_cast<Raw*>(out_x), out_idx, (int)n, a.flip);
+    TCS_CHECK_LAUNCH();
+    return TCS_OK;
+  }
   const SortLayout L = sort_layout(n, DT);
-  char* w = static_cast<char*>(ws);
-  auto* gbase = reinterpret_cast<uint64_t*>(w + L.gbase_off);
-  auto* partial = reinterpret_cast<uint64_t*>(w + L.part_off);
-  auto* tk = reinterpret_cast<Raw*>(scratch);
-  auto* tv = reinterpret_cast<int32_t*>(static_cast<char*>(scratch) + L.tmpv_off);
-  const uint32_t flip = desc ? (KT::kBits == 32 ? 0xffffffffu : ((1u << KT::kBits) - 1u)) : 0u;
-  hipLaunchKernelGGL((sort_hist_kernel<DT>), dim3(L.groups), dim3(kHistThreads), 0, st, static_cast<const Raw*>(x),
-                     n, L.chunk, flip, partial);
-  TCS_CHECK_LAUNCH();
-  auto* psum = reinterpret_cast<uint64_t*>(w + L.psum_off);
-  const int sum_per = (L.groups + kSortSumGroups - 1) / kSortSumGroups;
-  const int sum_groups = (L.groups + sum_per - 1) / sum_per;
-  hipLaunchKernelGGL(sort_sum_kernel, dim3(sum_groups, P), dim3(256), 0, st, partial, L.groups, sum_per, P, psum);
-  TCS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(sort_bucket_kernel, dim3(P), dim3(kBucketThreads), 0, st, psum, sum_groups, P, gbase);
-  TCS_CHECK_LAUNCH();
-  const uint32_t tiles = (uint32_t)((n + kSortTile - 1) / kSortTile);
-  const Raw* kin = static_cast<const Raw*>(x);
-  const int32_t* vin = idx_in;
+  const int rows = L.chunks * L.parts;
+  char* sc = static_cast<char*>(scratch);
+  auto* counts = reinterpret_cast<uint32_t*>(sc + L.counts_off);
+  auto* totals = rows > kSortFusedRows ? reinterpret_cast<uint32_t*>(sc + L.totals_off) : nullptr;
+  a.counts = counts;
+  a.totals = totals;
   for (int p = 0; p < P; ++p) {
     // The last pass writes the outputs; earlier ones alternate so that it does.
     const bool to_out = ((P - 1 - p) % 2) == 0;
-    Raw* kout = to_out ? static_cast<Raw*>(out_x) : tk;
-    int32_t* vout = to_out ? out_idx : tv;
-    if (p == 0 && !idx_in) {
-      hipLaunchKernelGGL((sort_pass_kernel<DT, true>), dim3(tiles), dim3(kSortNW * kWave), 0, st, kin, vin, kout,
-                         vout, gbase + p * 256, 8 * p, flip, n, ws, tiles);
+    a.kout = to_out ? static_cast<Raw*>(out_x) : reinterpret_cast<Raw*>(sc);
+    a.vout = to_out ? out_idx : reinterpret_cast<int32_t*>(sc + L.tmpv_off);
+    a.shift = 8u * (uint32_t)p;
+    if (L.wide) {
+      hipLaunchKernelGGL((sort_count_kernel<DT, 4>), dim3(rows), dim3(kSortThreads), 0, st, a.kin, n,
+                         L.chunk / L.parts, a.shift, a.flip, counts);
     } else {
-      hipLaunchKernelGGL((sort_pass_kernel<DT, false>), dim3(tiles), dim3(kSortNW * kWave), 0, st, kin, vin, kout,
-                         vout, gbase + p * 256, 8 * p, flip, n, ws, tiles);
+      hipLaunchKernelGGL((sort_count_kernel<DT, 1>), dim3(rows), dim3(kSortThreads), 0, st, a.kin, n,
+                         L.chunk / L.parts, a.shift, a.flip, counts);
     }
     TCS_CHECK_LAUNCH();
-    kin = kout;
-    vin = vout;
+    if (totals) {
+      hipLaunchKernelGGL(sort_row_scan_kernel, dim3(256 / kSortScanDigits), dim3(kSortScanThreads), 0, st, counts,
+                         rows, totals);
+      TCS_CHECK_LAUNCH();
+    }
+    if (p == 0 && !idx_in) {
+      sort_scatter<DT, true>(L, a, st);
+    } else {
+      sort_scatter<DT, false>(L, a, st);
+    }
+    TCS_CHECK_LAUNCH();
+    a.kin = a.kout;
+    a.vin = a.vout;
   }
   return TCS_OK;
 }
@@ -410,7 +680,7 @@ extern "C" {
 
 size_t tcs_sort_workspace_bytes(int64_t n, int dtype) {
   if (n < 0 || tcs::sort_passes(dtype) == 0) return 0;
-  return tcs::sort_layout(n, dtype).total;
+  return tcs::lookback_ws_bytes(0);
 }
 
 size_t tcs_sort_scratch_bytes(int64_t n, int dtype) {
@@ -428,17 +698,17 @@ int tcs_sort(const void* x, int dtype, const int32_t* idx_in, void* out_x, int32
   if (!x || !out_x || !out_idx) return TCS_ERR_INVALID_ARG;
   if (!aligned16(x) || (idx_in && !aligned16(idx_in))) return TCS_ERR_INVALID_ARG;
   const SortLayout L = sort_layout(n, dtype);
-  if (!workspace || workspace_bytes < L.total || !scratch || scratch_bytes < L.scratch) return TCS_ERR_WORKSPACE;
+  if (!workspace || workspace_bytes < lookback_ws_bytes(0) || !scratch || scratch_bytes < L.scratch) return TCS_ERR_WORKSPACE;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool d = descending != 0;
   switch (dtype) {
-    case TCS_F16: return sort_run<TCS_F16>(x, idx_in, out_x, out_idx, n, d, workspace, scratch, st);
-    case TCS_BF16: return sort_run<TCS_BF16>(x, idx_in, out_x, out_idx, n, d, workspace, scratch, st);
-    case TCS_F32: return sort_run<TCS_F32>(x, idx_in, out_x, out_idx, n, d, workspace, scratch, st);
-    case TCS_I8: return sort_run<TCS_I8>(x, idx_in, out_x, out_idx, n, d, workspace, scratch, st);
-    case TCS_I16: return sort_run<TCS_I16>(x, idx_in, out_x, out_idx, n, d, workspace, scratch, st);
-    case TCS_I32: return sort_run<TCS_I32>(x, idx_in, out_x, out_idx, n, d, workspace, scratch, st);
-    default: return sort_run<TCS_U32>(x, idx_in, out_x, out_idx, n, d, workspace, scratch, st);
+    case TCS_F16: return sort_run<TCS_F16>(x, idx_in, out_x, out_idx, n, d, scratch, st);
+    case TCS_BF16: return sort_run<TCS_BF16>(x, idx_in, out_x, out_idx, n, d, scratch, st);
+    case TCS_F32: return sort_run<TCS_F32>(x, idx_in, out_x, out_idx, n, d, scratch, st);
+    case TCS_I8: return sort_run<TCS_I8>(x, idx_in, out_x, out_idx, n, d, scratch, st);
+    case TCS_I16: return sort_run<TCS_I16>(x, idx_in, out_x, out_idx, n, d, scratch, st);
+    case TCS_I32: return sort_run<TCS_I32>(x, idx_in, out_x, out_idx, n, d, scratch, st);
+    default: return sort_run<TCS_U32>(x, idx_in, out_x, out_idx, n, d, scratch, st);
   }
 }
 

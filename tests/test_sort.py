@@ -205,3 +205,49 @@ def test_workspace_shared_across_sizes_and_ops(ops, dev):
         assert_exact(to_np(y), oracle.seg_sum_indptr(to_np(xs), indptr.numpy()), f"segsum n={n}")
         xi = torch.randint(-4, 5, (2 * n,), generator=gen(n + 2), dtype=torch.int8)
         assert_exact(to_np(ops.run_scan_multi_core(xi.to(dev), 32)), oracle.scan(to_np(xi)), f"scan n={n}")
+
+
+# Around the edges of the sort's forms: one workgroup up to 8192 keys, counts
+# summed by the scatter kernel up to 64 chunks of 2048 keys, 512 chunks from
+# 2^20 keys, wide workgroups above 6 * 2^20 (their tiles of 16384 and 32768
+# keys, and a chunk counted in one, two and four parts).
+FORM_EDGES = [8192, 8193, 64 * 2048, 64 * 2048 + 1, (1 << 20) - 1, (1 << 20) + 1, (6 << 20), (6 << 20) + 1,
+              1 << 23, (1 << 23) + 1, (1 << 24) + 4097]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", FORM_EDGES)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.int16, torch.float32, torch.int8], ids=str)
+def test_sort_form_edges(ops, dev, n, dtype):
+    if dtype.is_floating_point:
+        x = special(n, dtype, n).to(dev)
+    else:
+        info = torch.iinfo(dtype)
+        x = torch.randint(info.min, info.max + 1, (n,), generator=gen(n), dtype=torch.int64).to(dtype).to(dev)
+    for descending in (False, True):
+        v, i = ops.run_radix_sort_ex(x, descending)
+        _, ei = _torch_sort(x, descending)
+        assert torch.equal(i, ei), (n, descending)
+        bits = torch.int32 if x.element_size() == 4 else (torch.int16 if x.element_size() == 2 else torch.int8)
+        assert torch.equal(v.view(bits), x[ei.long()].view(bits)), (n, descending)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [100_000, 7_000_001])
+def test_sort_one_value(ops, dev, n):
+    # Every key in one bin of every pass: the identity.
+    v, i = ops.run_radix_sort(torch.full((n,), -2.5, device=dev), 128)
+    assert torch.equal(i, torch.arange(n, dtype=torch.int32, device=dev)) and bool((v == -2.5).all())
+
+
+@pytest.mark.gpu
+def test_sort_2p30(ops, dev):
+    # Outputs past the reach of 32-bit byte offsets.  Strictly increasing
+    # (value, position) pairs with value = x[position] are the stable sort.
+    n = (1 << 30) + 5
+    x = torch.randint(-2**15, 2**15, (n,), device=dev, dtype=torch.int16, generator=torch.Generator(dev).manual_seed(3))
+    v, i = ops.run_radix_sort(x, 128)
+    for a in range(0, n, 1 << 27):
+        vv, ii = v[a:a + (1 << 27) + 1], i[a:a + (1 << 27) + 1]
+        assert torch.equal(x[ii.long()], vv)
+        assert bool(((vv[:-1] < vv[1:]) | ((vv[:-1] == vv[1:]) & (ii[:-1] < ii[1:]))).all())
