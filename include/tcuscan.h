@@ -450,17 +450,24 @@ int tcs_topk_pivot(const void* x, int64_t n, int num_samples, void* out, int64_t
 int tcs_searchsorted(const int32_t* sorted, int64_t sorted_len, const int32_t* values, int32_t* out,
                      int64_t num_values, void* stream);
 
-/* Workspace bytes of tcs_searchsorted_indexed for a haystack of sorted_len
- * elements: a bucket table of 2^b + 1 int32, b = clamp(floor(log2(len)) - 4,
- * 10, 20) (at most 4 MiB + 4 bytes). */
+/* Least workspace bytes of tcs_searchsorted_indexed for a haystack of
+ * sorted_len elements: 2^b + 1 int32, b = clamp(floor(log2(len)) - 4, 10, 20)
+ * (at most 4 MiB + 4 bytes). */
 size_t tcs_searchsorted_workspace_bytes(int64_t sorted_len);
+
+/* Workspace bytes with which it is fastest: 512 counts and a table of
+ * 2^b + 1 int32, b = clamp(floor(log2(len)) - 2, 10, 22) (at most 16 MiB +
+ * 2052 bytes).  Any size from the least up is taken. */
+size_t tcs_searchsorted_preferred_bytes(int64_t sorted_len);
 
 /* tcs_searchsorted with a bucket index built in `workspace` first (no host
  * synchronisation): the haystack's order keys between its first and last
- * element are cut into 2^b buckets of equal width, the start of every
+ * element are cut into up to 2^b buckets of equal width, the start of every
  * bucket is found once, and each needle then searches only its bucket
- * (about 16 elements when the keys spread over their range; clustered keys
- * fall back to the sampled search of tcs_searchsorted).  Results identical
+ * (4 to 8 elements when the keys spread over their range and the workspace
+ * is the preferred one; clustered keys fall back to the sampled search of
+ * tcs_searchsorted, and a haystack of at most 16384 elements is searched
+ * whole in LDS).  Results identical
  * to tcs_searchsorted.  `workspace` is scratch that this call overwrites
  * from its first byte (any contents before, nothing kept after): it must
  * not be a look-back workspace that other calls use, unless that is zeroed

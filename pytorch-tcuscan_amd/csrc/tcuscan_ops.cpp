@@ -1192,7 +1192,7 @@ at::Tensor run_count_if(const at::Tensor& x_in, float pivot, uint32_t tile_len, 
 }
 
 // run_searchsorted takes the bucket index above these sizes.
-constexpr int64_t kIndexedMinLen = (int64_t)1 << 16, kIndexedMinNeedles = (int64_t)1 << 16;
+constexpr int64_t kIndexedMinLen = (int64_t)1 << 16, kIndexedMinNeedles = (int64_t)1 << 15;
 
 // src/torch/torch_searchsorted.h:33-82
 at::Tensor run_searchsorted(const at::Tensor& sorted_in, const at::Tensor& values_in) {
@@ -1206,11 +1206,11 @@ at::Tensor run_searchsorted(const at::Tensor& sorted_in, const at::Tensor& value
   at::Tensor out = at::empty({values.numel()}, values.options());  // flat, as the reference returns
   const at::hip::HIPGuardMasqueradingAsCUDA guard(values.device());
   // Haystacks beyond the LDS samples with many needles: the bucket index
-  // (its build costs about one search per 16 haystack elements).
-  if (sorted.numel() > kIndexedMinLen && values.numel() >= kIndexedMinNeedles) {
+  // (its build reads the haystack once).
+  if (sorted.numel() > kIndexedMinLen && values.numel() > kIndexedMinNeedles) {
     // The bucket table is scratch of this call only: a buffer of its own, not
     // the stream's look-back workspace (whose header it would overwrite).
-    const size_t tb = tcs_searchsorted_workspace_bytes(sorted.numel());
+    const size_t tb = tcs_searchsorted_preferred_bytes(sorted.numel());
     at::Tensor table = at::empty({(int64_t)tb}, values.options().dtype(at::kByte));
     check(tcs_searchsorted_indexed(sorted.data_ptr<int32_t>(), sorted.numel(), values.data_ptr<int32_t>(),
                                    out.data_ptr<int32_t>(), values.numel(), table.data_ptr(), tb,

@@ -139,3 +139,52 @@ def test_op_leaves_the_stream_workspace_intact(ops, dev):
         m = (torch.rand(xd.numel(), generator=gen(4)) < 0.3).to(torch.int8).to(dev)
         z = ops.run_compress(xd, m, 128)
         assert torch.equal(z.cpu(), x[m.cpu() == 1])
+
+
+@pytest.mark.parametrize("kind", ["uniform", "narrow", "constant", "clusters", "heavy_tail"])
+@pytest.mark.parametrize("n", [16385, 65537, (1 << 20) + 3, (1 << 22) + 5])
+def test_preferred_table(lib, dev, kind, n):
+    """The preferred table: needles in input order, and grouped (above 2^20
+    elements and 1.5 * 2^20 needles), a ragged last tile of needles included;
+    nothing written past the outputs and the workspace."""
+    lib.tcs_searchsorted_preferred_bytes.restype = ctypes.c_size_t
+    lib.tcs_searchsorted_preferred_bytes.argtypes = [ctypes.c_int64]
+    rng = np.random.default_rng(n + len(kind))
+    hay = _haystack(kind, n, rng)
+    h = torch.from_numpy(hay).to(dev)
+    wsb = lib.tcs_searchsorted_preferred_bytes(n)
+    assert wsb >= lib.tcs_searchsorted_workspace_bytes(n)
+    ws = torch.full((wsb // 4 + 8,), -1, dtype=torch.int32, device=dev)
+    s = torch.cuda.current_stream().cuda_stream
+    for m in (70_000, 1_600_001):
+        needles = _needles(rng, hay, m)
+        v = torch.from_numpy(needles).to(dev)
+        out = torch.full((len(needles) + 8,), -7, dtype=torch.int32, device=dev)
+        assert lib.tcs_searchsorted_indexed(h.data_ptr(), n, v.data_ptr(), out.data_ptr(), len(needles), ws.data_ptr(),
+                                            wsb, s) == 0
+        got = out.cpu().numpy()
+        assert np.array_equal(got[:-8], np.searchsorted(hay, needles, side="left").astype(np.int32)), (kind, m)
+        assert (got[-8:] == -7).all()
+        assert bool((ws[-8:] == -1).all())
+
+
+def test_unaligned_views(ops, dev):
+    """Haystack and needles that start one element into an allocation."""
+    rng = np.random.default_rng(9)
+    for n, m in ((70_001, 40_001), (300_003, 5_001), (1 << 21, 1_700_001)):
+        hay = _haystack("uniform", n, rng)
+        needles = _needles(rng, hay, m)
+        h, v = torch.from_numpy(hay).to(dev)[1:], torch.from_numpy(needles).to(dev)[1:]
+        exp = np.searchsorted(hay[1:], needles[1:], side="left").astype(np.int32)
+        assert np.array_equal(ops.run_searchsorted(h, v).cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 255, 257, 4097, 16384, 16385, 100_000])
+def test_few_needles(ops, dev, n):
+    """Sixteen lanes a needle, at lengths around powers of sixteen."""
+    rng = np.random.default_rng(n)
+    hay = _haystack("narrow" if n % 2 else "uniform", n, rng)
+    for m in (1, 3, 16, 1000):
+        needles = _needles(rng, hay, m)
+        got = ops.run_searchsorted(torch.from_numpy(hay).to(dev), torch.from_numpy(needles).to(dev)).cpu().numpy()
+        assert np.array_equal(got, np.searchsorted(hay, needles, side="left").astype(np.int32))
