@@ -212,7 +212,8 @@ __global__ __launch_bounds__(kSortScanThreads) void sort_row_scan_kernel(uint32_
 // GEN: positions are generated (the first pass without given indices); a
 // 16-bit key then shares a word with its tile-local position, and the tile
 // takes half the LDS.  BIG: 2^30 keys or more, whose outputs 32-bit byte
-// offsets do not reach.
+// offsets do not reach.  LIMIT: the outputs past the first `limit` are not
+// written.
 //
 // Bound by the write requests of the runs and by the ranking: 2^28 fp16
 // normals, first pass 0.73 ms and second 0.79 (8-wave workgroups with
@@ -220,12 +221,12 @@ __global__ __launch_bounds__(kSortScanThreads) void sort_row_scan_kernel(uint32_
 // without any write 0.50).  The look-back passes before took 1.34 and 1.25 ms.
 // Plain loads: nontemporal ones measured the same.
 // ---------------------------------------------------------------------------
-template <int DT, bool GEN, int NW, int IT, bool BIG>
+template <int DT, bool GEN, int NW, int IT, bool BIG, bool LIMIT>
 __global__ __launch_bounds__(NW * kWave, 4) void sort_scatter_kernel(
     const typename SortKey<DT>::Raw* __restrict__ kin, const int32_t* __restrict__ vin,
     typename SortKey<DT>::Raw* __restrict__ kout, int32_t* __restrict__ vout, const uint32_t* __restrict__ counts,
     const uint32_t* __restrict__ totals, int rows, int parts, uint32_t shift, uint32_t flip, int64_t n,
-    int64_t chunk) {
+    int64_t chunk, uint32_t limit) {
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
   constexpr int NT = NW * kWave, TILE = NT * IT;
@@ -392,6 +393,7 @@ __global__ __launch_bounds__(NW * kWave, 4) void sort_scatter_kernel(
 
     auto put = [&](int p, uint32_t d, uint32_t raw, uint32_t val) {
       const uint32_t dst = s_gofs[d] + (uint32_t)p;
+      if (LIMIT && dst >= limit) return;
       if constexpr (!BIG) {
         *reinterpret_cast<Raw*>(reinterpret_cast<char*>(kout) + dst * (uint32_t)sizeof(Raw)) = (Raw)raw;
         *reinterpret_cast<int32_t*>(reinterpret_cast<char*>(vout) + dst * 4u) = (int32_t)val;
@@ -460,7 +462,8 @@ constexpr int64_t kSortBlockMax = (int64_t)kSortBlockThreads * kSortBlockIT;
 template <int DT>
 __global__ __launch_bounds__(kSortBlockThreads) void sort_block_kernel(
     const typename SortKey<DT>::Raw* __restrict__ x, const int32_t* __restrict__ idx_in,
-    typename SortKey<DT>::Raw* __restrict__ out_x, int32_t* __restrict__ out_idx, int n, uint32_t flip) {
+    typename SortKey<DT>::Raw* __restrict__ out_x, int32_t* __restrict__ out_idx, int n, uint32_t flip,
+    int limit) {
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
   constexpr int NW = kSortBlockThreads / kWave, IT = kSortBlockIT, P = KT::kBits / 8;
@@ -529,7 +532,7 @@ __global__ __launch_bounds__(kSortBlockThreads) void sort_block_kernel(
       }
     }
   }
-  for (int p = tid; p < n; p += kSortBlockThreads) {
+  for (int p = tid; p < limit; p += kSortBlockThreads) {
     const uint64_t e = s_item[p];
     out_x[p] = (Raw)e;
     out_idx[p] = (int32_t)(uint32_t)(e >> 32);
@@ -596,13 +599,14 @@ struct SortArgs {
   const uint32_t *counts, *totals;
   uint32_t shift, flip;
   int64_t n;
+  uint32_t limit;  // outputs of the last pass, n of the others
 };
 
-template <int DT, bool GEN, int NW, int IT, bool BIG = false>
+template <int DT, bool GEN, int NW, int IT, bool BIG = false, bool LIMIT = false>
 static void sort_scatter_launch(const SortLayout& L, const SortArgs<DT>& a, hipStream_t st) {
-  hipLaunchKernelGGL((sort_scatter_kernel<DT, GEN, NW, IT, BIG>), dim3(L.chunks), dim3(NW * kWave), 0, st, a.kin,
+  hipLaunchKernelGGL((sort_scatter_kernel<DT, GEN, NW, IT, BIG, LIMIT>), dim3(L.chunks), dim3(NW * kWave), 0, st, a.kin,
                      a.vin, a.kout, a.vout, a.counts, a.totals, L.chunks * L.parts, L.parts, a.shift, a.flip, a.n,
-                     L.chunk);
+                     L.chunk, a.limit);
 }
 
 // A tile as large as the LDS of a compute unit allows for the wide form:
@@ -610,7 +614,9 @@ static void sort_scatter_launch(const SortLayout& L, const SortArgs<DT>& a, hipS
 template <int DT, bool GEN>
 static void sort_scatter(const SortLayout& L, const SortArgs<DT>& a, hipStream_t st) {
   constexpr int IT = GEN && SortKey<DT>::kBits <= 16 ? 32 : 16;
-  if (!L.wide) {
+  if (!L.wide && a.limit < a.n) {
+    sort_scatter_launch<DT, GEN, 8, 8, false, true>(L, a, st);
+  } else if (!L.wide) {
     sort_scatter_launch<DT, GEN, 8, 8>(L, a, st);
   } else if (a.n < ((int64_t)1 << 30)) {
     sort_scatter_launch<DT, GEN, 16, IT>(L, a, st);
@@ -619,9 +625,13 @@ static void sort_scatter(const SortLayout& L, const SortArgs<DT>& a, hipStream_t
   }
 }
 
+// The first k outputs to out_x and out_idx; passes before the last alternate
+// between scratch and mid_x / mid_idx, of n elements each (out_x and out_idx
+// themselves when k == n).  k < n only for keys that do not take the wide
+// form.
 template <int DT>
-static int sort_run(const void* x, const int32_t* idx_in, void* out_x, int32_t* out_idx, int64_t n, bool desc,
-                    void* scratch, hipStream_t st) {
+static int sort_run(const void* x, const int32_t* idx_in, void* mid_x, int32_t* mid_idx, void* out_x,
+                    int32_t* out_idx, int64_t n, int64_t k, bool desc, void* scratch, hipStream_t st) {
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
   constexpr int P = KT::kBits / 8;
@@ -632,7 +642,7 @@ static int sort_run(const void* x, const int32_t* idx_in, void* out_x, int32_t* 
   a.vin = idx_in;
   if (n <= kSortBlockMax) {
     hipLaunchKernelGGL((sort_block_kernel<DT>), dim3(1), dim3(kSortBlockThreads), 0, st, a.kin, idx_in,
-                       static_cast<Raw*>(out_x), out_idx, (int)n, a.flip);
+                       static_cast<Raw*>(out_x), out_idx, (int)n, a.flip, (int)k);
     TCS_CHECK_LAUNCH();
     return TCS_OK;
   }
@@ -644,10 +654,12 @@ static int sort_run(const void* x, const int32_t* idx_in, void* out_x, int32_t* 
   a.counts = counts;
   a.totals = totals;
   for (int p = 0; p < P; ++p) {
-    // The last pass writes the outputs; earlier ones alternate so that it does.
-    const bool to_out = ((P - 1 - p) % 2) == 0;
-    a.kout = to_out ? static_cast<Raw*>(out_x) : reinterpret_cast<Raw*>(sc);
-    a.vout = to_out ? out_idx : reinterpret_cast<int32_t*>(sc + L.tmpv_off);
+    // The last pass writes the outputs; earlier ones alternate so that it
+    // does not read what it writes.
+    const bool last = p == P - 1, mid = (P - 1 - p) % 2 == 0;
+    a.kout = last ? static_cast<Raw*>(out_x) : (mid ? static_cast<Raw*>(mid_x) : reinterpret_cast<Raw*>(sc));
+    a.vout = last ? out_idx : (mid ? mid_idx : reinterpret_cast<int32_t*>(sc + L.tmpv_off));
+    a.limit = (uint32_t)(last ? k : n);
     a.shift = 8u * (uint32_t)p;
     if (L.wide) {
       hipLaunchKernelGGL((sort_count_kernel<DT, 4>), dim3(rows), dim3(kSortThreads), 0, st, a.kin, n,
@@ -672,6 +684,33 @@ static int sort_run(const void* x, const int32_t* idx_in, void* out_x, int32_t* 
     a.vin = a.vout;
   }
   return TCS_OK;
+}
+
+static int sort_any(const void* x, int dtype, const int32_t* idx_in, void* mid_x, int32_t* mid_idx, void* out_x,
+                    int32_t* out_idx, int64_t n, int64_t k, bool desc, void* scratch, hipStream_t st) {
+  auto run = [&](auto f) { return f(x, idx_in, mid_x, mid_idx, out_x, out_idx, n, k, desc, scratch, st); };
+  switch (dtype) {
+    case TCS_F16: return run(sort_run<TCS_F16>);
+    case TCS_BF16: return run(sort_run<TCS_BF16>);
+    case TCS_F32: return run(sort_run<TCS_F32>);
+    case TCS_I8: return run(sort_run<TCS_I8>);
+    case TCS_I16: return run(sort_run<TCS_I16>);
+    case TCS_I32: return run(sort_run<TCS_I32>);
+    default: return run(sort_run<TCS_U32>);
+  }
+}
+
+// The second temporary copy follows the sort's own scratch.
+size_t sort_first_scratch_bytes(int64_t n, int dtype) {
+  return sort_layout(n, dtype).scratch + align256((size_t)n * sort_elem_bytes(dtype)) + (size_t)n * 4;
+}
+
+int sort_first(const void* x, int dtype, void* out_x, int32_t* out_idx, int64_t n, int64_t k, bool descending,
+               void* scratch, hipStream_t st) {
+  char* mid = static_cast<char*>(scratch) + sort_layout(n, dtype).scratch;
+  if (k < n && n > kSortWideMin) return TCS_ERR_INVALID_ARG;
+  return sort_any(x, dtype, nullptr, mid, reinterpret_cast<int32_t*>(mid + align256((size_t)n * sort_elem_bytes(dtype))),
+                  out_x, out_idx, n, k, descending, scratch, st);
 }
 
 }  // namespace tcs
@@ -700,16 +739,7 @@ int tcs_sort(const void* x, int dtype, const int32_t* idx_in, void* out_x, int32
   const SortLayout L = sort_layout(n, dtype);
   if (!workspace || workspace_bytes < lookback_ws_bytes(0) || !scratch || scratch_bytes < L.scratch) return TCS_ERR_WORKSPACE;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const bool d = descending != 0;
-  switch (dtype) {
-    case TCS_F16: return sort_run<TCS_F16>(x, idx_in, out_x, out_idx, n, d, scratch, st);
-    case TCS_BF16: return sort_run<TCS_BF16>(x, idx_in, out_x, out_idx, n, d, scratch, st);
-    case TCS_F32: return sort_run<TCS_F32>(x, idx_in, out_x, out_idx, n, d, scratch, st);
-    case TCS_I8: return sort_run<TCS_I8>(x, idx_in, out_x, out_idx, n, d, scratch, st);
-    case TCS_I16: return sort_run<TCS_I16>(x, idx_in, out_x, out_idx, n, d, scratch, st);
-    case TCS_I32: return sort_run<TCS_I32>(x, idx_in, out_x, out_idx, n, d, scratch, st);
-    default: return sort_run<TCS_U32>(x, idx_in, out_x, out_idx, n, d, scratch, st);
-  }
+  return sort_any(x, dtype, idx_in, out_x, out_idx, out_x, out_idx, n, n, descending != 0, scratch, st);
 }
 
 }  // extern "C"

@@ -2,20 +2,37 @@
 // of the k-th largest value.
 //
 // tcs_topk replaces run_topk_fp16 / run_topk_int16 (src/torch/torch_topk.h:
-// 69-207; the reference narrows [x_min, x_max] with parallel splits).  Here
-// the k-th largest order key T is found one 8-bit digit at a time, from the
-// top: a histogram of digit r over the keys whose higher digits equal the
-// digits chosen so far, then one workgroup picks the bin holding the k-th
-// largest.  State passes between launches in the workspace, so no result
-// reaches the host until the end.  An ordered selection then takes every
-// key above T and the first `need` keys equal to T in input order (per-tile
-// counts, their scan, and placement by the tiles that hold any of them),
-// and the stable radix sort orders those k, largest first (ties by input
-// position).  The per-tile counts of keys of two or more bytes come from a
-// record the last digit round keeps (keys above the higher digits, low
-// bytes of the few matching them), so reads are one pass per key byte plus
-// the tiles that hold selected keys (one-byte keys: one more pass for the
-// tile counts).
+// 69-207; the reference narrows [x_min, x_max] with parallel splits).  By
+// size (topk_run):
+//
+// Few keys: the radix sort, whose last pass writes the first k only.
+//
+// Many keys, k <= kTkRankMax: one pass over the keys keeps the largest order
+// key of every sub-chunk and of every group of sub-chunks.  The k-th largest
+// group maximum, ties to the lowest sub-chunk, bounds the k-th key from below
+// (k groups each hold a key at or above it), so only the sub-chunks whose
+// maximum reaches it are read again, and their keys at or above it, about
+// 1.15 k of them when the keys are in no particular order, are ranked by
+// counting.  If they do not fit (the largest keys lie together), the radix
+// select below runs instead: its kernels are launched behind this path and
+// leave at once when it has succeeded, so nothing waits for the host.  2^28
+// fp16 normals, k = 2048: 134 us, of which the read takes 94, the select's two
+// reads and eleven launches 278; sorted keys, which give too many candidates,
+// 600 against 429.
+//
+// Otherwise radix select: the k-th largest order key T is found one 8-bit
+// digit at a time, from the top: a histogram of digit r over the keys whose
+// higher digits equal the digits chosen so far, then one workgroup picks the
+// bin holding the k-th largest.  State passes between launches in the
+// workspace, so no result reaches the host until the end.  An ordered
+// selection then takes every key above T and the first `need` keys equal to
+// T in input order (per-tile counts, their scan, and placement by the tiles
+// that hold any of them), and those k are ranked by counting or, when they
+// are many, by the radix sort (ties by input position).  The per-tile counts
+// of keys of two or more bytes come from a record the last digit round keeps
+// (keys above the higher digits, low bytes of the few matching them), so
+// reads are one pass per key byte plus the tiles that hold selected keys
+// (one-byte keys: one more pass for the tile counts).
 //
 // tcs_topk_pivot follows run_topk_pivot_fp16 (src/torch/torch_topk.h:
 // 23-60, src/kernels/kernel_topk_pivot.h): per block, over its first eight
@@ -57,6 +74,90 @@ constexpr int kTkMaxChunkTiles = 256;
 
 inline int64_t topk_tile(int key_bytes) { return (int64_t)kTkNW * (key_bytes <= 2 ? 4 : 2) * kWave * kTkG; }
 
+// The kernels of the radix select take `gate`: null, or the candidate count
+// of the maxima path, which has succeeded when the count fits.
+constexpr uint32_t kTkCandMax = 8192;  // 64 KiB of LDS
+__device__ __forceinline__ bool topk_done(const uint32_t* gate) { return gate && *gate <= kTkCandMax; }
+
+// Behind a gate the last workgroup of a launch also runs the small step that
+// follows (a launch that leaves at once still takes about 4 us in the
+// stream).  What the workgroups leave for it they write, and it reads, with
+// device-scope accesses, which need no fence (a fence in every workgroup
+// writes back and invalidates the L2s: 2^28 keys, 1300 us); a workgroup
+// arrives when its own writes have left.  `arrived` is zero at the launch's
+// start and again after it.
+__device__ __forceinline__ bool topk_last_arrival(uint32_t* arrived) {
+  __shared__ uint32_t s_ticket;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    s_ticket = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (s_ticket == gridDim.x - 1) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return s_ticket == gridDim.x - 1;
+}
+template <bool SHARED>
+__device__ __forceinline__ uint64_t topk_read(const uint64_t* p) {
+  return SHARED ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
+}
+__device__ __forceinline__ void topk_leave(uint64_t* p, uint64_t v, bool shared) {
+  if (shared) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    *p = v;
+  }
+}
+
+// Picks digit r of the k-th largest key: the bin b where the count of keys
+// in bins >= b first reaches the number still to take.  One workgroup of NT
+// threads.
+template <int NT, bool SHARED>
+__device__ __forceinline__ void topk_pick(const uint64_t* partial, int groups, int r, int first, int64_t k,
+                                          uint64_t* state) {
+  constexpr int NQ = NT / 256;
+  const int tid = threadIdx.x, d = tid & 255, q = tid >> 8;
+  uint32_t s = 0;
+  int g = q;
+  for (; g + 7 * NQ < groups; g += 8 * NQ) {  // eight loads in flight
+    uint64_t v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = topk_read<SHARED>(&partial[(size_t)(g + NQ * u) * 256 + d]);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += (uint32_t)v[u];
+  }
+  for (; g < groups; g += NQ) s += (uint32_t)topk_read<SHARED>(&partial[(size_t)g * 256 + d]);
+  __shared__ uint32_t sr[NQ][256];
+  __shared__ uint32_t ws[4];
+  __shared__ uint64_t s_state[2];
+  sr[q][d] = s;
+  if (tid == 0) {
+    s_state[0] = first ? 0 : state[0];
+    s_state[1] = first ? (uint64_t)k : state[1];
+  }
+  __syncthreads();
+  // suffix[b] = keys in bins >= b: an inclusive scan over b' = 255 - b.
+  uint32_t cnt = 0, incl = 0;
+  if (tid < 256) {
+#pragma unroll
+    for (int e = 0; e < NQ; ++e) cnt += sr[e][255 - tid];
+    incl = wave_incl_scan(cnt);
+    if (__lane_id() == kWave - 1) ws[tid / kWave] = incl;
+  }
+  __syncthreads();
+  if (tid < 256) {
+    uint32_t before = 0;
+    for (int w = 0; w < tid / kWave; ++w) before += ws[w];
+    const uint64_t suffix = before + incl;  // keys in bins >= 255 - tid
+    const uint64_t need = s_state[1];
+    if (suffix >= need && suffix - cnt < need) {
+      const uint32_t b = 255u - (uint32_t)tid;
+      state[0] = s_state[0] | ((uint64_t)b << (8 * r));
+      state[1] = need - (suffix - cnt);
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Digit histogram among the keys matching the chosen higher digits.
 // state[0]: key digits chosen so far; state[1]: how many of the keys
@@ -71,10 +172,12 @@ inline int64_t topk_tile(int key_bytes) { return (int64_t)kTkNW * (key_bytes <= 
 template <int DT, bool FUSE>
 __global__ __launch_bounds__(kTkThreads) void topk_hist_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
                                                                int64_t n, int64_t chunk, uint32_t flip, int r,
-                                                               const uint64_t* __restrict__ state,
-                                                               uint64_t* __restrict__ partial,
+                                                               int64_t k_all, uint64_t* state, uint64_t* partial,
                                                                uint64_t* __restrict__ tstat,
-                                                               uint8_t* __restrict__ tlist) {
+                                                               uint8_t* __restrict__ tlist,
+                                                               const uint32_t* __restrict__ gate,
+                                                               uint32_t* __restrict__ arrived) {
+  if (topk_done(gate)) return;
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
   constexpr int NWV = kTkThreads / kWave, C = 4, NH = NWV * C;
@@ -182,7 +285,7 @@ __global__ __launch_bounds__(kTkThreads) void topk_hist_kernel(const typename So
     uint32_t s = 0;
 #pragma unroll
     for (int w = 0; w < NH; ++w) s += h[w][e];
-    partial[(size_t)blockIdx.x * 256 + e] = s;
+    topk_leave(&partial[(size_t)blockIdx.x * 256 + e], s, gate != nullptr);
   }
   if constexpr (FUSE) {
     const int64_t t0 = c0 / TILE;
@@ -194,6 +297,8 @@ __global__ __launch_bounds__(kTkThreads) void topk_hist_kernel(const typename So
     for (int e = tid; e < ntl * kTkListMax; e += kTkThreads)
       tlist[t0 * kTkListMax + e] = s_list[e / kTkListMax][e % kTkListMax];
   }
+  // Behind a gate the last workgroup picks the digit.
+  if (gate && topk_last_arrival(arrived)) topk_pick<kTkThreads, true>(partial, gridDim.x, r, hs >= KT::kBits, k_all, state);
 }
 
 // First level of the digit-count sum: workgroup q adds the partials of
@@ -218,50 +323,10 @@ __global__ __launch_bounds__(256) void topk_sum_kernel(const uint64_t* __restric
   psum[(size_t)blockIdx.x * 256 + d] = s;
 }
 
-// Picks digit r of the k-th largest key: the bin b where the count of keys
-// in bins >= b first reaches the number still to take.
 __global__ __launch_bounds__(kTkPickThreads) void topk_pick_kernel(const uint64_t* __restrict__ partial,
                                                                    int groups, int r, int first, int64_t k,
                                                                    uint64_t* __restrict__ state) {
-  const int tid = threadIdx.x, d = tid & 255, q = tid >> 8;
-  uint32_t s = 0;
-  int g = q;
-  for (; g + 28 < groups; g += 32) {  // eight loads in flight
-    uint64_t v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = partial[(size_t)(g + 4 * u) * 256 + d];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += (uint32_t)v[u];
-  }
-  for (; g < groups; g += 4) s += (uint32_t)partial[(size_t)g * 256 + d];
-  __shared__ uint32_t sr[4][256];
-  __shared__ uint32_t ws[4];
-  __shared__ uint64_t s_state[2];
-  sr[q][d] = s;
-  if (tid == 0) {
-    s_state[0] = first ? 0 : state[0];
-    s_state[1] = first ? (uint64_t)k : state[1];
-  }
-  __syncthreads();
-  // suffix[b] = keys in bins >= b: an inclusive scan over b' = 255 - b.
-  uint32_t cnt = 0, incl = 0;
-  if (tid < 256) {
-    cnt = sr[0][255 - tid] + sr[1][255 - tid] + sr[2][255 - tid] + sr[3][255 - tid];
-    incl = wave_incl_scan(cnt);
-    if (__lane_id() == kWave - 1) ws[tid / kWave] = incl;
-  }
-  __syncthreads();
-  if (tid < 256) {
-    uint32_t before = 0;
-    for (int w = 0; w < tid / kWave; ++w) before += ws[w];
-    const uint64_t suffix = before + incl;  // keys in bins >= 255 - tid
-    const uint64_t need = s_state[1];
-    if (suffix >= need && suffix - cnt < need) {
-      const uint32_t b = 255u - (uint32_t)tid;
-      state[0] = s_state[0] | ((uint64_t)b << (8 * r));
-      state[1] = need - (suffix - cnt);
-    }
-  }
+  topk_pick<kTkPickThreads, false>(partial, groups, r, first, k, state);
 }
 
 // ---------------------------------------------------------------------------
@@ -318,93 +383,20 @@ __device__ __forceinline__ void topk_classify_any(const typename SortKey<DT>::Ra
   }
 }
 
-// tcnt[tile] = (keys above T) << 32 | (keys equal to T) in the tile.
-template <int DT>
-__global__ __launch_bounds__(kTkNW * kWave) void topk_tilecount_kernel(
-    const typename SortKey<DT>::Raw* __restrict__ x, int64_t n, uint32_t flip,
-    const uint64_t* __restrict__ state, uint64_t* __restrict__ tcnt) {
-  constexpr int J = TopkGeom<DT>::J, NW = kTkNW;
-  __shared__ int s_w[NW];
-  const int lane = __lane_id(), wid = threadIdx.x / kWave;
-  Packed<typename SortKey<DT>::Raw, kTkG> xv[J];
-  uint32_t gtb[J], eqb[J];
-  topk_classify_any<DT>(x, n, flip, (uint32_t)state[0], blockIdx.x, wid, lane, xv, gtb, eqb);
-  int c = 0;
-#pragma unroll
-  for (int j = 0; j < J; ++j) c += (__builtin_popcount(gtb[j]) << 16) | __builtin_popcount(eqb[j]);
-  c = wave_sum(c);
-  if (lane == 0) s_w[wid] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int t = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) t += s_w[w];
-    tcnt[blockIdx.x] = ((uint64_t)((uint32_t)t >> 16) << 32) | ((uint32_t)t & 0xffffu);
-  }
-}
-
-// tcnt[tile] as topk_tilecount_kernel writes it, from the record of the
-// last digit round: keys above T are those whose higher digits are above
-// T's plus the recorded matching keys whose low byte is above T's, keys
-// equal to T the recorded ones with T's low byte.  A tile with more matching
-// keys than were recorded is counted from its keys.  One wave per tile.
-template <int DT>
-__global__ __launch_bounds__(256) void topk_tilefix_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
-                                                           int64_t n, uint32_t flip,
-                                                           const uint64_t* __restrict__ state,
-                                                           const uint64_t* __restrict__ tstat,
-                                                           const uint8_t* __restrict__ tlist,
-                                                           uint64_t* __restrict__ tcnt, uint32_t tiles) {
-  using KT = SortKey<DT>;
-  using Raw = typename KT::Raw;
-  constexpr int64_t TILE = TopkGeom<DT>::kTile;
-  constexpr int V = 16 / (int)sizeof(Raw);
-  const int lane = __lane_id();
-  const uint32_t tile = blockIdx.x * (256 / kWave) + threadIdx.x / kWave;
-  if (tile >= tiles) return;
-  const uint32_t T = (uint32_t)state[0];
-  const uint64_t rec = tstat[tile];
-  const uint32_t m = (uint32_t)rec & 0xffffu;
-  uint32_t g, e;
-  if (m <= (uint32_t)kTkListMax) {
-    const bool in = lane < (int)m;
-    const uint32_t low = in ? (uint32_t)tlist[(size_t)tile * kTkListMax + lane] : 0u;
-    g = (uint32_t)(rec >> 32) + (uint32_t)__popcll(__ballot(in && low > (T & 0xffu)));
-    e = (uint32_t)__popcll(__ballot(in && low == (T & 0xffu)));
-  } else {
-    const int64_t t0 = (int64_t)tile * TILE;
-    const int64_t t1 = t0 + TILE < n ? t0 + TILE : n;
-    uint32_t gl = 0, el = 0;
-    for (int64_t b = t0 + (int64_t)lane * V; b < t1; b += (int64_t)kWave * V) {
-      Raw v[V];
-      load_items<Raw, V>(x, b, t1, v);
-#pragma unroll
-      for (int i = 0; i < V; ++i) {
-        const uint32_t kk = KT::key(v[i]) ^ flip;
-        const bool ok = b + i < t1;
-        gl += ok && kk > T ? 1u : 0u;
-        el += ok && kk == T ? 1u : 0u;
-      }
-    }
-    g = (uint32_t)wave_sum((int)gl);
-    e = (uint32_t)wave_sum((int)el);
-  }
-  if (lane == 0) tcnt[tile] = ((uint64_t)g << 32) | e;
-}
-
 // In place: tcnt[t] = sum of tcnt over the tiles before t, for t in
-// [0, tiles]; one workgroup, 16384 tiles per round.  Wave w takes the
+// [0, tiles]; one workgroup of NT
+// threads, 16 NT tiles per round.  Wave w takes the
 // round's tiles [w * 1024, (w + 1) * 1024), lane l tiles w * 1024 + 64q + l
 // (coalesced loads and stores: 16 consecutive tiles per thread put every
 // lane of a load in a different line, 17.8 us per scan of 16384 tiles),
 // scanned as 16 wave scans in order.  The packed halves sum without a carry
 // (each total is below 2^31).
 constexpr int kTkScanThreads = 1024, kTkScanPer = 16;
-__global__ __launch_bounds__(kTkScanThreads) void topk_tilescan_kernel(uint64_t* __restrict__ tcnt,
-                                                                       uint32_t tiles) {
-  constexpr int NWV = kTkScanThreads / kWave;
+template <int NT, bool SHARED>
+__device__ __forceinline__ void topk_tilescan(uint64_t* tcnt, uint32_t tiles) {
+  constexpr int NWV = NT / kWave;
   constexpr int64_t WSPAN = (int64_t)kWave * kTkScanPer;
-  constexpr int64_t ROUND = (int64_t)kTkScanThreads * kTkScanPer;
+  constexpr int64_t ROUND = (int64_t)NT * kTkScanPer;
   __shared__ int64_t s_w[NWV];
   const int tid = threadIdx.x, lane = __lane_id(), wid = tid / kWave;
   int64_t carry = 0;
@@ -412,7 +404,7 @@ __global__ __launch_bounds__(kTkScanThreads) void topk_tilescan_kernel(uint64_t*
     const int64_t wb = r0 + (int64_t)wid * WSPAN + lane;
     int64_t v[kTkScanPer];
 #pragma unroll
-    for (int q = 0; q < kTkScanPer; ++q) v[q] = wb + q * kWave < tiles ? (int64_t)tcnt[wb + q * kWave] : 0;
+    for (int q = 0; q < kTkScanPer; ++q) v[q] = wb + q * kWave < tiles ? (int64_t)topk_read<SHARED>(&tcnt[wb + q * kWave]) : 0;
     int64_t run = 0;  // the wave's tiles before row q
 #pragma unroll
     for (int q = 0; q < kTkScanPer; ++q) {
@@ -439,6 +431,95 @@ __global__ __launch_bounds__(kTkScanThreads) void topk_tilescan_kernel(uint64_t*
   if (tid == 0) tcnt[tiles] = (uint64_t)carry;
 }
 
+// tcnt[tile] = (keys above T) << 32 | (keys equal to T) in the tile.
+template <int DT>
+__global__ __launch_bounds__(kTkNW * kWave) void topk_tilecount_kernel(
+    const typename SortKey<DT>::Raw* __restrict__ x, int64_t n, uint32_t flip,
+    const uint64_t* __restrict__ state, uint64_t* tcnt, const uint32_t* __restrict__ gate,
+    uint32_t* __restrict__ arrived) {
+  constexpr int J = TopkGeom<DT>::J, NW = kTkNW;
+  if (topk_done(gate)) return;
+  __shared__ int s_w[NW];
+  const int lane = __lane_id(), wid = threadIdx.x / kWave;
+  Packed<typename SortKey<DT>::Raw, kTkG> xv[J];
+  uint32_t gtb[J], eqb[J];
+  topk_classify_any<DT>(x, n, flip, (uint32_t)state[0], blockIdx.x, wid, lane, xv, gtb, eqb);
+  int c = 0;
+#pragma unroll
+  for (int j = 0; j < J; ++j) c += (__builtin_popcount(gtb[j]) << 16) | __builtin_popcount(eqb[j]);
+  c = wave_sum(c);
+  if (lane == 0) s_w[wid] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int t = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) t += s_w[w];
+    topk_leave(&tcnt[blockIdx.x], ((uint64_t)((uint32_t)t >> 16) << 32) | ((uint32_t)t & 0xffffu), gate != nullptr);
+  }
+  // Behind a gate the last workgroup scans the counts.
+  if (gate && topk_last_arrival(arrived)) topk_tilescan<kTkNW * kWave, true>(tcnt, gridDim.x);
+}
+
+// tcnt[tile] as topk_tilecount_kernel writes it, from the record of the
+// last digit round: keys above T are those whose higher digits are above
+// T's plus the recorded matching keys whose low byte is above T's, keys
+// equal to T the recorded ones with T's low byte.  A tile with more matching
+// keys than were recorded is counted from its keys.  One wave per tile.
+template <int DT>
+__global__ __launch_bounds__(256) void topk_tilefix_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
+                                                           int64_t n, uint32_t flip,
+                                                           const uint64_t* __restrict__ state,
+                                                           const uint64_t* __restrict__ tstat,
+                                                           const uint8_t* __restrict__ tlist,
+                                                           uint64_t* tcnt, uint32_t tiles,
+                                                           const uint32_t* __restrict__ gate,
+                                                           uint32_t* __restrict__ arrived) {
+  if (topk_done(gate)) return;
+  using KT = SortKey<DT>;
+  using Raw = typename KT::Raw;
+  constexpr int64_t TILE = TopkGeom<DT>::kTile;
+  constexpr int V = 16 / (int)sizeof(Raw);
+  const int lane = __lane_id();
+  const uint32_t tile = blockIdx.x * (256 / kWave) + threadIdx.x / kWave;
+  if (tile < tiles) {
+    const uint32_t T = (uint32_t)state[0];
+    const uint64_t rec = tstat[tile];
+    const uint32_t m = (uint32_t)rec & 0xffffu;
+    uint32_t g, e;
+    if (m <= (uint32_t)kTkListMax) {
+      const bool in = lane < (int)m;
+      const uint32_t low = in ? (uint32_t)tlist[(size_t)tile * kTkListMax + lane] : 0u;
+      g = (uint32_t)(rec >> 32) + (uint32_t)__popcll(__ballot(in && low > (T & 0xffu)));
+      e = (uint32_t)__popcll(__ballot(in && low == (T & 0xffu)));
+    } else {
+      const int64_t t0 = (int64_t)tile * TILE;
+      const int64_t t1 = t0 + TILE < n ? t0 + TILE : n;
+      uint32_t gl = 0, el = 0;
+      for (int64_t b = t0 + (int64_t)lane * V; b < t1; b += (int64_t)kWave * V) {
+        Raw v[V];
+        load_items<Raw, V>(x, b, t1, v);
+  #pragma unroll
+        for (int i = 0; i < V; ++i) {
+          const uint32_t kk = KT::key(v[i]) ^ flip;
+          const bool ok = b + i < t1;
+          gl += ok && kk > T ? 1u : 0u;
+          el += ok && kk == T ? 1u : 0u;
+        }
+      }
+      g = (uint32_t)wave_sum((int)gl);
+      e = (uint32_t)wave_sum((int)el);
+    }
+    if (lane == 0) topk_leave(&tcnt[tile], ((uint64_t)g << 32) | e, gate != nullptr);
+  }
+  // Behind a gate the last workgroup scans the counts.
+  if (gate && topk_last_arrival(arrived)) topk_tilescan<256, true>(tcnt, tiles);
+}
+
+__global__ __launch_bounds__(kTkScanThreads) void topk_tilescan_kernel(uint64_t* __restrict__ tcnt,
+                                                                       uint32_t tiles) {
+  topk_tilescan<kTkScanThreads, false>(tcnt, tiles);
+}
+
 // One wave per tile, no workgroup barrier: wave w of the grid takes tiles
 // w, w + W, ... (W waves in all), reads the counts of 64 of them at once
 // and ballots which place anything; for each such tile it reads the keys
@@ -450,13 +531,18 @@ __global__ __launch_bounds__(kTkScanThreads) void topk_tilescan_kernel(uint64_t*
 // tiles place; reading all of each took 31-39 us of the placement's 45-58
 // (scattered 32 KB reads run far below the streaming rate), reading only
 // the first 1 KB of each 4-5 us.
+// WORDS: the selected keys go to cand_w as rank words (topk_word), else as
+// values and positions.
 constexpr int kTkPlaceThreads = 256;
-template <int DT>
+__device__ __forceinline__ uint64_t topk_word(uint32_t key, uint32_t pos) { return ((uint64_t)~key << 32) | pos; }
+template <int DT, bool WORDS>
 __global__ __launch_bounds__(kTkPlaceThreads) void topk_place_kernel(
     const typename SortKey<DT>::Raw* __restrict__ x, int64_t n, uint32_t flip,
     const uint64_t* __restrict__ state, int64_t k, const uint64_t* __restrict__ tcnt,
     const uint64_t* __restrict__ tstat, typename SortKey<DT>::Raw* __restrict__ cand_v,
-    int32_t* __restrict__ cand_i, uint32_t num_tiles) {
+    int32_t* __restrict__ cand_i, uint64_t* __restrict__ cand_w, uint32_t num_tiles,
+    const uint32_t* __restrict__ gate) {
+  if (topk_done(gate)) return;
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
   constexpr int G = kTkG;
@@ -523,17 +609,21 @@ __global__ __launch_bounds__(kTkPlaceThreads) void topk_place_kernel(
           if ((gtb | eqb) != 0) {
             const int ex = incl - c;
             int64_t gp = gpos + (ex >> 16), ep = epos + (ex & 0xffff);
+            auto put = [&](int64_t at, Raw r, int64_t pos) {
+              if constexpr (WORDS) {
+                cand_w[at] = topk_word(KT::key(r) ^ flip, (uint32_t)pos);
+              } else {
+                cand_v[at] = r;
+                cand_i[at] = (int32_t)pos;
+              }
+            };
 #pragma unroll
             for (int i = 0; i < G; ++i) {
               if ((gtb >> i) & 1u) {
-                cand_v[gp] = xv[q][i];
-                cand_i[gp] = (int32_t)(gb + i);
+                put(gp, xv[q][i], gb + i);
                 ++gp;
               } else if ((eqb >> i) & 1u) {
-                if (ep < need) {
-                  cand_v[c_gt + ep] = xv[q][i];
-                  cand_i[c_gt + ep] = (int32_t)(gb + i);
-                }
+                if (ep < need) put(c_gt + ep, xv[q][i], gb + i);
                 ++ep;
               }
             }
@@ -621,101 +711,361 @@ __global__ __launch_bounds__(256) void topk_pivot_kernel(const uint16_t* __restr
   if (tid == 0) out[blockIdx.x] = best_r;
 }
 
-// Orders k <= kTkSmallSort selected keys in one workgroup: a bitonic sort
-// of 64-bit words (inverted order key << 32 | candidate index), so keys go
-// largest first by the order key after flip and equal keys keep candidate
-// order, which is input order: the order the stable radix sort gives, in one
-// launch instead of five.  The workgroup sorts P = 1024 E words; lane l of
-// wave w holds positions w * 64E + 64e + l, e < E, in registers, so the
-// compare-exchange steps of stride below 64 are lane shuffles, strides 64 to
-// 32E are swaps inside a lane, and only the larger strides go through LDS
-// with barriers (2^28 fp16, k = 2048: 36.8 us for the radix sort's five
-// launches, 21.7 us with every step in LDS).
-constexpr int kTkSmallSort = 4096, kTkSortThreads = 1024;
-template <int DT, int E>
-__global__ __launch_bounds__(kTkSortThreads) void topk_small_sort_kernel(
-    const typename SortKey<DT>::Raw* __restrict__ cand_v, const int32_t* __restrict__ cand_i, int k, uint32_t flip,
-    typename SortKey<DT>::Raw* __restrict__ out_v, int32_t* __restrict__ out_i) {
+// ---------------------------------------------------------------------------
+// Maxima path.  A sub-chunk is U vectors of 64 lanes of 16 bytes; wave g of
+// the grid takes the `per` sub-chunks from g * per (per <= 64): submax[s] =
+// the sub-chunk's largest order key, gcomp[g] = the group's largest << 32 |
+// ~(its first sub-chunk that holds it).  Reads at the streaming rate: seven
+// packed instructions map two 16-bit keys and one takes their maximum (2^28
+// fp16 keys 94 us, 5.7 TB/s; with plain loads 106).
+// ---------------------------------------------------------------------------
+constexpr int kTkMaxThreads = 256;
+
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  auto step = [&](uint32_t o) { v = v > o ? v : o; };
+  step(dpp_mov<kRowShr1>(v));
+  step(dpp_mov<kRowShr2>(v));
+  step(dpp_mov<kRowShr4>(v));
+  step(dpp_mov<kRowShr8>(v));
+  step(dpp_mov<kRowBcast15, 0xa>(v));
+  step(dpp_mov<kRowBcast31, 0xc>(v));
+  return (uint32_t)readlane((int)v, kWave - 1);
+}
+
+template <int DT, int U>
+struct TopkSub {
+  using Raw = typename SortKey<DT>::Raw;
+  static constexpr int V = 16 / (int)sizeof(Raw);
+  static constexpr int64_t kKeys = (int64_t)U * kWave * V;
+};
+
+template <int DT, int U>
+__global__ __launch_bounds__(kTkMaxThreads) void topk_max_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
+                                                                 int64_t n, uint32_t flip, int per, uint32_t subs,
+                                                                 uint32_t groups, uint32_t* __restrict__ submax,
+                                                                 uint64_t* __restrict__ gcomp,
+                                                                 uint32_t* __restrict__ state) {
   using KT = SortKey<DT>;
-  constexpr int P = kTkSortThreads * E, SEG = kWave * E;
-  static_assert(E == 2 || E == 4, "two or four words per lane");
-  __shared__ uint64_t s[P];
-  const int tid = threadIdx.x, lane = __lane_id();
-  const int seg = (tid / kWave) * SEG + lane;  // position of word 0
-  uint64_t a[E];
+  using Raw = typename KT::Raw;
+  constexpr int V = TopkSub<DT, U>::V;
+  constexpr int64_t SUB = TopkSub<DT, U>::kKeys;
+  const int lane = __lane_id();
+  // Candidates, counted by the gather kernel, and the gated arrivals.
+  if (blockIdx.x == 0 && threadIdx.x == 0) state[0] = state[8] = 0;
+  const uint32_t g = blockIdx.x * (kTkMaxThreads / kWave) + threadIdx.x / kWave;
+  if (g >= groups) return;
+  const uint32_t s0 = g * (uint32_t)per;
+  const uint32_t s1 = s0 + per < subs ? s0 + per : subs;
+  uint32_t mine = 0, best = 0, at = s0;
+  for (uint32_t s = s0; s < s1; ++s) {
+    const int64_t b = (int64_t)s * SUB + lane * V;
+    uint32_t m = 0;
+    if ((int64_t)(s + 1) * SUB <= n) {
+      Packed<Raw, V> v[U];
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int pos = seg + e * kWave;
-    a[e] = pos < k ? ((uint64_t)(~(KT::key(cand_v[pos]) ^ flip)) << 32) | (uint32_t)pos : ~0ull;
-  }
-  // Swaps inside the lane: words e and e + D (stride 64 D).
-  auto cas_regs = [&](int size, auto d_c) {
-    constexpr int D = decltype(d_c)::value;
+      for (int u = 0; u < U; ++u) {
+        const u32x4 q = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(x + b + u * (kWave * V)));
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      if ((e & D) == 0) {
-        const bool up = ((seg + e * kWave) & size) == 0;
-        const uint64_t x0 = a[e], x1 = a[e + D];
-        if ((x0 > x1) == up) {
-          a[e] = x1;
-          a[e + D] = x0;
-        }
+        for (int c = 0; c < 4; ++c) v[u].w[c] = q[c];
       }
-    }
-  };
-  for (int size = 2; size <= P; size <<= 1) {
-    int stride = size >> 1;
-    if (stride >= SEG) {
+      if constexpr (KT::kBits == 16) {
+        u16x2 mp = {0, 0};
 #pragma unroll
-      for (int e = 0; e < E; ++e) s[seg + e * kWave] = a[e];
-      __syncthreads();
-      for (; stride >= SEG; stride >>= 1) {
-        for (int t = tid; t < P / 2; t += kTkSortThreads) {
-          const int lo = 2 * t - (t & (stride - 1));  // the pair (lo, lo + stride), bit `stride` of lo clear
-          const bool up = (lo & size) == 0;            // this bitonic block ascends
-          const uint64_t x0 = s[lo], x1 = s[lo + stride];
-          if ((x0 > x1) == up) {
-            s[lo] = x1;
-            s[lo + stride] = x0;
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+          for (int i = 0; i < V / 2; ++i)
+            mp = __builtin_elementwise_max(mp, __builtin_bit_cast(u16x2, KT::pair(v[u].w[i]) ^ (flip * 0x10001u)));
+        }
+        m = mp[0] > mp[1] ? mp[0] : mp[1];
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+          for (int i = 0; i < V; ++i) {
+            const uint32_t k = KT::key(v[u][i]) ^ flip;
+            m = m > k ? m : k;
           }
         }
-        __syncthreads();
       }
-      // Each thread reads back only its own positions, which no thread
-      // touches again before the barrier of the next LDS phase.
+    } else {
 #pragma unroll
-      for (int e = 0; e < E; ++e) a[e] = s[seg + e * kWave];
-    }
-    if constexpr (E == 4) {
-      if (stride == 2 * kWave) {
-        cas_regs(size, std::integral_constant<int, 2>{});
-        stride >>= 1;
-      }
-    }
-    if (stride == kWave) {
-      cas_regs(size, std::integral_constant<int, 1>{});
-      stride >>= 1;
-    }
-    for (; stride > 0; stride >>= 1) {
-      const bool lo = (lane & stride) == 0;
+      for (int u = 0; u < U; ++u) {
+        Raw r[V];
+        load_items<Raw, V, false>(x, b + u * (kWave * V), n, r);
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const bool up = ((seg + e * kWave) & size) == 0;
-        const uint32_t blo = (uint32_t)__shfl_xor((int)(uint32_t)a[e], stride);
-        const uint32_t bhi = (uint32_t)__shfl_xor((int)(uint32_t)(a[e] >> 32), stride);
-        const uint64_t b = ((uint64_t)bhi << 32) | blo;
-        const uint64_t mn = a[e] < b ? a[e] : b, mx = a[e] < b ? b : a[e];
-        a[e] = lo == up ? mn : mx;
+        for (int i = 0; i < V; ++i) {
+          const uint32_t k = b + u * (kWave * V) + i < n ? KT::key(r[i]) ^ flip : 0u;
+          m = m > k ? m : k;
+        }
       }
+    }
+    m = wave_max(m);
+    if (lane == (int)(s - s0)) mine = m;
+    if (m > best) {
+      best = m;
+      at = s;
     }
   }
+  if (s0 + lane < s1) submax[s0 + lane] = mine;
+  if (lane == 0) gcomp[g] = ((uint64_t)best << 32) | (uint32_t)~at;
+}
+
+// state[1] = T, state[2] = P: the k-th largest of the groups' (maximum,
+// lowest sub-chunk first) is (T, sub-chunk P).  One workgroup, the maxima in
+// LDS; T two bits at a time from the top (the counts of maxima at or above
+// three trials by ballots: a histogram's atomics would meet in the few bins
+// the maxima fall into).  Short loops on purpose: code
+// unrolled over registers took as long to fetch as to run.
+constexpr int kTkBoundThreads = 1024;
+constexpr uint32_t kTkMaxGroupsM = 16384;
+__global__ __launch_bounds__(kTkBoundThreads) void topk_bound_kernel(const uint64_t* __restrict__ gcomp,
+                                                                     uint32_t groups,
+                                                                     const uint32_t* __restrict__ submax,
+                                                                     uint32_t subs, uint32_t k, int bits,
+                                                                     uint32_t* __restrict__ state) {
+  __shared__ uint32_t s_key[kTkMaxGroupsM];
+  __shared__ uint32_t s_row[kTkMaxGroupsM / kWave];
+  __shared__ uint32_t s_cnt[16][3], s_above, s_at[2];
+  const int tid = threadIdx.x, lane = __lane_id(), wid = tid / kWave;
+  for (uint32_t g0 = tid; g0 < groups; g0 += 8 * kTkBoundThreads) {  // eight loads in flight
+    uint64_t c[8];
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int pos = seg + e * kWave;
-    if (pos < k) {
-      const uint32_t c = (uint32_t)a[e];
-      out_v[pos] = cand_v[c];
-      out_i[pos] = cand_i[c];
+    for (int u = 0; u < 8; ++u) c[u] = gcomp[g0 + u * kTkBoundThreads < groups ? g0 + u * kTkBoundThreads : 0];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (g0 + u * kTkBoundThreads < groups) s_key[g0 + u * kTkBoundThreads] = (uint32_t)(c[u] >> 32);
+  }
+  if (tid < 48) (&s_cnt[0][0])[tid] = 0;
+  if (tid == 0) s_above = 0;
+  __syncthreads();
+  uint32_t T = 0;
+#pragma unroll 1
+  for (int b = bits - 2; b >= 0; b -= 2) {
+    uint32_t c[3] = {};
+#pragma unroll 1
+    for (uint32_t g0 = tid; g0 - lane < groups; g0 += 4 * kTkBoundThreads) {
+      uint32_t key[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) key[u] = s_key[(g0 + u * kTkBoundThreads) % kTkMaxGroupsM];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool in = g0 + u * kTkBoundThreads < groups;
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          c[e] += (uint32_t)__popcll(__ballot(in && key[u] >= (T | ((uint32_t)(e + 1) << b))));
+      }
+    }
+    if (lane < 3) atomicAdd(&s_cnt[b / 2][lane], lane == 0 ? c[0] : (lane == 1 ? c[1] : c[2]));
+    __syncthreads();
+    const uint32_t* sc = s_cnt[b / 2];
+    T |= (uint32_t)((sc[0] >= k) + (sc[1] >= k) + (sc[2] >= k)) << b;
+  }
+  // Groups above T, and those at T in every row of 64.
+  uint32_t above = 0;
+#pragma unroll 1
+  for (uint32_t g0 = wid * kWave; g0 < groups; g0 += kTkBoundThreads) {
+    const bool in = g0 + lane < groups;
+    const uint32_t key = in ? s_key[g0 + lane] : 0u;
+    above += (uint32_t)__popcll(__ballot(in && key > T));
+    const uint32_t e = (uint32_t)__popcll(__ballot(in && key == T));
+    if (lane == 0) s_row[g0 / kWave] = e;
+  }
+  if (lane == 0) atomicAdd(&s_above, above);
+  __syncthreads();
+  uint32_t need = k - s_above;  // >= 1: fewer than k maxima lie above T
+  // Wave 0: among e (one a lane), the lane that holds the need-th, or 64 with
+  // `need` less all of them.
+  auto find = [&](uint32_t e) {
+    const uint32_t incl = wave_incl_scan(e);
+    const uint64_t reach = __ballot(incl >= need);
+    if (reach == 0) {
+      need -= (uint32_t)readlane((int)incl, kWave - 1);
+      return kWave;
+    }
+    const int l = __builtin_ctzll(reach);
+    need -= (uint32_t)readlane((int)(incl - e), l);
+    return l;
+  };
+  if (need <= k / 4) {
+    // The row, and in it the group: the need-th at T in order.
+    if (wid != 0) return;
+    const int rows = (int)((groups + kWave - 1) / kWave);
+    int row = 0;
+#pragma unroll 1
+    for (int r0 = 0; r0 < rows; r0 += kWave) {
+      const int l = find(r0 + lane < rows ? s_row[r0 + lane] : 0u);
+      if (l < kWave) {
+        row = r0 + l;
+        break;
+      }
+    }
+    const uint32_t g = (uint32_t)row * kWave + lane;
+    const int l = find(g < groups && s_key[g] == T ? 1u : 0u);
+    if (lane == l) {
+      state[1] = T;
+      state[2] = ~(uint32_t)gcomp[g];
+    }
+    return;
+  }
+  // Many groups at T (a value that repeats): the need-th sub-chunk at T is as
+  // good a bound as the need-th group, and as much lower as a group holds
+  // sub-chunks at T.
+  constexpr int V = 16;
+#pragma unroll 1
+  for (uint32_t b = 0; b < subs; b += kTkBoundThreads * V) {
+    // Wave w takes 64 V sub-chunks from b + 64 V w, row by row.
+    uint32_t m[V];
+    const uint32_t wb = b + (uint32_t)wid * kWave * V + lane;
+#pragma unroll
+    for (int u = 0; u < V; ++u) m[u] = submax[wb + u * kWave < subs ? wb + u * kWave : 0];
+    __syncthreads();  // s_row was read
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      const uint32_t e = (uint32_t)__popcll(__ballot(wb + u * kWave < subs && m[u] == T));
+      if (lane == 0) s_row[wid * V + u] = e;
+    }
+    __syncthreads();
+    if (wid == 0) {
+      int row = -1;
+#pragma unroll 1
+      for (int r0 = 0; r0 < kTkBoundThreads / kWave * V && row < 0; r0 += kWave) {
+        const int l = find(s_row[r0 + lane]);
+        if (l < kWave) row = r0 + l;
+      }
+      if (lane == 0) {
+        s_at[0] = (uint32_t)row;
+        s_at[1] = need;
+      }
+    }
+    __syncthreads();
+    if ((int)s_at[0] >= 0) {
+      if ((int)s_at[0] / V == wid) {
+        need = s_at[1];
+        const uint32_t sub = b + s_at[0] * kWave + lane;
+        const int l = find(sub < subs && submax[sub] == T ? 1u : 0u);
+        if (lane == l) {
+          state[1] = T;
+          state[2] = sub;
+        }
+      }
+      return;
+    }
+  }
+}
+
+// Appends the keys above T, or equal to T in a sub-chunk up to P, as rank
+// words.  A wave looks at kTkGatherSubs sub-chunk maxima and reads the
+// sub-chunks that reach the bound; a workgroup's words meet in LDS and take
+// their place in cand_w with one atomic.  state[0] counts them all, stored
+// or not.
+constexpr int kTkGatherThreads = 512, kTkGatherSubs = 32;
+template <int DT, int U>
+__global__ __launch_bounds__(kTkGatherThreads) void topk_gather_kernel(
+    const typename SortKey<DT>::Raw* __restrict__ x, int64_t n, uint32_t flip, uint32_t subs,
+    const uint32_t* __restrict__ submax, uint32_t* __restrict__ state, uint64_t* __restrict__ cand_w) {
+  using KT = SortKey<DT>;
+  using Raw = typename KT::Raw;
+  constexpr int V = TopkSub<DT, U>::V;
+  constexpr int64_t SUB = TopkSub<DT, U>::kKeys;
+  constexpr uint32_t kList = 4096;
+  __shared__ uint64_t s_list[kList];
+  __shared__ uint32_t s_n, s_base;
+  const int tid = threadIdx.x, lane = __lane_id(), wid = tid / kWave;
+  if (tid == 0) s_n = 0;
+  const uint32_t T = state[1], P = state[2];
+  __syncthreads();
+  const uint32_t first = (blockIdx.x * (kTkGatherThreads / kWave) + wid) * kTkGatherSubs;
+  const uint32_t s = first + lane;
+  const bool look = lane < kTkGatherSubs && s < subs;
+  const uint32_t m = look ? submax[s] : 0u;
+  uint64_t active = __ballot(look && (m > T || (m == T && s <= P)));
+  // A workgroup whose list has overflowed has told the fallback enough.
+  while (active != 0 && __hip_atomic_load(&s_n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= kList) {
+    const int l = __builtin_ctzll(active);
+    active &= active - 1;
+    const uint32_t sub = first + l;
+    const int64_t b = (int64_t)sub * SUB + lane * V;
+    const uint32_t least = sub <= P ? T : T + 1;  // T + 1 wraps only if nothing is above T
+    const bool none = sub > P && T == 0xffffffffu;
+    auto take = [&](auto full_c) {
+      constexpr bool FULL = decltype(full_c)::value;
+      Packed<Raw, V> r[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) load_items<Raw, V, FULL>(x, b + u * (kWave * V), n, r[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          const int64_t p = b + u * (kWave * V) + i;
+          const uint32_t key = KT::key(r[u][i]) ^ flip;
+          if ((FULL || p < n) && key >= least && !none) {
+            const uint32_t q = atomicAdd(&s_n, 1u);
+            if (q < kList) s_list[q] = topk_word(key, (uint32_t)p);
+          }
+        }
+      }
+    };
+    if ((int64_t)(sub + 1) * SUB <= n) {
+      take(std::integral_constant<bool, true>{});
+    } else {
+      take(std::integral_constant<bool, false>{});
+    }
+  }
+  __syncthreads();
+  const uint32_t c = s_n;
+  if (c == 0) return;
+  // More than the list holds: the count alone tells the fallback.
+  if (tid == 0) s_base = atomicAdd(&state[0], c <= kList ? c : kTkCandMax + 1);
+  __syncthreads();
+  if (c > kList) return;
+  for (uint32_t q = tid; q < c; q += kTkGatherThreads)
+    if (s_base + q < kTkCandMax) cand_w[s_base + q] = s_list[q];
+}
+
+// Orders the candidates by counting: a word's rank is the number of smaller
+// words (all differ), and those ranked below k go to their place.  Every
+// workgroup holds all words in LDS; a wave ranks four at a time.  *count
+// words, or k when count is null or has outgrown the candidates (the radix
+// select has then placed exactly k).  2400 words 5 us, where a bitonic sort
+// in one workgroup took 17.
+constexpr int kTkRankThreads = 512, kTkRankBlocks = 256;
+constexpr int64_t kTkRankMax = 4096;
+template <int DT>
+__global__ __launch_bounds__(kTkRankThreads) void topk_rank_kernel(const uint64_t* __restrict__ cand_w,
+                                                                   const uint32_t* __restrict__ count,
+                                                                   const typename SortKey<DT>::Raw* __restrict__ x,
+                                                                   uint32_t k,
+                                                                   typename SortKey<DT>::Raw* __restrict__ out_v,
+                                                                   int32_t* __restrict__ out_i) {
+  constexpr int Q = 4;
+  __shared__ uint64_t s_w[kTkCandMax];
+  const int tid = threadIdx.x, lane = __lane_id();
+  uint32_t m = k;
+  if (count && *count <= kTkCandMax) m = *count;
+  const uint32_t first = (blockIdx.x * (kTkRankThreads / kWave) + tid / kWave) * Q;
+  if (blockIdx.x * (kTkRankThreads / kWave) * Q >= m) return;
+  // A whole row of 64 past the end, of words larger than any.
+  const uint32_t padded = (m + kWave - 1) / kWave * kWave;
+  for (uint32_t j = tid; j < padded; j += kTkRankThreads) s_w[j] = j < m ? cand_w[j] : ~0ull;
+  __syncthreads();
+  for (uint32_t i = first; i < m; i += kTkRankBlocks * (kTkRankThreads / kWave) * Q) {
+    uint64_t w[Q];
+    int c[Q] = {};
+#pragma unroll
+    for (int q = 0; q < Q; ++q) w[q] = s_w[i + q < m ? i + q : m - 1];
+    for (uint32_t j = lane; j < padded; j += kWave) {
+      const uint64_t o = s_w[j];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) c[q] += o < w[q] ? 1 : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const uint32_t rank = (uint32_t)wave_sum(c[q]);
+      if (lane == 0 && i + q < m && rank < k) {
+        const uint32_t pos = (uint32_t)w[q];
+        out_v[rank] = x[pos];
+        out_i[rank] = (int32_t)pos;
+      }
     }
   }
 }
@@ -726,12 +1076,12 @@ __global__ __launch_bounds__(kTkSortThreads) void topk_small_sort_kernel(
 // parallel.  2^28 fp16, k = 2048: a workgroup of 8 waves per tile (block
 // scans between the waves) took 42 us with 2048 workgroups of which about
 // 512 fit at once and 52 us with the resident grid.
-template <int DT>
+template <int DT, bool WORDS>
 static uint32_t topk_place_grid() {
   static std::atomic<int> cached[kMaxCachedDevices];
   return (uint32_t)device_cached(cached, [](int dev) {
     int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, topk_place_kernel<DT>, kTkPlaceThreads, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, topk_place_kernel<DT, WORDS>, kTkPlaceThreads, 0) !=
             hipSuccess ||
         per_cu < 1)
       per_cu = 1;
@@ -751,11 +1101,48 @@ inline int topk_elem_bytes(int dt) {
   }
 }
 
+// Sub-chunks of one vector (U = 1) up to 2^17 of them, of four above; groups
+// of `per` sub-chunks, 4096 of them or as many as leave the bound tight.
+struct TopkMaxima {
+  int U, per;
+  uint32_t subs, groups;
+};
+
+inline TopkMaxima topk_maxima(int64_t n, int64_t k, int key_bytes) {
+  TopkMaxima m{};
+  const int64_t vec = kWave * (16 / key_bytes);
+  m.U = n > vec << 17 ? 4 : 1;
+  m.subs = (uint32_t)((n + m.U * vec - 1) / (m.U * vec));
+  int64_t most = 4096;  // enough waves for the read, four times the winners
+  while (most < 4 * k && most < kTkMaxGroupsM) most *= 2;
+  m.per = (int)((m.subs + most - 1) / most);
+  if (m.per < 1) m.per = 1;
+  m.groups = (m.subs + m.per - 1) / m.per;
+  return m;
+}
+
+enum class TopkPath { kSort, kMaxima, kSelect };
+
+// The sort while its passes cost less than the maxima path's launches; the
+// maxima path where it has groups enough for its bound to be tight (three
+// times as many as winners: about 1.2 k candidates); the sort again up to
+// 2^21 or 2^22 more keys than that; the radix select beyond.  fp16, k = 300:
+// 2^21 keys 31 us sorted, 30 by maxima; k = 3000, 4e6 keys: 45 us sorted, the
+// select 114; fp32, k = 300: 5e5 keys 51 us sorted, 1e6 by maxima 44.
+inline TopkPath topk_path(const TopkMaxima& m, int64_t n, int64_t k, int key_bytes) {
+  if (n <= (key_bytes <= 2 ? (int64_t)1 << 21 : (int64_t)1 << 18)) return TopkPath::kSort;
+  if (k <= kTkRankMax && (int64_t)m.groups >= 3 * k && m.per <= kWave) return TopkPath::kMaxima;
+  return n <= (key_bytes <= 2 ? (int64_t)6 << 20 : (int64_t)3 << 20) ? TopkPath::kSort : TopkPath::kSelect;
+}
+
 struct TopkLayout {
   size_t state_off, part_off, psum_off, own_total;
   size_t cand_i_off, tcnt_off, tstat_off, tlist_off, sort_scratch_off, scratch;
+  size_t word_off, submax_off, gcomp_off, mstate_off;  // maxima path and rank words
   int groups;
   int64_t chunk;
+  TopkMaxima mx;
+  TopkPath path;
 };
 
 inline TopkLayout topk_layout(int64_t n, int64_t k, int dt) {
@@ -780,31 +1167,35 @@ inline TopkLayout topk_layout(int64_t n, int64_t k, int dt) {
   L.tstat_off = align256(L.tcnt_off + (size_t)(tiles + 1) * 8);
   L.tlist_off = align256(L.tstat_off + (size_t)tiles * 8);
   L.sort_scratch_off = align256(L.tlist_off + (size_t)tiles * kTkListMax);
-  L.scratch = L.sort_scratch_off + tcs_sort_scratch_bytes(k, dt);
+  const int kb = topk_elem_bytes(dt);
+  L.mx = topk_maxima(n, k, kb);
+  L.path = topk_path(L.mx, n, k, kb);
+  L.word_off = align256(L.sort_scratch_off +
+                        (L.path == TopkPath::kSort ? sort_first_scratch_bytes(n, dt) : tcs_sort_scratch_bytes(k, dt)));
+  L.submax_off = align256(L.word_off + (size_t)kTkCandMax * 8);
+  L.gcomp_off = align256(L.submax_off + (size_t)L.mx.subs * 4);
+  L.mstate_off = align256(L.gcomp_off + (size_t)L.mx.groups * 8);
+  L.scratch = L.mstate_off + 256;
   return L;
 }
 
-template <int DT>
-static int topk_run(const void* x, int64_t n, int64_t k, bool largest, void* out_v, int32_t* out_i, void* ws,
-                    size_t ws_bytes, void* scratch, size_t scratch_bytes, hipStream_t st) {
+// The k selected keys of the radix select, by rank words (WORDS) or as
+// values and positions; gated as its kernels are.
+template <int DT, bool WORDS>
+static int topk_select(const typename SortKey<DT>::Raw* xr, int64_t n, int64_t k, uint32_t flip, const TopkLayout& L,
+                       char* w, char* sc, uint32_t* gate, hipStream_t st) {
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
   constexpr int P = KT::kBits / 8;
-  const TopkLayout L = topk_layout(n, k, DT);
-  char* w = static_cast<char*>(ws);
   auto* state = reinterpret_cast<uint64_t*>(w + L.state_off);
   auto* partial = reinterpret_cast<uint64_t*>(w + L.part_off);
   auto* psum = reinterpret_cast<uint64_t*>(w + L.psum_off);
+  // Arrivals of the gated launches, zeroed with the gate by the maxima pass.
+  uint32_t* arrived = gate ? gate + 8 : nullptr;
   const int sum_per = (L.groups + kTkSumGroups - 1) / kTkSumGroups;
   const int sum_groups = (L.groups + sum_per - 1) / sum_per;
-  char* sc = static_cast<char*>(scratch);
-  auto* cand_v = reinterpret_cast<Raw*>(sc);
-  auto* cand_i = reinterpret_cast<int32_t*>(sc + L.cand_i_off);
-  const uint32_t flip = largest ? 0u : (KT::kBits == 32 ? 0xffffffffu : ((1u << KT::kBits) - 1u));
-  const Raw* xr = static_cast<const Raw*>(x);
   constexpr int64_t kTile = TopkGeom<DT>::kTile;
   static_assert(kTile == (int64_t)kTkNW * (sizeof(Raw) <= 2 ? 4 : 2) * kWave * kTkG, "topk_tile");
-  if (L.chunk % kTile != 0 || L.chunk / kTile > kTkMaxChunkTiles) return TCS_ERR_INVALID_ARG;
   const uint32_t tiles = (uint32_t)((n + kTile - 1) / kTile);
   auto* tcnt = reinterpret_cast<uint64_t*>(sc + L.tcnt_off);
   auto* tstat = reinterpret_cast<uint64_t*>(sc + L.tstat_off);
@@ -813,50 +1204,97 @@ static int topk_run(const void* x, int64_t n, int64_t k, bool largest, void* out
   for (int r = P - 1; r >= 0; --r) {
     if (kFuse && r == 0) {
       hipLaunchKernelGGL((topk_hist_kernel<DT, kFuse>), dim3(L.groups), dim3(kTkThreads), 0, st, xr, n, L.chunk,
-                         flip, r, state, partial, tstat, tlist);
+                         flip, r, k, state, partial, tstat, tlist, gate, arrived);
     } else {
       hipLaunchKernelGGL((topk_hist_kernel<DT, false>), dim3(L.groups), dim3(kTkThreads), 0, st, xr, n, L.chunk,
-                         flip, r, state, partial, nullptr, nullptr);
+                         flip, r, k, state, partial, nullptr, nullptr, gate, arrived);
     }
     TCS_CHECK_LAUNCH();
-    hipLaunchKernelGGL(topk_sum_kernel, dim3(sum_groups), dim3(256), 0, st, partial, L.groups, sum_per, psum);
-    TCS_CHECK_LAUNCH();
-    hipLaunchKernelGGL(topk_pick_kernel, dim3(1), dim3(kTkPickThreads), 0, st, psum, sum_groups, r,
-                       r == P - 1 ? 1 : 0, k, state);
-    TCS_CHECK_LAUNCH();
+    if (!gate) {
+      hipLaunchKernelGGL(topk_sum_kernel, dim3(sum_groups), dim3(256), 0, st, partial, L.groups, sum_per, psum);
+      TCS_CHECK_LAUNCH();
+      hipLaunchKernelGGL(topk_pick_kernel, dim3(1), dim3(kTkPickThreads), 0, st, psum, sum_groups, r,
+                         r == P - 1 ? 1 : 0, k, state);
+      TCS_CHECK_LAUNCH();
+    }
   }
   if constexpr (kFuse) {
     hipLaunchKernelGGL((topk_tilefix_kernel<DT>), dim3((tiles + 3) / 4), dim3(256), 0, st, xr, n, flip, state, tstat,
-                       tlist, tcnt, tiles);
+                       tlist, tcnt, tiles, gate, arrived);
   } else {
     hipLaunchKernelGGL((topk_tilecount_kernel<DT>), dim3(tiles), dim3(kTkNW * kWave), 0, st, xr, n, flip, state,
-                       tcnt);
+                       tcnt, gate, arrived);
   }
   TCS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(topk_tilescan_kernel, dim3(1), dim3(kTkScanThreads), 0, st, tcnt, tiles);
-  TCS_CHECK_LAUNCH();
-  const uint32_t resident = topk_place_grid<DT>();
+  if (!gate) {
+    hipLaunchKernelGGL(topk_tilescan_kernel, dim3(1), dim3(kTkScanThreads), 0, st, tcnt, tiles);
+    TCS_CHECK_LAUNCH();
+  }
+  const uint32_t resident = topk_place_grid<DT, WORDS>();
   const uint32_t wave_groups = (tiles + kTkPlaceThreads / kWave - 1) / (kTkPlaceThreads / kWave);  // a wave per tile
   const uint32_t place_grid = wave_groups < resident ? wave_groups : resident;
-  hipLaunchKernelGGL((topk_place_kernel<DT>), dim3(place_grid), dim3(kTkPlaceThreads), 0, st, xr, n, flip, state, k,
-                     tcnt, kFuse ? tstat : nullptr, cand_v, cand_i, tiles);
+  hipLaunchKernelGGL((topk_place_kernel<DT, WORDS>), dim3(place_grid), dim3(kTkPlaceThreads), 0, st, xr, n, flip,
+                     state, k, tcnt, kFuse ? tstat : nullptr, reinterpret_cast<Raw*>(sc),
+                     reinterpret_cast<int32_t*>(sc + L.cand_i_off), reinterpret_cast<uint64_t*>(sc + L.word_off),
+                     tiles, gate);
   TCS_CHECK_LAUNCH();
-  // Order the k selected: largest first (smallest first for !largest), ties
-  // in input order.  The radix sort reuses this workspace (same header and
-  // epoch).
-  if (k <= kTkSmallSort) {
-    if (k <= kTkSortThreads * 2) {
-      hipLaunchKernelGGL((topk_small_sort_kernel<DT, 2>), dim3(1), dim3(kTkSortThreads), 0, st, cand_v, cand_i,
-                         (int)k, flip, static_cast<Raw*>(out_v), out_i);
+  return TCS_OK;
+}
+
+template <int DT, int U>
+static void topk_maxima_launch(const typename SortKey<DT>::Raw* xr, int64_t n, int64_t k, uint32_t flip,
+                               const TopkLayout& L, char* sc, uint32_t* mstate, hipStream_t st) {
+  auto* submax = reinterpret_cast<uint32_t*>(sc + L.submax_off);
+  auto* gcomp = reinterpret_cast<uint64_t*>(sc + L.gcomp_off);
+  constexpr uint32_t W = kTkMaxThreads / kWave, W2 = kTkGatherThreads / kWave * kTkGatherSubs;
+  hipLaunchKernelGGL((topk_max_kernel<DT, U>), dim3((L.mx.groups + W - 1) / W), dim3(kTkMaxThreads), 0, st, xr, n,
+                     flip, L.mx.per, L.mx.subs, L.mx.groups, submax, gcomp, mstate);
+  hipLaunchKernelGGL(topk_bound_kernel, dim3(1), dim3(kTkBoundThreads), 0, st, gcomp, L.mx.groups, submax,
+                     L.mx.subs, (uint32_t)k, SortKey<DT>::kBits, mstate);
+  hipLaunchKernelGGL((topk_gather_kernel<DT, U>), dim3((L.mx.subs + W2 - 1) / W2),
+                     dim3(kTkGatherThreads), 0, st, xr, n, flip, L.mx.subs, submax, mstate,
+                     reinterpret_cast<uint64_t*>(sc + L.word_off));
+}
+
+template <int DT>
+static int topk_run(const void* x, int64_t n, int64_t k, bool largest, void* out_v, int32_t* out_i, void* ws,
+                    size_t ws_bytes, void* scratch, size_t scratch_bytes, hipStream_t st) {
+  using KT = SortKey<DT>;
+  using Raw = typename KT::Raw;
+  const TopkLayout L = topk_layout(n, k, DT);
+  char* w = static_cast<char*>(ws);
+  char* sc = static_cast<char*>(scratch);
+  if (L.path == TopkPath::kSort)
+    return sort_first(x, DT, out_v, out_i, n, k, largest, sc + L.sort_scratch_off, st);
+  const uint32_t flip = largest ? 0u : (KT::kBits == 32 ? 0xffffffffu : ((1u << KT::kBits) - 1u));
+  const Raw* xr = static_cast<const Raw*>(x);
+  constexpr int64_t kTile = TopkGeom<DT>::kTile;
+  if (L.chunk % kTile != 0 || L.chunk / kTile > kTkMaxChunkTiles) return TCS_ERR_INVALID_ARG;
+  if (k > kTkRankMax) {
+    const int rc = topk_select<DT, false>(xr, n, k, flip, L, w, sc, nullptr, st);
+    if (rc != TCS_OK) return rc;
+    // Largest first (smallest first for !largest), ties in input order.
+    return tcs_sort(sc, DT, reinterpret_cast<int32_t*>(sc + L.cand_i_off), out_v, out_i, k, largest ? 1 : 0, ws,
+                    ws_bytes, sc + L.sort_scratch_off, scratch_bytes - L.sort_scratch_off, st);
+  }
+  auto* mstate = reinterpret_cast<uint32_t*>(sc + L.mstate_off);
+  uint32_t* gate = nullptr;
+  if (L.path == TopkPath::kMaxima) {
+    if (L.mx.U == 1) {
+      topk_maxima_launch<DT, 1>(xr, n, k, flip, L, sc, mstate, st);
     } else {
-      hipLaunchKernelGGL((topk_small_sort_kernel<DT, 4>), dim3(1), dim3(kTkSortThreads), 0, st, cand_v, cand_i,
-                         (int)k, flip, static_cast<Raw*>(out_v), out_i);
+      topk_maxima_launch<DT, 4>(xr, n, k, flip, L, sc, mstate, st);
     }
     TCS_CHECK_LAUNCH();
-    return TCS_OK;
+    gate = mstate;
   }
-  return tcs_sort(cand_v, DT, cand_i, out_v, out_i, k, largest ? 1 : 0, ws, ws_bytes, sc + L.sort_scratch_off,
-                  scratch_bytes - L.sort_scratch_off, st);
+  const int rc = topk_select<DT, true>(xr, n, k, flip, L, w, sc, gate, st);
+  if (rc != TCS_OK) return rc;
+  hipLaunchKernelGGL((topk_rank_kernel<DT>), dim3(kTkRankBlocks), dim3(kTkRankThreads), 0, st,
+                     reinterpret_cast<const uint64_t*>(sc + L.word_off), gate, xr, (uint32_t)k,
+                     static_cast<Raw*>(out_v), out_i);
+  TCS_CHECK_LAUNCH();
+  return TCS_OK;
 }
 
 }  // namespace tcs

@@ -231,3 +231,50 @@ def test_topk_pivot_reference_bound(ops, dev, n):
     est = torch.sort(ops.run_topk_pivot_fp16(x, 8)).values[-1]
     kth = torch.sort(torch.topk(x, 2048, largest=True).values).values[0]
     assert kth > est, (float(kth), float(est))
+
+
+def _path_input(kind, n, dtype, dev):
+    g = torch.Generator(dev).manual_seed(n)
+    if dtype.is_floating_point:
+        x = torch.randn(n, generator=g, device=dev).to(dtype)
+    else:
+        i = torch.iinfo(dtype)
+        x = torch.randint(i.min, i.max + 1, (n,), generator=g, device=dev, dtype=torch.int64).to(dtype)
+    if kind == "sorted":  # the largest keys lie together: candidates overflow
+        x = torch.sort(x).values
+    elif kind == "ties":  # few values, each many times
+        x = x.remainder(5) if not dtype.is_floating_point else (x * 2).round()
+    elif kind == "constant":
+        x = torch.full_like(x, 3)
+    elif kind == "special" and dtype.is_floating_point:
+        v = torch.tensor([0.0, -0.0, float("inf"), float("-inf"), float("nan")], device=dev).to(dtype)
+        at = torch.randint(0, n, (2000,), generator=g, device=dev)
+        x[at] = v.repeat(400)
+    elif kind == "lump":  # 30000 equal largest keys in one place, 100 above them elsewhere
+        top = x.max() if dtype.is_floating_point else torch.iinfo(dtype).max - 1
+        x[n // 3:n // 3 + 30000] = top
+        x[:: n // 100] = top + 1 if not dtype.is_floating_point else float("inf")
+    return x
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["random", "sorted", "ties", "constant", "special", "lump"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.int16, torch.int8, torch.int32], ids=str)
+def test_topk_paths(ops, dev, kind, dtype):
+    """Sizes on both sides of the sort's limit (2^22 keys of 1 and 2 bytes,
+    2^19 of 4), with maxima of 1-vector and of 4-vector sub-chunks, enough
+    groups for the maxima path or not, and more winners than it takes, against
+    the stable sort's first k.  Sorted, constant and lumped inputs give more
+    candidates than fit, so the radix select runs behind the maxima."""
+    b = torch.empty(0, dtype=dtype).element_size()
+    sizes = ([1 << 22, (1 << 22) + 1, 9_000_001, 70_000_003] if b <= 2 else
+             [1 << 19, (1 << 19) + 1, 3_000_001, 34_000_003])
+    for n in sizes:
+        x = _path_input(kind, n, dtype, dev)
+        for largest in (True, False):
+            _, ei = torch.sort(x, descending=largest, stable=True)
+            for k in (1, 37, 2048, 4096, 4097):
+                v, i = ops.run_topk(x, k, largest)
+                assert torch.equal(i.long(), ei[:k]), (n, k, largest)
+                bits = {1: torch.int8, 2: torch.int16, 4: torch.int32}[b]
+                assert torch.equal(v.view(bits), x[ei[:k]].view(bits)), (n, k, largest)
