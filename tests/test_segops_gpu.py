@@ -435,3 +435,25 @@ def test_compress_ind_full_size_2p28(ops, dev):
     ev, ei = oracle.compress_ind(to_np(x), to_np(idx), to_np(mask))
     assert_exact(to_np(zv), ev)
     assert_exact(to_np(zi), ei)
+
+
+# --- int8 sums at the edges of their 16384-value tiles -----------------------
+@pytest.mark.parametrize("idx", [torch.int32, torch.int64], ids=str)
+@pytest.mark.parametrize("nnz", [1, 15, 16384, 16385, 5 * 16384 - 1, 5 * 16384 + 17])
+def test_seg_sum_int8_tile_edges(ops, dev, nnz, idx):
+    """Rows that end at, before and after tile edges, rows cut by one and by
+    several tiles, runs of empty rows on both sides of an edge, one row over
+    everything, one value per row, and values past the last row."""
+    rng = np.random.default_rng(nnz)
+    x = rng.integers(-128, 128, nnz).astype(np.int8)
+    edges = [t + d for t in range(0, nnz + 16385, 16384) for d in (-17, -16, -1, 0, 0, 0, 1, 15, 16, 17)]
+    cuts = sorted(min(max(c, 0), nnz) for c in edges)
+    some = np.sort(rng.integers(0, nnz + 1, 300))
+    layouts = [[0] + cuts + [nnz], [0, nnz], list(range(nnz + 1)), [0] * 5 + [nnz] * 5, [0] + list(some) + [nnz],
+               [0, nnz // 3, nnz // 2]]
+    xd = torch.from_numpy(x).to(dev)
+    for ip in layouts:
+        ip = np.asarray(ip, dtype=np.int64)
+        y = ops.run_seg_sum_multi_core(xd, torch.from_numpy(ip).to(idx).to(dev), 128)
+        pre = np.concatenate([[0], np.cumsum(x.astype(np.int64))])
+        assert_exact(to_np(y), (pre[ip[1:]] - pre[ip[:-1]]).astype(np.int32), f"rows {len(ip) - 1}")
