@@ -644,6 +644,127 @@ __global__ __launch_bounds__((NW + 1) * kWave) void scan_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// Short plain scans: one 4096-element tile per workgroup and no pipeline.
+// Every workgroup publishes its tile's aggregate and then reads those of all
+// tiles before it at once, one or two a thread, so a tile waits out one round
+// trip instead of a walk of six descriptors a step; no tile publishes an
+// inclusive descriptor.  Eight waves of data and one that fetches the launch
+// state meanwhile.  Bound by latency.  fp16 against the pipelined kernel: 2^16
+// elements 5.7 and 7.3 us, 2^20 6.9 and 10.4, 2^21 8.7 and 11.6, 3e6 10.2 and
+// 12.7, 2^22 13.6 and 13.8, 6e6 16.9 and 16.4 (reading every aggregate grows
+// with the square of the tiles).
+// ---------------------------------------------------------------------------
+constexpr int kShortNW = 8, kShortE = 8;
+constexpr int64_t kShortWave = (int64_t)kWave * kShortE, kShortTile = kShortWave * kShortNW;
+constexpr int kShortThreads = (kShortNW + 1) * kWave;
+constexpr int64_t kShortMax = (int64_t)3 << 20;
+
+// Inclusive scan over the wave of the lanes' sums of wave segment `seg` (512
+// elements from 512 * seg); `v` receives the lane's elements.
+template <class C>
+__device__ __forceinline__ typename C::Acc short_wave_scan(const typename C::In* __restrict__ x, int64_t n,
+                                                           int64_t seg, Packed<typename C::In, kShortE>& v) {
+  const int64_t b = seg * kShortWave + (int64_t)__lane_id() * kShortE;
+  if ((seg + 1) * kShortWave <= n) {
+    load_items<typename C::In, kShortE, true>(x, b, n, v);
+  } else {
+    load_items<typename C::In, kShortE, false>(x, b, n, v);
+  }
+  typename C::Acc s = typename C::Acc(0);
+#pragma unroll
+  for (int i = 0; i < kShortE; ++i) s = s + C::conv(v[i]);
+  return wave_incl_scan(s);
+}
+
+template <class C>
+__global__ __launch_bounds__(kShortThreads) void scan_short_kernel(const typename C::In* __restrict__ x,
+                                                                   typename C::Out* __restrict__ y,
+                                                                   typename C::Acc start, void* ws, int64_t n) {
+  using Acc = typename C::Acc;
+  constexpr int NW = kShortNW, E = kShortE;
+  __shared__ Acc s_wval[NW], s_before[NW + 1];
+  __shared__ LaunchTag s_tag;
+  const int lane = __lane_id(), wid = threadIdx.x / kWave;
+  const uint32_t tile = blockIdx.x;
+  Packed<typename C::In, E> v;
+  Acc incl = Acc(0);
+  if (wid == NW) {
+    if (lane == 0) s_tag = launch_arrive(ws);
+  } else {
+    incl = short_wave_scan<C>(x, n, (int64_t)tile * NW + wid, v);
+    if (lane == kWave - 1) s_wval[wid] = incl;
+  }
+  __syncthreads();
+  Acc wx = Acc(0), agg = Acc(0);
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    if (w == wid) wx = agg;
+    agg = agg + s_wval[w];
+  }
+  uint64_t* desc = ws_desc(ws);
+  if (threadIdx.x == 0) desc_publish<Acc>(desc, tile, agg, s_tag.tag, kFlagAgg);
+  // The aggregates of the tiles before this one.  A tile that has not
+  // published after the poll limit is summed here, in the same order.
+  Acc before = Acc(0);
+  for (uint32_t i0 = wid * kWave; i0 < tile; i0 += kShortThreads) {
+    const uint32_t i = i0 + lane;
+    Acc val = Acc(0);
+    int flag = 0;
+    bool ok = i >= tile || desc_try_read<Acc>(desc, i, s_tag.tag, val, flag);
+    for (int polls = 0;; ++polls) {
+      uint64_t missing = __ballot(!ok);
+      if (missing == 0) break;
+      if (polls >= s_tag.polls) {
+        while (missing != 0) {
+          const int l = __builtin_ctzll(missing);
+          missing &= missing - 1;
+          Acc a = Acc(0);
+          for (int w = 0; w < NW; ++w) {
+            Packed<typename C::In, E> u;
+            a = a + readlane(short_wave_scan<C>(x, n, (int64_t)(i0 + l) * NW + w, u), kWave - 1);
+          }
+          if (lane == l) val = a;
+        }
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      if (!ok) ok = desc_try_read<Acc>(desc, i, s_tag.tag, val, flag);
+    }
+    before = before + val;
+  }
+  before = wave_sum(before);
+  if (lane == 0) s_before[wid] = before;
+  __syncthreads();
+  if (wid == NW) return;
+  Acc run = start;
+#pragma unroll
+  for (int w = 0; w <= NW; ++w) run = run + s_before[w];
+  run = run + wx;
+  const Acc ev = dpp_mov<kWaveShr1>(incl);
+  run = run + (lane == 0 ? Acc(0) : ev);
+  typename C::Out o[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    run = run + C::conv(v[i]);
+    o[i] = C::out(run);
+  }
+  const int64_t b = (int64_t)tile * kShortTile + (int64_t)wid * kShortWave + (int64_t)lane * E;
+  if (((int64_t)tile * NW + wid + 1) * kShortWave <= n) {
+    store_items<typename C::Out, E, true>(y, b, n, o);
+  } else {
+    store_items<typename C::Out, E, false>(y, b, n, o);
+  }
+}
+
+template <class C>
+static int launch_scan_short(const void* x, void* y, int64_t n, typename C::Acc start, void* ws, hipStream_t st) {
+  hipLaunchKernelGGL((scan_short_kernel<C>), dim3((uint32_t)((n + kShortTile - 1) / kShortTile)), dim3(kShortThreads),
+                     0, st, static_cast<const typename C::In*>(x), static_cast<typename C::Out*>(y), start, ws, n);
+  TCS_CHECK_LAUNCH();
+  return TCS_OK;
+}
+
 // Resident workgroups of one scan_kernel instantiation on the current
 // device: the persistent grid size.
 template <class C, int NW, int J, int SEG, int LOC>
@@ -746,6 +867,7 @@ static int scan_dispatch(const void* x, int x_dtype, void* y, const int8_t* flag
   // N = 2^28 with the default tiles: DPP for every dtype (fp16 5.6 vs 3.7
   // TB/s on the matrix units; int8 5.1 vs 4.4).
   if (method == TCS_METHOD_AUTO) method = TCS_METHOD_DPP;
+  const bool dflt = tiles_per_wg <= 0 && method == TCS_METHOD_DPP && window == 0;
   // Default look-back window, measured the same way: 6 for DPP (fp16 265 us
   // at 6 vs 272 at 8, 284 at 16, 420 at 1; bf16 263 vs 270; int8 level from
   // 5 to 8), 32 for the matrix-unit scan.
@@ -758,6 +880,21 @@ static int scan_dispatch(const void* x, int x_dtype, void* y, const int8_t* flag
   if (!x || !y || (SEG == kSegFlags && !flags)) return TCS_ERR_INVALID_ARG;
   if (SEG == kSegFixed && seg_len <= 0) return TCS_ERR_INVALID_ARG;
   if (!aligned16(x) || !aligned16(y) || (flags && !aligned16(flags))) return TCS_ERR_INVALID_ARG;
+  // Short plain scans with no tile, method or window asked for, where the
+  // workspace holds their descriptors.
+  if constexpr (SEG == kSegNone) {
+    if (dflt && n <= kShortMax && ws && ws_bytes >= lookback_ws_bytes((uint64_t)((n + kShortTile - 1) / kShortTile))) {
+      hipStream_t st = static_cast<hipStream_t>(stream);
+      switch (x_dtype) {
+        case TCS_F16: return launch_scan_short<CodecF16>(x, y, n, (double)(float)start, ws, st);
+        case TCS_BF16: return launch_scan_short<CodecBF16>(x, y, n, (double)(float)start, ws, st);
+        case TCS_F32: return launch_scan_short<CodecF32>(x, y, n, (double)(float)start, ws, st);
+        case TCS_I8: return launch_scan_short<CodecI8>(x, y, n, (int)start, ws, st);
+        case TCS_I32: return launch_scan_short<CodecI32>(x, y, n, (int)start, ws, st);
+        default: return TCS_ERR_UNSUPPORTED_DTYPE;
+      }
+    }
+  }
   // Default tile (tiles_per_wg <= 0), measured best on MI355X: 64K elements
   // for plain int8 scans (5.41 vs 5.09 TB/s at 32K), 32K for other 16-bit
   // and 8-bit inputs, 16K for 32-bit inputs (the 64-group maximum of 4-wide
@@ -770,10 +907,11 @@ static int scan_dispatch(const void* x, int x_dtype, void* y, const int8_t* flag
                  : (method == TCS_METHOD_MFMA && x_dtype == TCS_BF16) ? 8192
                  : (x_dtype == TCS_F32 || x_dtype == TCS_I32) ? 16384
                  : i8_plain_dpp ? 65536 : 32768;
-  // Short inputs take smaller DPP tiles, so that more workgroups share
-  // them (fp16 back to back, look-back window 6: 2^18 8.4 us at 8K, 8.6 at
-  // 16K; 2^20 10.4 at 8K, 10.0 at 16K, 13.9 at 32K; 2^21 12.1 at 8K, 11.2 at
-  // 16K; at 2^22 16K and 32K tie).
+  // Shorter inputs (row and segmented scans, and plain ones past kShortMax)
+  // take smaller DPP tiles, so that more workgroups share them (fp16 back to
+  // back, look-back window 6: 2^18 8.4 us at 8K, 8.6 at 16K; 2^20 10.4 at 8K,
+  // 10.0 at 16K, 13.9 at 32K; 2^21 12.1 at 8K, 11.2 at 16K; at 2^22 16K and
+  // 32K tie).
   if (tiles_per_wg <= 0 && method == TCS_METHOD_DPP) {
     if (n <= ((int64_t)1 << 18) && tile > 8192) tile = 8192;
     else if (n <= ((int64_t)1 << 23) && tile > 16384) tile = 16384;

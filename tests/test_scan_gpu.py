@@ -227,3 +227,23 @@ def test_seg_scan_flags(ops, dev, n, density, dtype):
     for fn in (ops.run_seg_scan, ops.run_seg_scan_vec):
         y = fn(x.to(dev), f.to(dev), 32)
         assert_exact(to_np(y), oracle.seg_scan_flags(to_np(x), to_np(f)))
+
+
+# Short scans: 4096-element tiles of eight 512-element waves up to 3 * 2^20
+# elements; 576 threads read the aggregates of the tiles before theirs.
+@pytest.mark.parametrize("n", [7, 8, 9, 511, 512, 513, 4096, 64 * 4096 + 1, 575 * 4096, 576 * 4096 + 1, 577 * 4096 - 3,
+                               3 << 20, (3 << 20) + 1])
+@pytest.mark.parametrize("dtype", [torch.int8, torch.float16, torch.bfloat16, torch.float32], ids=str)
+def test_short_scan_edges(ops, dev, dtype, n):
+    x = (torch.randint(-4, 5, (n,), generator=gen(n), dtype=torch.int8) if dtype == torch.int8 else
+         (torch.randint(-64, 65, (n,), generator=gen(n)) / 16).to(dtype))
+    y = ops.run_scan_single_core(x.to(dev), 128, -2.0)
+    assert_exact(to_np(y), oracle.scan(to_np(x), -2.0), f"{dtype} n={n}")
+
+
+def test_short_scan_nonfinite(ops, dev):
+    x = torch.ones(20_000, dtype=torch.float16)
+    x[9000], x[15000] = float("inf"), float("-inf")
+    y = ops.run_scan_multi_core(x.to(dev), 128).cpu()
+    assert torch.equal(y[:9000], torch.arange(1, 9001, dtype=torch.float32))
+    assert bool((y[9000:15000] == float("inf")).all()) and bool(torch.isnan(y[15000:]).all())
