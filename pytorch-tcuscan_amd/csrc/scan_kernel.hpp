@@ -871,7 +871,17 @@ static int scan_dispatch(const void* x, int x_dtype, void* y, const int8_t* flag
   // Default look-back window, measured the same way: 6 for DPP (fp16 265 us
   // at 6 vs 272 at 8, 284 at 16, 420 at 1; bf16 263 vs 270; int8 level from
   // 5 to 8), 32 for the matrix-unit scan.
-  if (window == 0) window = method == TCS_METHOD_MFMA ? 32 : 6;
+  // Plain DPP scans of up to 2^26 elements look further back: their tiles are
+  // nearly all in flight at once, so a walk meets aggregates only, and a wide
+  // step saves round trips (fp16, 4e6 elements: 14.1 us at 6, 12.2 at 16, 11.2
+  // at 64; 3.3e7: 37.6, 36.2, 36.9; 6.7e7: 64.7 at 6, 63.9 at 16, 66.1 at 64;
+  // 1e8: 92.2 at 6, 92.7 at 16).
+  if (window == 0) {
+    window = method == TCS_METHOD_MFMA                        ? 32
+             : SEG != kSegNone || n > ((int64_t)1 << 26)      ? 6
+             : n <= ((int64_t)1 << 23)                        ? 64
+                                                              : 16;
+  }
   // An integer scan's start is an int32: reject what does not convert
   // (NaN, infinities, values outside the int32 range) rather than cast it.
   if ((x_dtype == TCS_I8 || x_dtype == TCS_I32) && !(start >= -2147483648.0 && start <= 2147483647.0))
@@ -912,9 +922,13 @@ static int scan_dispatch(const void* x, int x_dtype, void* y, const int8_t* flag
   // back, look-back window 6: 2^18 8.4 us at 8K, 8.6 at 16K; 2^20 10.4 at 8K,
   // 10.0 at 16K, 13.9 at 32K; 2^21 12.1 at 8K, 11.2 at 16K; at 2^22 16K and
   // 32K tie).
+  // Plain int8: 16K up to 6 * 2^20 (6e6: 12.9 us, 13.1 at 32K; 8e6: 14.4 and
+  // 13.2), 32K up to 2^26 (3.4e7, whose 513 tiles of 64K leave one over: 31.8
+  // us, 33.1 at 64K; 6.7e7: 55.3 either way).
   if (tiles_per_wg <= 0 && method == TCS_METHOD_DPP) {
     if (n <= ((int64_t)1 << 18) && tile > 8192) tile = 8192;
-    else if (n <= ((int64_t)1 << 23) && tile > 16384) tile = 16384;
+    else if (n <= (i8_plain_dpp ? (int64_t)6 << 20 : (int64_t)1 << 23) && tile > 16384) tile = 16384;
+    else if (n <= ((int64_t)1 << 26) && tile > 32768) tile = 32768;
   }
   // Lane group width: 4 for 32-bit inputs, 8 for 16-bit and int8, 16 for
   // int8 on the matrix-unit scan (one group per 1024-element unit).
