@@ -455,10 +455,12 @@ int tcs_searchsorted(const int32_t* sorted, int64_t sorted_len, const int32_t* v
  * (at most 4 MiB + 4 bytes). */
 size_t tcs_searchsorted_workspace_bytes(int64_t sorted_len);
 
-/* Workspace bytes with which it is fastest: 512 counts and a table of
- * 2^b + 1 int32, b = clamp(floor(log2(len)) - 2, 10, 22) (at most 16 MiB +
- * 2052 bytes).  Any size from the least up is taken. */
-size_t tcs_searchsorted_preferred_bytes(int64_t sorted_len);
+/* Workspace bytes with which it is fastest for num_values needles: 512 counts
+ * and a table of 2^b + 1 int32, b = clamp(floor(log2(len)) - 2, 10, 22) (at
+ * most 16 MiB + 2052 bytes); at most 43 MiB where the needles are many
+ * (below).  Any size
+ * from the least up is taken. */
+size_t tcs_searchsorted_preferred_bytes(int64_t sorted_len, int64_t num_values);
 
 /* tcs_searchsorted with a bucket index built in `workspace` first (no host
  * synchronisation): the haystack's order keys between its first and last
@@ -467,8 +469,10 @@ size_t tcs_searchsorted_preferred_bytes(int64_t sorted_len);
  * (4 to 8 elements when the keys spread over their range and the workspace
  * is the preferred one; clustered keys fall back to the sampled search of
  * tcs_searchsorted, and a haystack of at most 16384 elements is searched
- * whole in LDS).  Results identical
- * to tcs_searchsorted.  `workspace` is scratch that this call overwrites
+ * whole in LDS).  Many needles (above 2^19 to 3 * 2^20, the more the shorter
+ * the haystack) are instead grouped by slices of the haystack, in batches
+ * that the workspace holds, with `out` as scratch.  Results identical to
+ * tcs_searchsorted.  `workspace` is scratch that this call overwrites
  * from its first byte (any contents before, nothing kept after): it must
  * not be a look-back workspace that other calls use, unless that is zeroed
  * again (tcs_workspace_reset) before its next look-back use.  Replaces

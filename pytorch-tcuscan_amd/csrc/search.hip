@@ -3,34 +3,59 @@
 // reference's run_searchsorted (src/torch/torch_searchsorted.h:33-82,
 // tests/test_searchsorted.py).
 //
-// Each workgroup first stages every B-th haystack element in LDS
-// (B = ceil(len / kSamples), so at most kSamples of them; the whole
-// haystack when it fits).  A needle's lower bound c among the samples
-// brackets its answer: sorted[(c-1)B] < key <= sorted[cB], so the answer
-// lies in [(c-1)B + 1, min(cB, len)] (0 when c = 0), and a binary search
-// over that window of fewer than B elements in global memory finishes it.
-// The LDS stage replaces the upper levels of the search, whose probes all
-// needles share; the lower levels are random probes into the haystack and
-// bound the kernel.
+// Four ways, by size: sixteen lanes a needle (few needles); a search tree of
+// samples in LDS (short haystacks, or no workspace); a table of buckets over
+// the key range; and, for many needles, needles grouped by slices of the
+// haystack that are searched in LDS.
 #include "tcs_common.hpp"
 
 namespace tcs {
 
 constexpr int kSsThreads = 1024;
-constexpr int kSsSamples = 16384;  // 64 KiB of LDS per workgroup
+constexpr int kSsLog = 14, kSsNodes = 1 << kSsLog;  // 64 KiB of LDS per workgroup
+constexpr int kSsU = 4;                             // needles of a thread in flight
 
-// The samples of `sorted` in LDS: every B-th element, at most kSsSamples.
-struct SsSamples {
-  int32_t B, ns;
-};
+// A search tree of 2^log - 1 nodes over the sorted samples p[0], p[step],
+// ..., p[(ns - 1) * step] in breadth-first order (children of node k: 2k and
+// 2k + 1): the first steps of a wave's lanes fall on distinct banks, where
+// the halving of a sorted array puts them on one.  Nodes past the samples
+// hold INT32_MAX, which no key exceeds.  A workgroup of kSsThreads.
+__device__ __forceinline__ void stage_tree(int32_t* tree, int log, const int32_t* __restrict__ p, int64_t step,
+                                           int32_t ns) {
+  constexpr int R = 8;  // loads in flight
+  const int32_t nodes = 1 << log;
+  for (int32_t r0 = threadIdx.x; r0 < nodes; r0 += R * kSsThreads) {
+    int32_t v[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int32_t r = r0 + i * kSsThreads - 1;
+      v[i] = ns > 0 ? p[(r < 0 ? 0 : (r < ns ? r : ns - 1)) * step] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int32_t r = r0 + i * kSsThreads;  // rank of the sample, from 1
+      if (r > 0 && r < nodes) {
+        const int z = __builtin_ctz(r);
+        tree[(nodes >> (z + 1)) + (r >> (z + 1))] = r <= ns ? v[i] : 0x7fffffff;
+      }
+    }
+  }
+}
 
-__device__ __forceinline__ SsSamples stage_samples(int32_t* s_samp, const int32_t* __restrict__ sorted,
-                                                   int32_t len) {
-  const int32_t B = (int32_t)(((int64_t)len + kSsSamples - 1) / kSsSamples);
-  const int32_t ns = len > 0 ? (int32_t)(((int64_t)len + B - 1) / B) : 0;  // <= kSsSamples
-  for (int i = threadIdx.x; i < ns; i += kSsThreads) s_samp[i] = sorted[(int64_t)i * B];
-  __syncthreads();
-  return SsSamples{B, ns};
+// c[u] = number of samples of the tree below key[u].  Three vector
+// instructions a step: the node's byte offset, not its number, is carried.
+template <int U>
+__device__ __forceinline__ void tree_count(const int32_t* tree, int log, const int32_t (&key)[U], int32_t (&c)[U]) {
+  const char* t = reinterpret_cast<const char*>(tree);
+#pragma unroll
+  for (int u = 0; u < U; ++u) c[u] = 4;
+  for (int s = 0; s < log; ++s) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      c[u] = (c[u] << 1) + (*reinterpret_cast<const int32_t*>(t + c[u]) < key[u] ? 4 : 0);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) c[u] = (c[u] >> 2) - (1 << log);
 }
 
 // Lower bound of key in sorted[lo, lo + count] (the answer is known to lie
@@ -46,32 +71,51 @@ __device__ __forceinline__ int32_t lower_bound_in(const int32_t* __restrict__ so
   return lo;
 }
 
-// Lower bound of key in sorted[0, len): the samples bracket it, then a
-// search over the window of fewer than B elements between two samples.
-__device__ __forceinline__ int32_t lower_bound_staged(const int32_t* s_samp, SsSamples sm,
-                                                      const int32_t* __restrict__ sorted, int32_t len,
-                                                      int32_t key) {
-  // Invariant of both searches: the answer lies in [lo, lo + count].
-  int32_t lo = 0, count = sm.ns;
-  while (count > 0) {
-    const int32_t half = count >> 1;
-    const bool right = s_samp[lo + half] < key;
-    lo = right ? lo + half + 1 : lo;
-    count = right ? count - half - 1 : half;
+// All needles by samples: every B-th element, B the least that leaves the
+// tree room for them, then the window of fewer than B elements between two
+// samples.  2^24 needles into 2^14 elements: 40.7 us (4.1e11 needles a
+// second; bound by the steps' LDS reads), 187 with one needle a thread at a
+// time and a sorted array of samples.
+__device__ __forceinline__ void search_staged(int32_t* s_tree, const int32_t* __restrict__ sorted, int32_t len,
+                                              const int32_t* __restrict__ values, int32_t* __restrict__ out,
+                                              int64_t nv) {
+  if (len == 0) {
+    for (int64_t i = (int64_t)blockIdx.x * kSsThreads + threadIdx.x; i < nv; i += (int64_t)gridDim.x * kSsThreads)
+      out[i] = 0;
+    return;
   }
-  const int64_t hi = (int64_t)lo * sm.B < len ? (int64_t)lo * sm.B : len;
-  const int32_t glo = lo == 0 ? 0 : (lo - 1) * sm.B + 1;
-  return lower_bound_in(sorted, glo, lo == 0 ? 0 : (int32_t)hi - glo, key);
+  const int32_t B = (int32_t)(((int64_t)len + kSsNodes - 1) / kSsNodes);
+  const int32_t ns = (int32_t)(((int64_t)len + B - 1) / B);  // at most kSsNodes: the first apart, the rest in the tree
+  const int log = ns > 1 ? 32 - __builtin_clz(ns - 1) : 0;
+  stage_tree(s_tree, log, sorted + B, B, ns - 1);
+  const int32_t first = sorted[0];
+  __syncthreads();
+  const int64_t stride = (int64_t)gridDim.x * kSsThreads;
+  for (int64_t i = (int64_t)blockIdx.x * kSsThreads + threadIdx.x; i < nv; i += kSsU * stride) {
+    int32_t key[kSsU], c[kSsU];
+#pragma unroll
+    for (int u = 0; u < kSsU; ++u) key[u] = values[i + u * stride < nv ? i + u * stride : nv - 1];
+    tree_count<kSsU>(s_tree, log, key, c);
+#pragma unroll
+    for (int u = 0; u < kSsU; ++u) {
+      c[u] += first < key[u] ? 1 : 0;
+      int32_t lo = c[u];
+      if (B > 1 && lo > 0) {
+        // sorted[(c - 1) B] < key <= sorted[c B].
+        const int64_t hi = (int64_t)c[u] * B < len ? (int64_t)c[u] * B : len;
+        lo = (c[u] - 1) * B + 1;
+        lo = lower_bound_in(sorted, lo, (int32_t)hi - lo, key[u]);
+      }
+      if (i + u * stride < nv) out[i + u * stride] = lo;
+    }
+  }
 }
 
 __global__ __launch_bounds__(kSsThreads) void searchsorted_kernel(const int32_t* __restrict__ sorted, int32_t len,
                                                                   const int32_t* __restrict__ values,
                                                                   int32_t* __restrict__ out, int64_t nv) {
-  __shared__ int32_t s_samp[kSsSamples];
-  const SsSamples sm = stage_samples(s_samp, sorted, len);
-  const int64_t stride = (int64_t)gridDim.x * kSsThreads;
-  for (int64_t i = (int64_t)blockIdx.x * kSsThreads + threadIdx.x; i < nv; i += stride)
-    out[i] = lower_bound_staged(s_samp, sm, sorted, len, values[i]);
+  __shared__ int32_t s_tree[kSsNodes];
+  search_staged(s_tree, sorted, len, values, out, nv);
 }
 
 // ---------------------------------------------------------------------------
@@ -292,22 +336,20 @@ __device__ __forceinline__ bool bucket_clustered(const int32_t* __restrict__ wid
   return m.shift > 0 && *s_sum > len / 16;
 }
 
-// Needles in input order, four per thread in flight.
-constexpr int kSsU = 4;
+// Needles in input order, kSsU per thread in flight.
 __global__ __launch_bounds__(kSsThreads) void searchsorted_indexed_kernel(const int32_t* __restrict__ sorted,
                                                                           int32_t len, int bits,
                                                                           const int32_t* __restrict__ wide,
                                                                           const int32_t* __restrict__ start,
                                                                           const int32_t* __restrict__ values,
                                                                           int32_t* __restrict__ out, int64_t nv) {
-  __shared__ int32_t s_samp[kSsSamples];
+  __shared__ int32_t s_tree[kSsNodes];
   const BucketMap m = bucket_map(sorted, len, bits);
   const int64_t stride = (int64_t)gridDim.x * kSsThreads;
   const int64_t first = (int64_t)blockIdx.x * kSsThreads + threadIdx.x;
-  if (bucket_clustered(wide, len, m, s_samp)) {
-    __syncthreads();  // s_samp is rewritten
-    const SsSamples sm = stage_samples(s_samp, sorted, len);
-    for (int64_t i = first; i < nv; i += stride) out[i] = lower_bound_staged(s_samp, sm, sorted, len, values[i]);
+  if (bucket_clustered(wide, len, m, s_tree)) {
+    __syncthreads();  // the sum has been read
+    search_staged(s_tree, sorted, len, values, out, nv);
     return;
   }
   for (int64_t i = first; i < nv; i += stride * kSsU) {
@@ -321,122 +363,357 @@ __global__ __launch_bounds__(kSsThreads) void searchsorted_indexed_kernel(const 
   }
 }
 
-// Haystacks beyond an XCD's L2: a workgroup takes 8192 needles at a time and
-// searches them grouped by the top eight bits of their place in the key
-// range, lowest group first, so that all workgroups sweep the haystack and
-// the table in the same direction and a line fetched into an L2 serves the
-// needles of every workgroup of that XCD.  2^24 needles into 2^24 keys: 520
-// us, in input order 650 (each needle fetches two lines past the L2s).
-constexpr int kSgThreads = 512, kSgRows = 16, kSgTile = kSgThreads * kSgRows;
-__global__ __launch_bounds__(kSgThreads) void searchsorted_grouped_kernel(const int32_t* __restrict__ sorted,
-                                                                          int32_t len, int bits,
-                                                                          const int32_t* __restrict__ wide,
-                                                                          const int32_t* __restrict__ start,
-                                                                          const int32_t* __restrict__ values,
-                                                                          int32_t* __restrict__ out, int64_t nv) {
-  static_assert(kSgThreads >= kSsBuildBlocks && kSgTile <= 65536, "one count word per thread; 16-bit positions");
-  __shared__ int32_t s_key[kSgTile];
-  __shared__ uint16_t s_at[kSgTile];
-  __shared__ uint32_t s_cnt[256];
-  __shared__ uint32_t s_wsum[4];
-  const int tid = threadIdx.x, lane = __lane_id(), wid = tid / kWave;
-  const BucketMap m = bucket_map(sorted, len, bits);
-  if (bucket_clustered(wide, len, m, reinterpret_cast<int*>(s_cnt))) {
-    __syncthreads();
-    const int32_t B = (int32_t)(((int64_t)len + kSgTile - 1) / kSgTile);
-    const int32_t ns = (int32_t)(((int64_t)len + B - 1) / B);
-    for (int i = tid; i < ns; i += kSgThreads) s_key[i] = sorted[(int64_t)i * B];
-    __syncthreads();
-    for (int64_t i = (int64_t)blockIdx.x * kSgThreads + tid; i < nv; i += (int64_t)gridDim.x * kSgThreads)
-      out[i] = lower_bound_staged(s_key, SsSamples{B, ns}, sorted, len, values[i]);
-    return;
+// ---------------------------------------------------------------------------
+// Large haystacks with many needles: the needles go to the haystack.  The
+// haystack is cut into slices of 16384 samples (every B-th element; B = 1 up
+// to 2^24 elements), at most 1024 of them, whose samples fit in LDS as a
+// search tree.  Four kernels over batches of at most 1024 tiles of 16384
+// needles:
+//   split:   a tile's needles, grouped by slice, into its part of `out`, with
+//            every needle's place in the tile (16 bits) and the start of
+//            every slice's group;
+//   columns: a workgroup per slice scans its groups' sizes over the tiles;
+//   sweep:   a workgroup per slice, or per share of the needles of one that
+//            many need, searches them in LDS and writes the answers in their
+//            place;
+//   unsplit: a tile's answers back to the needles' order.
+// All memory is read and written in runs of a group (64 bytes for 2^24
+// elements) or longer, where a search per needle reads a line of the haystack
+// and one of a table for each.  Slices hold equal numbers of elements and
+// shares equal numbers of needles, whatever the keys.  2^24 needles into 2^24
+// elements: 161 us (split 51, columns 12, sweep 83, unsplit 27 alone; a table
+// searched by groups of 8192 needles 551).  Split and unsplit run at 3.1 and 5.9
+// TB/s; the sweep is bound by its vector instructions (112 a row of 64
+// needles, 70% busy) and by the tree's LDS reads (50% busy).
+// ---------------------------------------------------------------------------
+constexpr int kSwThreads = kSsThreads, kSwRows = 16, kSwTile = kSwThreads * kSwRows;
+constexpr int kSwSlices = 1024, kSwSamples = kSsNodes;
+constexpr int kSwShare = 20480;  // most needles of a share
+
+// Inclusive maximum scan over a wave's lanes of values >= 0.
+__device__ __forceinline__ int32_t wave_incl_max(int32_t v) {
+  v = max(v, dpp_mov<kRowShr1>(v));
+  v = max(v, dpp_mov<kRowShr2>(v));
+  v = max(v, dpp_mov<kRowShr4>(v));
+  v = max(v, dpp_mov<kRowShr8>(v));
+  v = max(v, dpp_mov<kRowBcast15, 0xa>(v));
+  return max(v, dpp_mov<kRowBcast31, 0xc>(v));
+}
+
+// Exclusive scan of one value per thread over a workgroup of kSwThreads, and
+// the total; s_w holds a word per wave.  Ends with a barrier.
+__device__ __forceinline__ int32_t sw_block_scan(int32_t v, int32_t* s_w, int32_t* total) {
+  constexpr int W = kSwThreads / kWave;
+  const int lane = __lane_id(), wid = threadIdx.x / kWave;
+  const int32_t incl = wave_incl_scan(v);
+  if (lane == kWave - 1) s_w[wid] = incl;
+  __syncthreads();
+  int32_t before = incl - v, all = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    before += w < wid ? s_w[w] : 0;
+    all += s_w[w];
   }
-  const uint32_t range = m.umax - m.umin;
-  const int width = range == 0 ? 0 : 32 - __builtin_clz(range);
-  const int gshift = width > 8 ? width - 8 : 0;
-  for (int64_t t0 = (int64_t)blockIdx.x * kSgTile; t0 < nv; t0 += (int64_t)gridDim.x * kSgTile) {
-    const int tvalid = t0 + kSgTile <= nv ? kSgTile : (int)(nv - t0);
-    __syncthreads();  // the previous tile's counts and results have been read
-    if (tid < 256) s_cnt[tid] = 0;
-    int32_t key[kSgRows];
-    uint32_t gr[kSgRows];  // group << 16 | rank in it (in no particular order)
+  *total = all;
+  __syncthreads();
+  return before;
+}
+
+__global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8))) void searchsorted_split_kernel(
+    const int32_t* __restrict__ sorted, int64_t slice, int nb, int log, const int32_t* values, int32_t* out,
+    int64_t nv, uint16_t* __restrict__ pos, uint16_t* __restrict__ start) {
+  __shared__ int32_t s_key[kSwTile];
+  __shared__ int32_t s_tree[kSwSlices];
+  __shared__ int32_t s_cnt[kSwSlices + 1];
+  __shared__ int32_t s_w[kSwThreads / kWave];
+  const int tid = threadIdx.x;
+  stage_tree(s_tree, log, sorted + slice, slice, nb - 1);
+  const int64_t t0 = (int64_t)blockIdx.x * kSwTile;
+  const int tvalid = t0 + kSwTile <= nv ? kSwTile : (int)(nv - t0);
+  values += t0;
+  out += t0;
+  pos += t0;
+  s_cnt[tid] = 0;
+  if (tid == 0) s_cnt[kSwSlices] = 0;
+  int32_t key[kSwRows], br[kSwRows];  // slice << 16 | rank in it (in no particular order)
 #pragma unroll
-    for (int i = 0; i < kSgRows; ++i) {
-      const int p = i * kSgThreads + tid;
-      key[i] = values[t0 + (p < tvalid ? p : tvalid - 1)];
-    }
-    __syncthreads();
+  for (int i = 0; i < kSwRows; ++i) {
+    const int p = i * kSwThreads + tid;
+    key[i] = values[p < tvalid ? p : tvalid - 1];
+  }
+  int again = tid;  // places are found anew in each phase, not kept in registers
+  asm volatile("" : "+v"(again));
+  __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kSgRows; ++i) {
-      const uint32_t o = order_key(key[i]);
-      const uint32_t g = o <= m.umin ? 0u : (o >= m.umax ? range >> gshift : (o - m.umin) >> gshift);
-      gr[i] = g << 16;
-      if (i * kSgThreads + tid < tvalid) gr[i] |= atomicAdd(&s_cnt[g], 1u);
-    }
-    __syncthreads();
-    uint32_t cnt = 0, incl = 0;
-    if (tid < 256) {
-      cnt = s_cnt[tid];
-      incl = wave_incl_scan(cnt);
-      if (lane == kWave - 1) s_wsum[wid] = incl;
-    }
-    __syncthreads();
-    if (tid < 256) {
-      uint32_t before = incl - cnt;
-      for (int w = 0; w < wid; ++w) before += s_wsum[w];
-      s_cnt[tid] = before;
-    }
-    __syncthreads();
+  for (int i = 0; i < kSwRows; i += 4) {
+    const int32_t k4[4] = {key[i], key[i + 1], key[i + 2], key[i + 3]};
+    int32_t c4[4];
+    tree_count<4>(s_tree, log, k4, c4);
 #pragma unroll
-    for (int i = 0; i < kSgRows; ++i) {
-      const int p = i * kSgThreads + tid;
-      if (p < tvalid) {
-        const uint32_t q = s_cnt[gr[i] >> 16] + (gr[i] & 0xffffu);
-        s_key[q] = key[i];
-        s_at[q] = (uint16_t)p;
+    for (int u = 0; u < 4; ++u) {
+      // Rows past the end count in a word of their own.
+      const int32_t b = (i + u) * kSwThreads + again < tvalid ? c4[u] : kSwSlices;
+      br[i + u] = b << 16 | atomicAdd(&s_cnt[b], 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __syncthreads();
+  int32_t all;
+  const int32_t first = sw_block_scan(s_cnt[tid], s_w, &all);
+  s_cnt[tid] = first;
+  if (tid == 0) s_cnt[kSwSlices] = tvalid;
+  if (tid < nb) start[(int64_t)blockIdx.x * nb + tid] = (uint16_t)first;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kSwRows; ++i) {
+    br[i] = s_cnt[br[i] >> 16] + (br[i] & 0xffff);
+    s_key[br[i]] = key[i];
+    if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+  }
+  __syncthreads();
+  asm volatile("" : "+v"(again));
+#pragma unroll
+  for (int i = 0; i < kSwRows; ++i) {
+    const int p = i * kSwThreads + again;
+    if (p < tvalid) {
+      pos[p] = (uint16_t)br[i];
+      out[p] = s_key[p];
+    }
+    if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// groups[slice][tile] = {needles of the slice in earlier tiles, place of the
+// group in `out` less that}; total[slice].
+__global__ __launch_bounds__(kSwThreads) void searchsorted_columns_kernel(const uint16_t* __restrict__ start, int nb,
+                                                                          int nt, int64_t nv,
+                                                                          i32x2u* __restrict__ groups,
+                                                                          int32_t* __restrict__ total) {
+  __shared__ int32_t s_w[kSwThreads / kWave];
+  const int t = threadIdx.x, b = blockIdx.x;
+  int32_t s = 0, e = 0;
+  if (t < nt) {
+    const int64_t left = nv - (int64_t)t * kSwTile;
+    s = start[(int64_t)t * nb + b];
+    e = b + 1 < nb ? start[(int64_t)t * nb + b + 1] : (left < kSwTile ? (int)left : kSwTile);
+  }
+  int32_t all;
+  const int32_t before = sw_block_scan(e - s, s_w, &all);
+  if (t < nt) groups[(int64_t)b * nt + t] = i32x2u{before, t * kSwTile + s - before};
+  if (t == 0) total[b] = all;
+}
+
+__global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8))) void searchsorted_sweep_kernel(
+    const int32_t* __restrict__ sorted, int32_t len, int32_t B, int nb, int nt, const i32x2u* __restrict__ groups,
+    const int32_t* __restrict__ total, int32_t* __restrict__ out) {
+  constexpr int W = kSwThreads / kWave, U = 4;
+  __shared__ int32_t s_tree[kSwSamples];
+  __shared__ int32_t s_before[kSwThreads + 1];  // needles of the slice in earlier tiles
+  __shared__ int32_t s_at[kSwThreads];      // place of the tile's group less that
+  __shared__ uint8_t s_own[W][U * kWave] __attribute__((aligned(4)));
+  __shared__ int32_t s_w[W];
+  __shared__ int32_t s_first[W];
+  __shared__ int32_t s_slice, s_share, s_shares;
+  const int tid = threadIdx.x, lane = __lane_id(), wid = tid / kWave;
+  if (tid == 0) s_shares = 0;
+  const int32_t tot = tid < nb ? total[tid] : 0;
+  const int32_t shares = (tot + kSwShare - 1) / kSwShare;
+  int32_t all;
+  const int32_t before = sw_block_scan(shares, s_w, &all);
+  const int32_t me = (int32_t)blockIdx.x - before;
+  if (me >= 0 && me < shares) {
+    s_slice = tid;
+    s_share = me;
+    s_shares = shares;
+    s_w[0] = tot;
+  }
+  __syncthreads();
+  if (s_shares == 0) return;
+  const int b = s_slice;
+  const int32_t btot = s_w[0];
+  const int32_t j0 = (int32_t)((int64_t)btot * s_share / s_shares);
+  const int32_t j1 = (int32_t)((int64_t)btot * (s_share + 1) / s_shares);
+  const int32_t per = ((j1 - j0 + W - 1) / W + kWave - 1) / kWave * kWave;  // needles of a wave
+  // The slice's samples: 0 apart (only slice 0 has needles that do not exceed
+  // it), the rest in the tree.
+  const int64_t e0 = (int64_t)b * kSwSamples * B;
+  const int64_t rest = (len - e0 + B - 1) / B;
+  stage_tree(s_tree, kSsLog, sorted + e0 + B, B, (int32_t)(rest < kSwSamples ? rest : kSwSamples) - 1);
+  const int32_t first = sorted[e0];
+  // This thread's tile holds the slice's needles [p0, p1).
+  int32_t p0 = btot, p1 = btot;
+  if (tid < nt) {
+    const i32x2u g = groups[(int64_t)b * nt + tid];
+    p0 = g[0];
+    s_at[tid] = g[1];
+    if (tid + 1 < nt) p1 = groups[(int64_t)b * nt + tid + 1][0];
+  }
+  s_before[tid] = p0;
+  if (tid == 0) s_before[kSwThreads] = btot;
+  if (p0 < p1) {
+    // The tile of each wave's first needle.
+    int32_t w = p0 > j0 ? (p0 - j0 + per - 1) / per : 0;
+    for (; w < W && j0 + w * per < p1; ++w) s_first[w] = tid;
+  }
+  __syncthreads();
+  const int32_t w0 = j0 + wid * per;
+  const int32_t w1 = w0 + per < j1 ? w0 + per : j1;
+  if (w0 >= w1) return;
+  // Places of the wave's next rows of needles, from `r0` on: up to U rows, and
+  // no further than the 64 tiles from `cur` reach (one a lane).  Each tile
+  // marks its first needle; the nearest mark at or before a needle names its
+  // tile, tile `cur` where there is none.
+  int32_t cur = __builtin_amdgcn_readfirstlane(s_first[wid]), r0 = w0;
+  uint8_t* own = s_own[wid];
+  auto place = [&](int32_t (&at)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) at[u] = -1;
+    while (r0 < w1) {
+      const int32_t t = cur + lane;
+      const int32_t q0 = s_before[t < nt ? t : nt], q1 = s_before[t + 1 < nt ? t + 1 : nt];
+      const int32_t reach = readlane(q1, kWave - 1);
+      int32_t r1 = w1 < r0 + U * kWave ? w1 : r0 + U * kWave;
+      r1 = reach < r1 ? reach : r1;
+      if (r1 <= r0) {  // tiles without needles
+        cur += kWave;
+        continue;
       }
-    }
-    __syncthreads();
-    int32_t r[kSgRows];
+      reinterpret_cast<uint32_t*>(own)[lane] = 0;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (q0 >= r0 && q0 < r1 && q0 < q1) own[q0 - r0] = (uint8_t)lane;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      int32_t m[U];
 #pragma unroll
-    for (int i = 0; i < kSgRows; i += kSsU) {
-      int32_t k4[kSsU], r4[kSsU];
+      for (int u = 0; u < U; ++u) m[u] = own[u * kWave + lane];
+      int32_t carry = 0;
 #pragma unroll
-      for (int u = 0; u < kSsU; ++u) {
-        const int q = (i + u) * kSgThreads + tid;
-        k4[u] = s_key[q < tvalid ? q : tvalid - 1];
+      for (int u = 0; u < U; ++u) {
+        m[u] = max(wave_incl_max(m[u]), carry);
+        carry = readlane(m[u], kWave - 1);
+        const int32_t j = r0 + u * kWave + lane;
+        const int32_t a = s_at[cur + m[u]] + j;
+        at[u] = j < r1 ? a : -1;
       }
-      bucket_search<kSsU>(sorted, len, m, start, k4, r4);
-#pragma unroll
-      for (int u = 0; u < kSsU; ++u) r[i + u] = r4[u];
+      cur += __builtin_popcountll(__ballot(q1 <= r1));
+      r0 = r1;
+      break;
     }
-    __syncthreads();
+  };
+  int32_t at[U], key[U];
+  place(at);
 #pragma unroll
-    for (int i = 0; i < kSgRows; ++i) {
-      const int q = i * kSgThreads + tid;
-      if (q < tvalid) s_key[s_at[q]] = r[i];
+  for (int u = 0; u < U; ++u) key[u] = out[at[u] >= 0 ? at[u] : 0];
+  for (bool more = true; more;) {
+    // The next rows are on their way during the search.
+    int32_t nat[U], nkey[U], c[U];
+    more = r0 < w1;
+    if (more) {
+      place(nat);
+#pragma unroll
+      for (int u = 0; u < U; ++u) nkey[u] = out[nat[u] >= 0 ? nat[u] : 0];
     }
-    __syncthreads();
+    tree_count<U>(s_tree, kSsLog, key, c);
 #pragma unroll
-    for (int i = 0; i < kSgRows; ++i) {
-      const int p = i * kSgThreads + tid;
-      if (p < tvalid) out[t0 + p] = s_key[p];
+    for (int u = 0; u < U; ++u) {
+      c[u] += first < key[u] ? 1 : 0;  // samples below the needle
+      // Elements below it: B = 1, no more than the samples (c is 0 in slice 0
+      // only); otherwise between samples c - 1 and c.
+      int32_t lo = (int32_t)e0 + c[u];
+      if (B > 1 && c[u] > 0) {
+        const int64_t l = e0 + (int64_t)(c[u] - 1) * B + 1;
+        const int64_t hi = l + B - 1 < len ? l + B - 1 : len;
+        lo = lower_bound_in(sorted, (int32_t)l, (int32_t)(hi - l), key[u]);
+      }
+      if (at[u] >= 0) out[at[u]] = lo;
+      if (more) {
+        at[u] = nat[u];
+        key[u] = nkey[u];
+      }
     }
   }
 }
 
-// The grouped kernel from these sizes on: below, the grouping costs more than
-// the lines it saves (2^20 elements, 2^24 needles: 238 us against 205; 2^22
-// elements, 2^24 needles: 338 against 502; 2^24 elements, 2^20 needles: 87
-// against 65).
-constexpr int64_t kSgMinLen = (int64_t)1 << 20, kSgMinNeedles = (int64_t)3 << 19;
+__global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8))) void searchsorted_unsplit_kernel(
+    const uint16_t* __restrict__ pos, int32_t* __restrict__ out, int64_t nv) {
+  __shared__ int32_t s_r[kSwTile];
+  const int tid = threadIdx.x;
+  const int64_t t0 = (int64_t)blockIdx.x * kSwTile;
+  const int tvalid = t0 + kSwTile <= nv ? kSwTile : (int)(nv - t0);
+  int32_t r[kSwRows];
+  uint32_t q[kSwRows];
+#pragma unroll
+  for (int i = 0; i < kSwRows; ++i) {
+    const int p = i * kSwThreads + tid;
+    r[i] = out[t0 + (p < tvalid ? p : tvalid - 1)];
+    q[i] = pos[t0 + (p < tvalid ? p : tvalid - 1)];
+  }
+#pragma unroll
+  for (int i = 0; i < kSwRows; ++i) {
+    const int p = i * kSwThreads + tid;
+    if (p < tvalid) s_r[p] = r[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kSwRows; ++i) {
+    const int p = i * kSwThreads + tid;
+    if (p < tvalid) out[t0 + p] = s_r[q[i]];
+  }
+}
+
+// The sweep from these sizes on; below, its four launches and the slices read
+// by workgroups with few needles cost more than a table does (us, table and
+// sweep; 2^18 elements: 2^22 needles 46 and 47, 2^23 83 and 69; 2^20 elements:
+// 2^21 needles 35 and 44, 2^22 60 and 48; 2^21: 2^20 32 and 34, 2^21 52 and
+// 44; 2^22 and above: 2^19 27 and 27, 2^20 41 and 33).
+constexpr int64_t kSwMinLen = (int64_t)1 << 16;
+static int64_t sweep_min_needles(int64_t len) {
+  if (len <= (int64_t)1 << 20) return (int64_t)3 << 20;
+  return len <= (int64_t)1 << 21 ? (int64_t)1 << 20 : (int64_t)1 << 19;
+}
+
+// Slices, elements between samples, and the scratch of a batch of nt tiles:
+// groups, slice totals, group starts, places.
+struct SweepLayout {
+  int32_t B;
+  int nb, log;
+  size_t total, start, pos, end;
+};
+
+static SweepLayout sweep_layout(int64_t len, int64_t nt) {
+  SweepLayout l;
+  l.B = (int32_t)((len + (int64_t)kSwSamples * kSwSlices - 1) / ((int64_t)kSwSamples * kSwSlices));
+  const int64_t slice = (int64_t)kSwSamples * l.B;
+  l.nb = (int)((len + slice - 1) / slice);
+  l.log = 0;
+  while ((1 << l.log) < l.nb) ++l.log;
+  l.total = (size_t)l.nb * nt * sizeof(i32x2u);
+  l.start = l.total + (size_t)l.nb * sizeof(int32_t);
+  l.pos = l.start + ((size_t)l.nb * nt * sizeof(uint16_t) + 15) / 16 * 16;
+  l.end = l.pos + (size_t)nt * kSwTile * sizeof(uint16_t);
+  return l;
+}
+
+// Tiles of a batch in `bytes` of scratch; 0 where the sweep does not pay:
+// each batch reads the haystack, so it wants 256 tiles (or all there are).
+static int64_t sweep_tiles(int64_t len, int64_t nv, size_t bytes) {
+  if (len <= kSwMinLen || nv <= sweep_min_needles(len)) return 0;
+  const int64_t all = (nv + kSwTile - 1) / kSwTile;
+  int64_t nt = all < kSwThreads ? all : kSwThreads;
+  const int64_t least = nt < 256 ? nt : 256;
+  const SweepLayout one = sweep_layout(len, 1), two = sweep_layout(len, 2);
+  const size_t per_tile = two.end - one.end + 16;
+  if (sweep_layout(len, nt).end > bytes) nt = bytes > one.end ? (int64_t)((bytes - one.end) / per_tile) : 0;
+  return nt >= least ? nt : 0;
+}
 
 // Whether the needles are too few to pay for staging samples in every
-// workgroup, or for a table (2^14 needles into 2^20 elements: 5.3 us against
-// 14.7 sampled; 2^15 into 2^24: 16 us, with a table 28).
+// workgroup, or for a table (us, sixteen lanes and the other way; 2^16
+// needles into 2^16 elements: 7.4 and 9.1 sampled, 2^17 needles 12.2 and 9.2;
+// 2^16 into 2^20 11.4 and 11.2 with a table, into 2^22 18.9 and 16.1, into
+// 2^24 28.1 and 31, 2^15 into 2^22 10.8 and 15).
 static bool searchsorted_few(int64_t len, int64_t nv) {
-  if (len <= kSsSamples) return nv <= (int64_t)1 << 13;
-  return nv <= (len > ((int64_t)1 << 22) ? (int64_t)1 << 16 : (int64_t)1 << 15);
+  const bool mid = len > ((int64_t)1 << 18) && len <= ((int64_t)1 << 22);
+  return nv <= (mid ? (int64_t)1 << 15 : (int64_t)1 << 16);
 }
 
 // Four workgroups per CU of the current device (two are resident at a
@@ -467,9 +744,13 @@ int tcs_searchsorted(const int32_t* sorted, int64_t sorted_len, const int32_t* v
     TCS_CHECK_LAUNCH();
     return TCS_OK;
   }
-  const uint64_t need = (uint64_t)((num_values + kSsThreads - 1) / kSsThreads);
+  // A workgroup for each CU first, then kSsU needles a thread before more of
+  // them stage the samples (2^20 needles into 2^14: 16.4 us with one needle a
+  // thread, 7.4 with four).
   const uint64_t cap = searchsorted_grid();
-  const uint32_t blocks = (uint32_t)(need < cap ? need : cap);
+  const uint64_t rows = (uint64_t)((num_values + kSsThreads - 1) / kSsThreads);
+  const uint64_t few = rows < cap / 4 ? rows : cap / 4, need = (rows + kSsU - 1) / kSsU;
+  const uint32_t blocks = (uint32_t)(need < few ? few : (need < cap ? need : cap));
   hipLaunchKernelGGL(searchsorted_kernel, dim3(blocks), dim3(kSsThreads), 0, static_cast<hipStream_t>(stream),
                      sorted, (int32_t)sorted_len, values, out, num_values);
   TCS_CHECK_LAUNCH();
@@ -494,9 +775,41 @@ size_t tcs_searchsorted_workspace_bytes(int64_t sorted_len) {
 
 static int bucket_bits(int64_t len) { return clamp_int(floor_log2(len) - 2, 10, 22); }
 
-size_t tcs_searchsorted_preferred_bytes(int64_t sorted_len) {
+size_t tcs_searchsorted_preferred_bytes(int64_t sorted_len, int64_t num_values) {
+  using namespace tcs;
   if (sorted_len <= 0) return 0;
-  return (tcs::kSsBuildBlocks + ((size_t)1 << bucket_bits(sorted_len)) + 1) * sizeof(int32_t);
+  const int64_t nt = sweep_tiles(sorted_len, num_values, SIZE_MAX);
+  const size_t least = tcs_searchsorted_workspace_bytes(sorted_len);
+  if (nt > 0) {
+    const size_t sweep = sweep_layout(sorted_len, nt).end;
+    return sweep > least ? sweep : least;
+  }
+  return (kSsBuildBlocks + ((size_t)1 << bucket_bits(sorted_len)) + 1) * sizeof(int32_t);
+}
+
+static int sweep_batch(const int32_t* sorted, int64_t len, const int32_t* values, int32_t* out, int64_t nv,
+                       void* workspace, hipStream_t st) {
+  using namespace tcs;
+  const int64_t nt = (nv + kSwTile - 1) / kSwTile;
+  const SweepLayout l = sweep_layout(len, nt);
+  char* w = static_cast<char*>(workspace);
+  auto* groups = reinterpret_cast<i32x2u*>(w);
+  auto* total = reinterpret_cast<int32_t*>(w + l.total);
+  auto* start = reinterpret_cast<uint16_t*>(w + l.start);
+  auto* pos = reinterpret_cast<uint16_t*>(w + l.pos);
+  hipLaunchKernelGGL(searchsorted_split_kernel, dim3((uint32_t)nt), dim3(kSwThreads), 0, st, sorted,
+                     (int64_t)kSwSamples * l.B, l.nb, l.log, values, out, nv, pos, start);
+  TCS_CHECK_LAUNCH();
+  hipLaunchKernelGGL(searchsorted_columns_kernel, dim3(l.nb), dim3(kSwThreads), 0, st, start, l.nb, (int)nt, nv, groups,
+                     total);
+  TCS_CHECK_LAUNCH();
+  // At most one share more than full ones for each slice.
+  hipLaunchKernelGGL(searchsorted_sweep_kernel, dim3((uint32_t)(l.nb + nv / kSwShare)), dim3(kSwThreads), 0, st, sorted,
+                     (int32_t)len, l.B, l.nb, (int)nt, groups, total, out);
+  TCS_CHECK_LAUNCH();
+  hipLaunchKernelGGL(searchsorted_unsplit_kernel, dim3((uint32_t)nt), dim3(kSwThreads), 0, st, pos, out, nv);
+  TCS_CHECK_LAUNCH();
+  return TCS_OK;
 }
 
 int tcs_searchsorted_indexed(const int32_t* sorted, int64_t sorted_len, const int32_t* values, int32_t* out,
@@ -508,9 +821,17 @@ int tcs_searchsorted_indexed(const int32_t* sorted, int64_t sorted_len, const in
   if (sorted_len == 0) return tcs_searchsorted(sorted, sorted_len, values, out, num_values, stream);
   if (!workspace || workspace_bytes < tcs_searchsorted_workspace_bytes(sorted_len)) return TCS_ERR_WORKSPACE;
   // A haystack that fits in LDS needs no table.
-  if (sorted_len <= kSsSamples || searchsorted_few(sorted_len, num_values))
+  if (sorted_len <= kSsNodes || searchsorted_few(sorted_len, num_values))
     return tcs_searchsorted(sorted, sorted_len, values, out, num_values, stream);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t nt = sweep_tiles(sorted_len, num_values, workspace_bytes);
+  if (nt > 0) {
+    for (int64_t i = 0; i < num_values; i += nt * kSwTile) {
+      const int64_t n = num_values - i < nt * kSwTile ? num_values - i : nt * kSwTile;
+      if (const int rc = sweep_batch(sorted, sorted_len, values + i, out + i, n, workspace, st)) return rc;
+    }
+    return TCS_OK;
+  }
   const int64_t entries = (int64_t)(workspace_bytes / sizeof(int32_t)) - kSsBuildBlocks - 1;
   const int bits = clamp_int(bucket_bits(sorted_len), 1, floor_log2(entries));
   auto* wide = static_cast<int32_t*>(workspace);
@@ -521,16 +842,9 @@ int tcs_searchsorted_indexed(const int32_t* sorted, int64_t sorted_len, const in
                      wide, start);
   TCS_CHECK_LAUNCH();
   const uint64_t cap = searchsorted_grid();
-  if (sorted_len > kSgMinLen && num_values > kSgMinNeedles) {
-    const uint64_t tiles = (uint64_t)((num_values + kSgTile - 1) / kSgTile);
-    const uint64_t resident = cap / 4 * 3;  // three workgroups of 49 KiB of LDS on each CU
-    hipLaunchKernelGGL(searchsorted_grouped_kernel, dim3((uint32_t)(tiles < resident ? tiles : resident)),
-                       dim3(kSgThreads), 0, st, sorted, len, bits, wide, start, values, out, num_values);
-  } else {
-    const uint64_t need = (uint64_t)((num_values + kSsThreads - 1) / kSsThreads);
-    hipLaunchKernelGGL(searchsorted_indexed_kernel, dim3((uint32_t)(need < cap ? need : cap)), dim3(kSsThreads), 0, st,
-                       sorted, len, bits, wide, start, values, out, num_values);
-  }
+  const uint64_t need = (uint64_t)((num_values + kSsThreads - 1) / kSsThreads);
+  hipLaunchKernelGGL(searchsorted_indexed_kernel, dim3((uint32_t)(need < cap ? need : cap)), dim3(kSsThreads), 0, st,
+                     sorted, len, bits, wide, start, values, out, num_values);
   TCS_CHECK_LAUNCH();
   return TCS_OK;
 }

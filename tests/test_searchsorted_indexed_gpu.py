@@ -144,20 +144,20 @@ def test_op_leaves_the_stream_workspace_intact(ops, dev):
 @pytest.mark.parametrize("kind", ["uniform", "narrow", "constant", "clusters", "heavy_tail"])
 @pytest.mark.parametrize("n", [16385, 65537, (1 << 20) + 3, (1 << 22) + 5])
 def test_preferred_table(lib, dev, kind, n):
-    """The preferred table: needles in input order, and grouped (above 2^20
-    elements and 1.5 * 2^20 needles), a ragged last tile of needles included;
-    nothing written past the outputs and the workspace."""
+    """The preferred workspace: a table, and needles grouped by slices (from
+    2^22 elements and 2^19 needles), a ragged last tile included; nothing
+    written past the outputs and the workspace."""
     lib.tcs_searchsorted_preferred_bytes.restype = ctypes.c_size_t
-    lib.tcs_searchsorted_preferred_bytes.argtypes = [ctypes.c_int64]
+    lib.tcs_searchsorted_preferred_bytes.argtypes = [ctypes.c_int64, ctypes.c_int64]
     rng = np.random.default_rng(n + len(kind))
     hay = _haystack(kind, n, rng)
     h = torch.from_numpy(hay).to(dev)
-    wsb = lib.tcs_searchsorted_preferred_bytes(n)
-    assert wsb >= lib.tcs_searchsorted_workspace_bytes(n)
-    ws = torch.full((wsb // 4 + 8,), -1, dtype=torch.int32, device=dev)
     s = torch.cuda.current_stream().cuda_stream
     for m in (70_000, 1_600_001):
         needles = _needles(rng, hay, m)
+        wsb = lib.tcs_searchsorted_preferred_bytes(n, len(needles))
+        assert wsb >= lib.tcs_searchsorted_workspace_bytes(n)
+        ws = torch.full((wsb // 4 + 8,), -1, dtype=torch.int32, device=dev)
         v = torch.from_numpy(needles).to(dev)
         out = torch.full((len(needles) + 8,), -7, dtype=torch.int32, device=dev)
         assert lib.tcs_searchsorted_indexed(h.data_ptr(), n, v.data_ptr(), out.data_ptr(), len(needles), ws.data_ptr(),
@@ -188,3 +188,65 @@ def test_few_needles(ops, dev, n):
         needles = _needles(rng, hay, m)
         got = ops.run_searchsorted(torch.from_numpy(hay).to(dev), torch.from_numpy(needles).to(dev)).cpu().numpy()
         assert np.array_equal(got, np.searchsorted(hay, needles, side="left").astype(np.int32))
+
+
+@pytest.mark.parametrize("n,m", [((1 << 16) + 1, (3 << 20) + 1), ((1 << 21) - 16383, (1 << 20) + 16385),
+                                 ((1 << 24) + 1, (1 << 19) + 1), ((1 << 25) + 16386, 700_001),
+                                 ((1 << 16) + 16384, (1 << 24) + 5)])
+@pytest.mark.parametrize("needles", ["uniform", "one", "sorted", "few_values"])
+def test_grouped_by_slices(ops, dev, n, m, needles):
+    """Slices at their edges (one element in the last, samples of every second
+    or third element, more needles than one batch) with needles spread over
+    the slices, all in one, in order, and in a few: equal to torch's search
+    and to the general one."""
+    g = torch.Generator(device=dev).manual_seed(n + m)
+
+    def keys(k):
+        return torch.randint(I32_MIN, I32_MAX, (k,), generator=g, device=dev, dtype=torch.int32)
+
+    hay = keys(n).sort().values
+    hay[: n // 64] = I32_MIN  # runs of equal keys at both ends
+    hay[n - n // 64:] = I32_MAX
+    if needles == "one":
+        v = hay[n // 2].expand(m).contiguous()
+    elif needles == "few_values":
+        v = torch.tensor([I32_MIN, I32_MAX, 0, 12345], dtype=torch.int32, device=dev)[
+            torch.randint(0, 4, (m,), generator=g, device=dev)]
+    else:
+        v = keys(m)
+        v[: m // 3] = hay[torch.randint(0, n, (m // 3,), generator=g, device=dev)]
+        v = v.sort().values if needles == "sorted" else v[torch.randperm(m, generator=g, device=dev)]
+    got = ops.run_searchsorted(hay, v)
+    assert torch.equal(got, torch.searchsorted(hay, v, out_int32=True))
+
+
+@pytest.mark.parametrize("tiles", [5, 97, 300])
+def test_slices_in_less_workspace(lib, dev, tiles):
+    """Batches of as many tiles as the workspace holds, and the table where
+    that is too few: the same results."""
+    lib.tcs_searchsorted_preferred_bytes.restype = ctypes.c_size_t
+    lib.tcs_searchsorted_preferred_bytes.argtypes = [ctypes.c_int64, ctypes.c_int64]
+    n, m = (1 << 22) + 77, 16384 * 301 + 9
+    rng = np.random.default_rng(tiles)
+    h = torch.from_numpy(_haystack("uniform", n, rng)).to(dev)
+    v = torch.from_numpy(rng.integers(I32_MIN, I32_MAX, m, dtype=np.int64, endpoint=True).astype(np.int32)).to(dev)
+    full = lib.tcs_searchsorted_preferred_bytes(n, m)
+    wsb = max(full * tiles // 302, lib.tcs_searchsorted_workspace_bytes(n))
+    ws = torch.full((wsb // 4 + 8,), -1, dtype=torch.int32, device=dev)
+    out = torch.full((m + 8,), -7, dtype=torch.int32, device=dev)
+    assert lib.tcs_searchsorted_indexed(h.data_ptr(), n, v.data_ptr(), out.data_ptr(), m, ws.data_ptr(), wsb // 4 * 4,
+                                        torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out[:m], torch.searchsorted(h, v, out_int32=True))
+    assert bool((out[m:] == -7).all()) and bool((ws[wsb // 4:] == -1).all())
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 1023, 1024, 16384, 16385, 32768, 32769, 65536])
+def test_sample_tree(lib, dev, n):
+    """The tree of samples around powers of two and whole and thinned
+    haystacks."""
+    rng = np.random.default_rng(n)
+    for kind in ("uniform", "narrow", "clusters"):
+        hay = _haystack(kind, n, rng)
+        needles = _needles(rng, hay, 280_001)
+        exp = np.searchsorted(hay, needles, side="left").astype(np.int32)
+        assert np.array_equal(_search(lib, dev, hay, needles, indexed=False), exp)
