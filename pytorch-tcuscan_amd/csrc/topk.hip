@@ -14,11 +14,12 @@
 // maximum reaches it are read again, and their keys at or above it, about
 // 1.15 k of them when the keys are in no particular order, are ranked by
 // counting.  If they do not fit (the largest keys lie together), the radix
-// select below runs instead: its kernels are launched behind this path and
-// leave at once when it has succeeded, so nothing waits for the host.  2^28
-// fp16 normals, k = 2048: 134 us, of which the read takes 94, the select's two
-// reads and eleven launches 278; sorted keys, which give too many candidates,
-// 600 against 429.
+// select below runs instead, over the sub-chunks that reach the bound: its
+// kernels are launched behind this path and leave at once when it has
+// succeeded, so nothing waits for the host.  2^28 fp16 normals, k = 2048: 125
+// us, of which the read takes 86, the select's two reads and eleven launches
+// 278; sorted keys, which give too many candidates, 378 against 429 (2^25 of
+// them 138 against 115).
 //
 // Otherwise radix select: the k-th largest order key T is found one 8-bit
 // digit at a time, from the top: a histogram of digit r over the keys whose
@@ -176,7 +177,8 @@ __global__ __launch_bounds__(kTkThreads) void topk_hist_kernel(const typename So
                                                                uint64_t* __restrict__ tstat,
                                                                uint8_t* __restrict__ tlist,
                                                                const uint32_t* __restrict__ gate,
-                                                               uint32_t* __restrict__ arrived) {
+                                                               uint32_t* __restrict__ arrived,
+                                                               const uint32_t* __restrict__ submax, int sub_shift) {
   if (topk_done(gate)) return;
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
@@ -253,7 +255,29 @@ __global__ __launch_bounds__(kTkThreads) void topk_hist_kernel(const typename So
   };
   int64_t b0 = c0 + (int64_t)tid * V;
   const int64_t full_end = c0 + ((c1 - c0) / (U * STEP)) * (U * STEP);  // steps [c0, full_end) are whole
+  // Behind a gate a wave leaves out the steps whose sub-chunks all lie below
+  // the bound: no key there is selected, and the digits chosen count only
+  // keys at or above the k-th.  2^28 sorted fp16 keys (few sub-chunks hold
+  // them all): 615 us without, 378 with it and with groups
+  // of sub-chunks that lie apart.
+  const uint32_t bound = gate ? gate[1] : 0u;
+  const int64_t wave0 = (int64_t)__builtin_amdgcn_readfirstlane(wid) * (kWave * V);
+  auto below = [&](int64_t step0) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t q = submax[(step0 + u * STEP + wave0) >> sub_shift];
+      m = m > q ? m : q;
+    }
+    return m < bound;
+  };
+  int64_t step0 = c0;
+  bool next_below = gate && c0 < full_end && below(c0);
   for (; b0 < full_end; b0 += U * STEP) {
+    const bool skip = next_below;
+    step0 += U * STEP;
+    if (gate && step0 < full_end) next_below = below(step0);
+    if (skip) continue;
     Raw v[U][V];
 #pragma unroll
     for (int u = 0; u < U; ++u) load_items<Raw, V, true>(x, b0 + u * STEP, c1, v[u]);
@@ -713,8 +737,9 @@ __global__ __launch_bounds__(256) void topk_pivot_kernel(const uint16_t* __restr
 
 // ---------------------------------------------------------------------------
 // Maxima path.  A sub-chunk is U vectors of 64 lanes of 16 bytes; wave g of
-// the grid takes the `per` sub-chunks from g * per (per <= 64): submax[s] =
-// the sub-chunk's largest order key, gcomp[g] = the group's largest << 32 |
+// the grid takes sub-chunks g, g + groups, ... (at most 64; far apart, so that
+// large keys that lie together fall into many groups): submax[s] = the
+// sub-chunk's largest order key, gcomp[g] = the group's largest << 32 |
 // ~(its first sub-chunk that holds it).  Reads at the streaming rate: seven
 // packed instructions map two 16-bit keys and one takes their maximum (2^28
 // fp16 keys 94 us, 5.7 TB/s; with plain loads 106).
@@ -741,7 +766,7 @@ struct TopkSub {
 
 template <int DT, int U>
 __global__ __launch_bounds__(kTkMaxThreads) void topk_max_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
-                                                                 int64_t n, uint32_t flip, int per, uint32_t subs,
+                                                                 int64_t n, uint32_t flip, uint32_t subs,
                                                                  uint32_t groups, uint32_t* __restrict__ submax,
                                                                  uint64_t* __restrict__ gcomp,
                                                                  uint32_t* __restrict__ state) {
@@ -754,10 +779,9 @@ __global__ __launch_bounds__(kTkMaxThreads) void topk_max_kernel(const typename 
   if (blockIdx.x == 0 && threadIdx.x == 0) state[0] = state[8] = 0;
   const uint32_t g = blockIdx.x * (kTkMaxThreads / kWave) + threadIdx.x / kWave;
   if (g >= groups) return;
-  const uint32_t s0 = g * (uint32_t)per;
-  const uint32_t s1 = s0 + per < subs ? s0 + per : subs;
-  uint32_t mine = 0, best = 0, at = s0;
-  for (uint32_t s = s0; s < s1; ++s) {
+  uint32_t mine = 0, best = 0, at = g;
+  int j = 0;
+  for (uint32_t s = g; s < subs; s += groups, ++j) {
     const int64_t b = (int64_t)s * SUB + lane * V;
     uint32_t m = 0;
     if ((int64_t)(s + 1) * SUB <= n) {
@@ -800,32 +824,37 @@ __global__ __launch_bounds__(kTkMaxThreads) void topk_max_kernel(const typename 
       }
     }
     m = wave_max(m);
-    if (lane == (int)(s - s0)) mine = m;
+    if (lane == j) mine = m;
     if (m > best) {
       best = m;
       at = s;
     }
   }
-  if (s0 + lane < s1) submax[s0 + lane] = mine;
+  if (lane < j) submax[g + lane * groups] = mine;
   if (lane == 0) gcomp[g] = ((uint64_t)best << 32) | (uint32_t)~at;
 }
 
-// state[1] = T, state[2] = P: the k-th largest of the groups' (maximum,
-// lowest sub-chunk first) is (T, sub-chunk P).  One workgroup, the maxima in
-// LDS; T two bits at a time from the top (the counts of maxima at or above
-// three trials by ballots: a histogram's atomics would meet in the few bins
-// the maxima fall into).  Short loops on purpose: code
-// unrolled over registers took as long to fetch as to run.
+// state[1] = T, state[2] = P: at least k keys are above T, or equal to T in a
+// sub-chunk up to P.  T is the k-th largest of the groups' maxima, P by
+// default the last of the sub-chunks that hold the maxima of the first groups
+// at T.  One workgroup, the maxima in LDS; T two bits at a time from the top
+// (the counts of maxima at or above three trials by ballots: a histogram's
+// atomics would meet in the few bins the maxima fall into).  Short loops on
+// purpose: code unrolled over registers took as long to fetch as to run.
 constexpr int kTkBoundThreads = 1024;
 constexpr uint32_t kTkMaxGroupsM = 16384;
-__global__ __launch_bounds__(kTkBoundThreads) void topk_bound_kernel(const uint64_t* __restrict__ gcomp,
+template <int DT, int U>
+__global__ __launch_bounds__(kTkBoundThreads) void topk_bound_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
+                                                                     int64_t n, uint32_t flip,
+                                                                     const uint64_t* __restrict__ gcomp,
                                                                      uint32_t groups,
                                                                      const uint32_t* __restrict__ submax,
-                                                                     uint32_t subs, uint32_t k, int bits,
+                                                                     uint32_t subs, uint32_t k,
                                                                      uint32_t* __restrict__ state) {
+  constexpr int bits = SortKey<DT>::kBits;
   __shared__ uint32_t s_key[kTkMaxGroupsM];
   __shared__ uint32_t s_row[kTkMaxGroupsM / kWave];
-  __shared__ uint32_t s_cnt[16][3], s_above, s_at[2];
+  __shared__ uint32_t s_cnt[16][3], s_above, s_last, s_p;
   const int tid = threadIdx.x, lane = __lane_id(), wid = tid / kWave;
   for (uint32_t g0 = tid; g0 < groups; g0 += 8 * kTkBoundThreads) {  // eight loads in flight
     uint64_t c[8];
@@ -836,7 +865,7 @@ __global__ __launch_bounds__(kTkBoundThreads) void topk_bound_kernel(const uint6
       if (g0 + u * kTkBoundThreads < groups) s_key[g0 + u * kTkBoundThreads] = (uint32_t)(c[u] >> 32);
   }
   if (tid < 48) (&s_cnt[0][0])[tid] = 0;
-  if (tid == 0) s_above = 0;
+  if (tid == 0) s_above = s_p = 0;
   __syncthreads();
   uint32_t T = 0;
 #pragma unroll 1
@@ -887,69 +916,121 @@ __global__ __launch_bounds__(kTkBoundThreads) void topk_bound_kernel(const uint6
     return l;
   };
   if (need <= k / 4) {
-    // The row, and in it the group: the need-th at T in order.
-    if (wid != 0) return;
-    const int rows = (int)((groups + kWave - 1) / kWave);
-    int row = 0;
+    // The row, and in it the group: the need-th at T in order; P covers the
+    // groups at T up to it.
+    if (wid == 0) {
+      const int rows = (int)((groups + kWave - 1) / kWave);
+      int row = 0;
 #pragma unroll 1
-    for (int r0 = 0; r0 < rows; r0 += kWave) {
-      const int l = find(r0 + lane < rows ? s_row[r0 + lane] : 0u);
-      if (l < kWave) {
-        row = r0 + l;
-        break;
+      for (int r0 = 0; r0 < rows; r0 += kWave) {
+        const int l = find(r0 + lane < rows ? s_row[r0 + lane] : 0u);
+        if (l < kWave) {
+          row = r0 + l;
+          break;
+        }
       }
+      const uint32_t g = (uint32_t)row * kWave + lane;
+      const int l = find(g < groups && s_key[g] == T ? 1u : 0u);
+      if (lane == l) s_last = g;
     }
-    const uint32_t g = (uint32_t)row * kWave + lane;
-    const int l = find(g < groups && s_key[g] == T ? 1u : 0u);
-    if (lane == l) {
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t g = tid; g <= s_last; g += kTkBoundThreads)
+      if (s_key[g] == T) atomicMax(&s_p, ~(uint32_t)gcomp[g]);
+    __syncthreads();
+    if (tid == 0) {
       state[1] = T;
-      state[2] = ~(uint32_t)gcomp[g];
+      state[2] = s_p;
     }
     return;
   }
-  // Many groups at T (a value that repeats): the need-th sub-chunk at T is as
-  // good a bound as the need-th group, and as much lower as a group holds
-  // sub-chunks at T.
-  constexpr int V = 16;
+  // Many groups at T (a value that repeats).  The sub-chunks at T in order,
+  // the first `need` of them, replace the maxima in LDS ...
+  constexpr int V = 16, W = kTkBoundThreads / kWave;
+  uint32_t have = 0;
 #pragma unroll 1
-  for (uint32_t b = 0; b < subs; b += kTkBoundThreads * V) {
+  for (uint32_t b = 0; b < subs && have < need; b += kTkBoundThreads * V) {
     // Wave w takes 64 V sub-chunks from b + 64 V w, row by row.
-    uint32_t m[V];
+    uint32_t m[V], cnt = 0;
     const uint32_t wb = b + (uint32_t)wid * kWave * V + lane;
 #pragma unroll
     for (int u = 0; u < V; ++u) m[u] = submax[wb + u * kWave < subs ? wb + u * kWave : 0];
-    __syncthreads();  // s_row was read
+#pragma unroll
+    for (int u = 0; u < V; ++u) cnt += (uint32_t)__popcll(__ballot(wb + u * kWave < subs && m[u] == T));
+    __syncthreads();  // s_key and s_row were read
+    if (lane == 0) s_row[wid] = cnt;
+    __syncthreads();
+    uint32_t at = have;
+    for (int w = 0; w < W; ++w) {
+      at += w < wid ? s_row[w] : 0;
+      have += s_row[w];
+    }
 #pragma unroll
     for (int u = 0; u < V; ++u) {
-      const uint32_t e = (uint32_t)__popcll(__ballot(wb + u * kWave < subs && m[u] == T));
-      if (lane == 0) s_row[wid * V + u] = e;
+      const bool in = wb + u * kWave < subs && m[u] == T;
+      const uint64_t set = __ballot(in);
+      const uint32_t q = at + (uint32_t)__popcll(set & ~(~0ull << lane));
+      if (in && q < need) s_key[q] = wb + u * kWave;
+      at += (uint32_t)__popcll(set);
     }
-    __syncthreads();
-    if (wid == 0) {
-      int row = -1;
+  }
+  // ... and as a sub-chunk may hold many keys at T, those of the first are
+  // counted until they suffice, or until the rest, counted as one each, will
+  // give candidates that fit.  2^28 fp16 keys of four values: 148 us (763 by
+  // the radix select, which too many candidates lead to).
+  using KT = SortKey<DT>;
+  using Raw = typename KT::Raw;
+  constexpr int KV = TopkSub<DT, U>::V, Q = 4;
+  const uint32_t first = need;
+  uint32_t done = 0;
 #pragma unroll 1
-      for (int r0 = 0; r0 < kTkBoundThreads / kWave * V && row < 0; r0 += kWave) {
-        const int l = find(s_row[r0 + lane]);
-        if (l < kWave) row = r0 + l;
+  for (;;) {
+    __syncthreads();  // s_key is written, s_row was read
+#pragma unroll 1
+    for (int q = 0; q < Q; ++q) {
+      const uint32_t e = done + wid * Q + q;
+      uint32_t c = 0;
+      if (e < first) {
+        auto count = [&](auto full_c) {
+          constexpr bool FULL = decltype(full_c)::value;
+          const int64_t b = (int64_t)s_key[e] * TopkSub<DT, U>::kKeys + lane * KV;
+          Packed<Raw, KV> r[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) load_items<Raw, KV, FULL>(x, b + u * (kWave * KV), n, r[u]);
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int i = 0; i < KV; ++i)
+              c += (FULL || b + u * (kWave * KV) + i < n) && (KT::key(r[u][i]) ^ flip) == T ? 1u : 0u;
+          }
+        };
+        if ((int64_t)(s_key[e] + 1) * TopkSub<DT, U>::kKeys <= n) {
+          count(std::integral_constant<bool, true>{});
+        } else {
+          count(std::integral_constant<bool, false>{});
+        }
       }
-      if (lane == 0) {
-        s_at[0] = (uint32_t)row;
-        s_at[1] = need;
-      }
+      c = (uint32_t)wave_sum((int)c);
+      if (lane == 0) s_row[wid * Q + q] = c;
     }
     __syncthreads();
-    if ((int)s_at[0] >= 0) {
-      if ((int)s_at[0] / V == wid) {
-        need = s_at[1];
-        const uint32_t sub = b + s_at[0] * kWave + lane;
-        const int l = find(sub < subs && submax[sub] == T ? 1u : 0u);
-        if (lane == l) {
-          state[1] = T;
-          state[2] = sub;
-        }
+    // Every wave finds the same: 64 counts, one a lane.
+    const int l = find(s_row[lane]);
+    if (l < kWave) {
+      if (tid == 0) {
+        state[1] = T;
+        state[2] = s_key[done + l];
       }
       return;
     }
+    done += W * Q;
+    const uint32_t keys = first - need, expect = keys + need * (keys / done + 1);
+    if (expect + k <= kTkCandMax) break;
+  }
+  // `need` left, at most the sub-chunks not yet counted.
+  if (tid == 0) {
+    state[1] = T;
+    state[2] = s_key[done + need - 1];
   }
 }
 
@@ -1192,6 +1273,8 @@ static int topk_select(const typename SortKey<DT>::Raw* xr, int64_t n, int64_t k
   auto* psum = reinterpret_cast<uint64_t*>(w + L.psum_off);
   // Arrivals of the gated launches, zeroed with the gate by the maxima pass.
   uint32_t* arrived = gate ? gate + 8 : nullptr;
+  const auto* submax = reinterpret_cast<const uint32_t*>(sc + L.submax_off);
+  const int sub_shift = __builtin_ctz(L.mx.U * kWave * (16 / (int)sizeof(Raw)));
   const int sum_per = (L.groups + kTkSumGroups - 1) / kTkSumGroups;
   const int sum_groups = (L.groups + sum_per - 1) / sum_per;
   constexpr int64_t kTile = TopkGeom<DT>::kTile;
@@ -1204,10 +1287,10 @@ static int topk_select(const typename SortKey<DT>::Raw* xr, int64_t n, int64_t k
   for (int r = P - 1; r >= 0; --r) {
     if (kFuse && r == 0) {
       hipLaunchKernelGGL((topk_hist_kernel<DT, kFuse>), dim3(L.groups), dim3(kTkThreads), 0, st, xr, n, L.chunk,
-                         flip, r, k, state, partial, tstat, tlist, gate, arrived);
+                         flip, r, k, state, partial, tstat, tlist, gate, arrived, submax, sub_shift);
     } else {
       hipLaunchKernelGGL((topk_hist_kernel<DT, false>), dim3(L.groups), dim3(kTkThreads), 0, st, xr, n, L.chunk,
-                         flip, r, k, state, partial, nullptr, nullptr, gate, arrived);
+                         flip, r, k, state, partial, nullptr, nullptr, gate, arrived, submax, sub_shift);
     }
     TCS_CHECK_LAUNCH();
     if (!gate) {
@@ -1248,9 +1331,9 @@ static void topk_maxima_launch(const typename SortKey<DT>::Raw* xr, int64_t n, i
   auto* gcomp = reinterpret_cast<uint64_t*>(sc + L.gcomp_off);
   constexpr uint32_t W = kTkMaxThreads / kWave, W2 = kTkGatherThreads / kWave * kTkGatherSubs;
   hipLaunchKernelGGL((topk_max_kernel<DT, U>), dim3((L.mx.groups + W - 1) / W), dim3(kTkMaxThreads), 0, st, xr, n,
-                     flip, L.mx.per, L.mx.subs, L.mx.groups, submax, gcomp, mstate);
-  hipLaunchKernelGGL(topk_bound_kernel, dim3(1), dim3(kTkBoundThreads), 0, st, gcomp, L.mx.groups, submax,
-                     L.mx.subs, (uint32_t)k, SortKey<DT>::kBits, mstate);
+                     flip, L.mx.subs, L.mx.groups, submax, gcomp, mstate);
+  hipLaunchKernelGGL((topk_bound_kernel<DT, U>), dim3(1), dim3(kTkBoundThreads), 0, st, xr, n, flip, gcomp,
+                     L.mx.groups, submax, L.mx.subs, (uint32_t)k, mstate);
   hipLaunchKernelGGL((topk_gather_kernel<DT, U>), dim3((L.mx.subs + W2 - 1) / W2),
                      dim3(kTkGatherThreads), 0, st, xr, n, flip, L.mx.subs, submax, mstate,
                      reinterpret_cast<uint64_t*>(sc + L.word_off));

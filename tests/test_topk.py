@@ -250,6 +250,8 @@ def _path_input(kind, n, dtype, dev):
         v = torch.tensor([0.0, -0.0, float("inf"), float("-inf"), float("nan")], device=dev).to(dtype)
         at = torch.randint(0, n, (2000,), generator=g, device=dev)
         x[at] = v.repeat(400)
+    elif kind == "levels":  # a few keys of the largest value in every sub-chunk
+        x = torch.randint(-100, 100, (n,), generator=g, device=dev).to(dtype)
     elif kind == "lump":  # 30000 equal largest keys in one place, 100 above them elsewhere
         top = x.max() if dtype.is_floating_point else torch.iinfo(dtype).max - 1
         x[n // 3:n // 3 + 30000] = top
@@ -258,14 +260,15 @@ def _path_input(kind, n, dtype, dev):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind", ["random", "sorted", "ties", "constant", "special", "lump"])
+@pytest.mark.parametrize("kind", ["random", "sorted", "ties", "levels", "constant", "special", "lump"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.int16, torch.int8, torch.int32], ids=str)
 def test_topk_paths(ops, dev, kind, dtype):
     """Sizes on both sides of the sort's limit (2^22 keys of 1 and 2 bytes,
     2^19 of 4), with maxima of 1-vector and of 4-vector sub-chunks, enough
     groups for the maxima path or not, and more winners than it takes, against
-    the stable sort's first k.  Sorted, constant and lumped inputs give more
-    candidates than fit, so the radix select runs behind the maxima."""
+    the stable sort's first k.  With ties and levels the bound counts the keys
+    of the sub-chunks at it; sorted and lumped inputs give more candidates than
+    fit, so the radix select runs behind the maxima."""
     b = torch.empty(0, dtype=dtype).element_size()
     sizes = ([1 << 22, (1 << 22) + 1, 9_000_001, 70_000_003] if b <= 2 else
              [1 << 19, (1 << 19) + 1, 3_000_001, 34_000_003])
