@@ -496,20 +496,23 @@ __global__ __launch_bounds__((kCmpNW + 1) * kWave) void filter_kernel(
 
 // Counted compaction: the layout and helpers are in tcs_counted.hpp.
 
-// Block b (256 threads, 64K elements): wave w counts chunks w, w + 4, ...,
-// each lane 32 mask bytes of a chunk, four chunks' loads in flight at a
-// time.  Plain loads: the compaction that follows reads the mask again and
+// Block b (BLOCK threads, 64K elements): wave w counts chunks w, w + BLOCK /
+// 64, ..., each lane 32 mask bytes of a chunk, up to four chunks' loads in
+// flight at a time.  Plain loads: the compaction that follows reads the mask again and
 // finds part of it in the caches (count + compaction of fp32 values with
 // int32 indices at 2^28: 0.584 ms with nontemporal mask loads in both
 // passes, 0.547 ms with plain ones).
-__global__ __launch_bounds__(kCountBlock) void count_mask_chunks_kernel(const int8_t* __restrict__ mask,
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void count_mask_chunks_kernel(const int8_t* __restrict__ mask,
                                                                         int64_t n, int64_t* __restrict__ partial,
-                                                                        uint64_t* __restrict__ chunk_cnt) {
+                                                                        uint64_t* __restrict__ chunk_cnt,
+                                                                        int64_t* __restrict__ block_off,
+                                                                        int64_t* __restrict__ out) {
   const int lane = __lane_id();
   const int wid = threadIdx.x / kWave;
-  constexpr int kWaves = kCountBlock / kWave;
-  constexpr int kPerWave = kChunksPerBlock / kWaves;  // 8
-  constexpr int kBatch = 4;
+  constexpr int kWaves = BLOCK / kWave;
+  constexpr int kPerWave = kChunksPerBlock / kWaves;  // 8 or 2
+  constexpr int kBatch = kPerWave < 4 ? kPerWave : 4;
   const int64_t b0 = (int64_t)blockIdx.x * kCountChunk;
   uint32_t mine = 0;  // lane i keeps the count of chunk wid + 4i
   uint32_t tot = 0;
@@ -564,22 +567,28 @@ __global__ __launch_bounds__(kCountBlock) void count_mask_chunks_kernel(const in
 #pragma unroll
     for (int k = 0; k < kWaves; ++k) t += s[k];
     partial[blockIdx.x] = t;
+    if (gridDim.x == 1) {  // one block: count_scan_kernel is not run
+      block_off[0] = 0;
+      out[0] = t;
+    }
   }
 }
 
 // The chunk counts of a comparison (x cmp pivot) in the same layout: block
-// b (256 threads, 64K elements), wave w counts chunks w, w + 4, ..., each
+// b (BLOCK threads, 64K elements), wave w counts chunks w, w + BLOCK / 64, ..., each
 // lane 32 consecutive elements of a chunk; two chunks' loads in flight at
 // a time (plain loads, for the compaction's second read of x).  Elements
 // past n are not counted.
-template <class XT, class Keep>
-__global__ __launch_bounds__(kCountBlock) void count_keep_chunks_kernel(const XT* __restrict__ x, Keep keep,
+template <class XT, class Keep, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void count_keep_chunks_kernel(const XT* __restrict__ x, Keep keep,
                                                                         int64_t n, int64_t* __restrict__ partial,
-                                                                        uint64_t* __restrict__ chunk_cnt) {
+                                                                        uint64_t* __restrict__ chunk_cnt,
+                                                                        int64_t* __restrict__ block_off,
+                                                                        int64_t* __restrict__ out) {
   const int lane = __lane_id();
   const int wid = threadIdx.x / kWave;
-  constexpr int kWaves = kCountBlock / kWave;
-  constexpr int kPerWave = kChunksPerBlock / kWaves;  // 8
+  constexpr int kWaves = BLOCK / kWave;
+  constexpr int kPerWave = kChunksPerBlock / kWaves;  // 8 or 2
   constexpr int kBatch = 2;
   constexpr int kItems = (int)(kChunk / kWave);  // 32 per lane
   const int64_t b0 = (int64_t)blockIdx.x * kCountChunk;
@@ -627,6 +636,10 @@ __global__ __launch_bounds__(kCountBlock) void count_keep_chunks_kernel(const XT
 #pragma unroll
     for (int k = 0; k < kWaves; ++k) t += s[k];
     partial[blockIdx.x] = t;
+    if (gridDim.x == 1) {  // one block: count_scan_kernel is not run
+      block_off[0] = 0;
+      out[0] = t;
+    }
   }
 }
 
@@ -930,10 +943,15 @@ static int filter_count(const void* x, float pv, int64_t n, int64_t* count_out, 
   const int64_t np = (n + kCountChunk - 1) / kCountChunk;
   char* w = static_cast<char*>(ws);
   if (np > 0) {
-    hipLaunchKernelGGL((count_keep_chunks_kernel<XT, KeepCmp<DT, CMP>>), dim3((uint32_t)np), dim3(kCountBlock), 0,
-                       st, static_cast<const XT*>(x), KeepCmp<DT, CMP>{pv}, n,
-                       reinterpret_cast<int64_t*>(w + l.partial), reinterpret_cast<uint64_t*>(w + l.chunk_cnt));
+    const bool few = np <= kCountFewBlocks;
+    auto* kernel = few ? count_keep_chunks_kernel<XT, KeepCmp<DT, CMP>, kCountFewThreads>
+                       : count_keep_chunks_kernel<XT, KeepCmp<DT, CMP>, kCountBlock>;
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)np), dim3(few ? kCountFewThreads : kCountBlock), 0, st,
+                       static_cast<const XT*>(x), KeepCmp<DT, CMP>{pv}, n,
+                       reinterpret_cast<int64_t*>(w + l.partial), reinterpret_cast<uint64_t*>(w + l.chunk_cnt),
+                       reinterpret_cast<int64_t*>(w + l.block_off), count_out);
     TCS_CHECK_LAUNCH();
+    if (np == 1) return TCS_OK;
   }
   hipLaunchKernelGGL(count_scan_kernel, dim3(1), dim3(kScanBlock), 0, st,
                      reinterpret_cast<const int64_t*>(w + l.partial), np,
@@ -1003,9 +1021,13 @@ int tcs_count_mask(const int8_t* mask, int64_t n, int64_t* count_out, void* work
   const int64_t np = (n + kCountChunk - 1) / kCountChunk;
   char* w = static_cast<char*>(workspace);
   if (np > 0) {
-    hipLaunchKernelGGL(count_mask_chunks_kernel, dim3((uint32_t)np), dim3(kCountBlock), 0, st, mask, n,
-                       reinterpret_cast<int64_t*>(w + l.partial), reinterpret_cast<uint64_t*>(w + l.chunk_cnt));
+    const bool few = np <= kCountFewBlocks;
+    auto* kernel = few ? count_mask_chunks_kernel<kCountFewThreads> : count_mask_chunks_kernel<kCountBlock>;
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)np), dim3(few ? kCountFewThreads : kCountBlock), 0, st, mask, n,
+                       reinterpret_cast<int64_t*>(w + l.partial), reinterpret_cast<uint64_t*>(w + l.chunk_cnt),
+                       reinterpret_cast<int64_t*>(w + l.block_off), count_out);
     TCS_CHECK_LAUNCH();
+    if (np == 1) return TCS_OK;
   }
   hipLaunchKernelGGL(count_scan_kernel, dim3(1), dim3(kScanBlock), 0, st,
                      reinterpret_cast<const int64_t*>(w + l.partial), np,

@@ -25,8 +25,13 @@ template <> struct Bits<2> { using T = uint16_t; };
 template <> struct Bits<4> { using T = uint32_t; };
 template <> struct Bits<8> { using T = uint64_t; };
 
-// Count passes: 256-thread workgroups over 64K-element blocks.
+// Count passes: a workgroup for each 64K-element block, of 256 threads, or of
+// 1024 where there are no more blocks than CUs (all in flight at once, so the
+// pass takes as long as one: filter of 10000019 fp16 values, whole call, 35.7
+// us with 256 and 30.9 with 1024; 2^28 fp32 values 413 and 437).
 constexpr int kCountBlock = 256;
+constexpr int kCountFewThreads = 1024;
+constexpr int64_t kCountFewBlocks = 256;
 constexpr int64_t kCountChunk = 1 << 16;
 constexpr int64_t kChunk = 2048;                              // elements per wave chunk
 constexpr int kChunksPerBlock = (int)(kCountChunk / kChunk);  // 32

@@ -990,12 +990,14 @@ at::Tensor filter_impl(const at::Tensor& x_in, double pivot, int cmp, bool value
   TORCH_CHECK(n < ((int64_t)1 << 31), op, ": at most 2^31 - 1 elements");
   auto ws = workspace(x, tcs_compress_workspace_bytes(n));
   const at::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-  at::Tensor cnt = at::zeros({1}, x.options().dtype(at::kLong));
-  if (n > 0)
+  int64_t k = 0;
+  if (n > 0) {
+    at::Tensor cnt = at::empty({1}, x.options().dtype(at::kLong));
     check(tcs_count_filter(x.data_ptr(), dtype_code(t), pivot, cmp, n, cnt.data_ptr<int64_t>(), ws.first,
                            ws.second, stream_of(x)),
           op);
-  const int64_t k = cnt.item<int64_t>();
+    k = cnt.item<int64_t>();
+  }
   at::Tensor out = values ? at::empty({k}, x.options()) : at::empty({k}, x.options().dtype(at::kInt));
   if (k > 0) {
     // The count pass left the chunk counts in this workspace.

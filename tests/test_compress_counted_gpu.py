@@ -130,3 +130,16 @@ def test_counted_capacity_and_lookback_identical(lib, dev):
     z3, zi3, _, ox, _ = _run(lib, dev, x, m, 2, cap=cap)
     assert torch.equal(z3, z1[:cap]) and torch.equal(zi3, zi1[:cap])
     assert int(torch.count_nonzero(ox[cap:])) == 0
+
+
+@pytest.mark.parametrize("n", [65535, 65536, 65537, 256 * 65536, 256 * 65536 + 1])
+def test_count_blocks(ops, dev, n):
+    """One block (counted without the scan of the block counts), and the block
+    counts on both sides of the change of workgroup size."""
+    g = torch.Generator(device=dev).manual_seed(n)
+    x = torch.randn(n, generator=g, device=dev)
+    m = (torch.rand(n, generator=g, device=dev) < 0.3).to(torch.int8)
+    for v in (x, x.half()):
+        assert torch.equal(ops.run_compress(v, m, 128), v[m == 1])
+        assert torch.equal(ops.run_filter_greater_eq(v, 0.5, 128), v[v >= 0.5])
+        assert torch.equal(ops.run_where(v, 0.5, 128).long(), (v >= 0.5).nonzero().flatten())
