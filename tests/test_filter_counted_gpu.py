@@ -146,3 +146,29 @@ def test_counted_filter_rejects(lib, dev):
                                   ws.numel(), s) != 0
     assert lib.tcs_filter_counted(x.data_ptr(), F32, 0.0, CMP_GE, out.data_ptr(), None, 4096, 4096, ws.data_ptr(),
                                   64, s) != 0
+
+
+def test_counts_of_threads_and_streams(ops, dev):
+    """Filters and compactions of several threads, each on a stream of its
+    own, read their own counts."""
+    import threading
+
+    wrong = []
+
+    def run(seed):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for i in range(40):
+                x = torch.randn(1000 * seed + 37 * i + 1, generator=g, device=dev)
+                m = (x > 0.1 * seed).to(torch.int8)
+                if not torch.equal(ops.run_filter_greater_eq(x, 0.2 * seed, 128), x[x >= torch.tensor(0.2 * seed)]):
+                    wrong.append((seed, i))
+                if not torch.equal(ops.run_compress(x, m, 128), x[m == 1]):
+                    wrong.append((seed, -i))
+
+    threads = [threading.Thread(target=run, args=(s,)) for s in range(1, 5)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
