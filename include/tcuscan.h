@@ -376,6 +376,13 @@ int tcs_seg_scan_revert(const float* scan_x, const int32_t* scan_f, const float*
  * 352-353 and 392-393), which is torch code there. */
 int tcs_top_p_keep(const void* sorted_probs, const float* mass, float p, float* kept, int64_t n, void* stream);
 
+/* The same weights divided by their sum (added in double, rounded to float32
+ * once).  Every workgroup reads a double of each 2048 elements, so it suits
+ * n up to some 2^21.  Workspace: 8-byte aligned scratch, any contents. */
+size_t tcs_top_p_renorm_workspace_bytes(int64_t n);
+int tcs_top_p_renorm(const void* sorted_probs, const float* mass, float p, float* kept, int64_t n, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------
  * Split (stable partition)
  * --------------------------------------------------------------------- */

@@ -7,7 +7,8 @@ renormalise, draw with torch.multinomial and map the draw back through the
 sort's indices.  Here the sort is run_radix_sort_ex (descending, stable: the
 order of sample_top_p at :372-392; the reference's tcuscan_top_p sorts
 ascending), the scan run_scan_multi_core (fp16 in, float32 out, each prefix
-rounded once) and the mask one fused kernel (run_top_p_keep).
+rounded once) and the mask one fused kernel (run_top_p_keep, which also
+renormalises for the filter).
 
 sample_top_p draws by inverting the kept weights' cumulative distribution:
 their inclusive scan (run_scan_single_core, float32 rounded once per prefix)
@@ -22,12 +23,12 @@ import torch
 import tcuscan_ops
 
 
-def _kept(probs: torch.Tensor, p: float, S: int):
+def _kept(probs: torch.Tensor, p: float, S: int, renorm: bool = False):
     if probs.dim() != 1 or probs.dtype != torch.float16:
         raise RuntimeError("top_p: probs must be a 1-D float16 tensor")
     probs_sort, order = tcuscan_ops.run_radix_sort_ex(probs, True)
     mass = tcuscan_ops.run_scan_multi_core(probs_sort, S)
-    return tcuscan_ops.run_top_p_keep(probs_sort, mass, p), order
+    return tcuscan_ops.run_top_p_keep(probs_sort, mass, p, renorm), order
 
 
 def top_p_filter(probs: torch.Tensor, p: float, S: int = 128):
@@ -37,8 +38,7 @@ def top_p_filter(probs: torch.Tensor, p: float, S: int = 128):
 
     probs: 1-D float16 on the GPU.
     """
-    kept, order = _kept(probs, p, S)
-    return kept / kept.sum(), order
+    return _kept(probs, p, S, renorm=True)
 
 
 def sample_top_p(probs: torch.Tensor, p: float, S: int = 128, generator: torch.Generator | None = None):

@@ -103,3 +103,23 @@ def test_sample_top_p_frequencies(dev):
         sd = (draws * q * (1 - q)) ** 0.5
         assert abs(counts.get(i, 0) - draws * q) <= 5 * sd + 1, (i, counts.get(i, 0), draws * q)
     assert all(int(tcuscan.sample_top_p(x, 0.0, generator=g)) == 0 for _ in range(20))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 300_001, 1 << 21, (1 << 21) + 1])
+def test_top_p_keep_divided_by_its_sum(ops, dev, n):
+    """run_top_p_keep(renorm=True) against its weights divided by their sum in
+    float64: the sum and the quotient are rounded once each (two halves of
+    2^-23), above 2^21 elements torch adds in float32.  All weights dropped
+    give NaN, a NaN spreads, as 0 / 0 and the sum do."""
+    srt = torch.sort(_probs(n, n), descending=True).values.to(dev)
+    mass = ops.run_scan_multi_core(srt, 128)
+    for p in (0.0, 0.3, 2.0):
+        kept = ops.run_top_p_keep(srt, mass, p)
+        got = ops.run_top_p_keep(srt, mass, p, renorm=True)
+        exp = kept.double() / kept.double().sum()
+        assert got.dtype == torch.float32 and got.shape == kept.shape
+        assert torch.allclose(got.double(), exp, rtol=1e-6 if n > 1 << 21 else 2.0**-22, atol=0)
+    assert bool(ops.run_top_p_keep(srt, mass, -1.0, renorm=True).isnan().all())
+    srt[n // 2] = float("nan")
+    assert bool(ops.run_top_p_keep(srt, mass, 2.0, renorm=True).isnan().all())
