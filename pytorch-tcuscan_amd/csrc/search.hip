@@ -197,7 +197,7 @@ __device__ __forceinline__ BucketMap bucket_map(const int32_t* __restrict__ sort
 // kSsLongGap.  wide[block] = the block's elements whose bucket holds the
 // element kSsWide places back too.
 __global__ __launch_bounds__(kSsThreads) void bucket_start_kernel(const int32_t* __restrict__ sorted, int32_t len,
-                                                                  int32_t per_block, int bits,
+                                                                  int64_t per_block, int bits,
                                                                   int32_t* __restrict__ wide,
                                                                   int32_t* __restrict__ start) {
   static_assert(kSsWide == kWave, "the element kSsWide places back is the row before's");
@@ -837,7 +837,7 @@ int tcs_searchsorted_indexed(const int32_t* sorted, int64_t sorted_len, const in
   auto* wide = static_cast<int32_t*>(workspace);
   int32_t* start = wide + kSsBuildBlocks;
   const int32_t len = (int32_t)sorted_len;
-  const int32_t per_block = (len + kSsBuildBlocks - 1) / kSsBuildBlocks;
+  const int64_t per_block = (sorted_len + kSsBuildBlocks - 1) / kSsBuildBlocks;
   hipLaunchKernelGGL(bucket_start_kernel, dim3(kSsBuildBlocks), dim3(kSsThreads), 0, st, sorted, len, per_block, bits,
                      wide, start);
   TCS_CHECK_LAUNCH();

@@ -1,0 +1,51 @@
+"""searchsorted at the ends of what its arguments allow (GPU): the longest
+haystacks."""
+import ctypes
+import os
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(REPO, "pytorch-tcuscan_amd", "libtcuscan_hip.so")
+I32_MIN, I32_MAX = -2**31, 2**31 - 1
+
+
+@pytest.fixture(scope="module")
+def lib():
+    lib = ctypes.CDLL(LIB)
+    lib.tcs_searchsorted_indexed.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
+                                             ctypes.c_int64, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+    for f in (lib.tcs_searchsorted_workspace_bytes, lib.tcs_searchsorted_preferred_bytes):
+        f.restype = ctypes.c_size_t
+    lib.tcs_searchsorted_workspace_bytes.argtypes = [ctypes.c_int64]
+    lib.tcs_searchsorted_preferred_bytes.argtypes = [ctypes.c_int64, ctypes.c_int64]
+    return lib
+
+
+def _indexed(lib, hay, needles, wsb):
+    """The lower bounds by tcs_searchsorted_indexed with wsb bytes of stale
+    workspace; nothing written past it."""
+    ws = torch.full((wsb // 4 + 8,), -1, dtype=torch.int32, device=hay.device)
+    out = torch.full_like(needles, -7)
+    assert lib.tcs_searchsorted_indexed(hay.data_ptr(), hay.numel(), needles.data_ptr(), out.data_ptr(),
+                                        needles.numel(), ws.data_ptr(), wsb,
+                                        torch.cuda.current_stream().cuda_stream) == 0
+    assert bool((ws[wsb // 4:] == -1).all())
+    return out
+
+
+@pytest.mark.parametrize("n", [2**31 - 512, 2**31 - 1])
+def test_longest_haystacks(lib, ops, dev, n):
+    """n elements -2^30, -2^30 + 1, ...: from n = 2^31 - 511 on the table
+    build's elements per workgroup, rounded up, pass int32."""
+    hay = torch.arange(-2**30, n - 2**30, dtype=torch.int32, device=dev)
+    g = torch.Generator(device=dev).manual_seed(31)
+    v = torch.randint(I32_MIN, I32_MAX, ((1 << 23) + 5,), generator=g, device=dev, dtype=torch.int32)
+    v[:4] = torch.tensor([I32_MIN, I32_MAX, -2**30, n - 2**30 - 1], dtype=torch.int32)
+    exp = (v.long() + 2**30).clamp(0, n).int()
+    for m in (70_000, v.numel()):
+        assert torch.equal(ops.run_searchsorted(hay, v[:m].contiguous()), exp[:m])
+        assert torch.equal(_indexed(lib, hay, v[:m].contiguous(), lib.tcs_searchsorted_workspace_bytes(n)), exp[:m])
