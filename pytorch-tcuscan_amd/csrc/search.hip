@@ -211,7 +211,15 @@ __global__ __launch_bounds__(kSsThreads) void bucket_start_kernel(const int32_t*
   const int lane = __lane_id(), wid = threadIdx.x / kWave;
   const int64_t b0 = (int64_t)blockIdx.x * per_block;
   const int64_t b1 = b0 + per_block < len ? b0 + per_block : len;
-  auto bucket = [&](int32_t v) { return (order_key(v) - m.umin) >> m.shift; };
+  // A haystack that is not sorted may hold keys outside [umin, umax] and
+  // buckets that fall.  Buckets end at m.used - 1 and only a rise writes
+  // entries, so every write lies in the table; and as the first element's
+  // bucket is 0 and the last one's m.used - 1, every entry is crossed by a
+  // rise and holds an index of the haystack.
+  auto bucket = [&](int32_t v) {
+    const uint32_t k = (order_key(v) - m.umin) >> m.shift;
+    return k < m.used ? k : m.used - 1u;
+  };
   int nwide = 0;
   for (int64_t w = b0 + (int64_t)wid * (R * kWave); w < b1; w += (int64_t)kSsThreads * R) {
     // Row -1 first; rows past the end repeat the haystack's last element.
@@ -231,7 +239,8 @@ __global__ __launch_bounds__(kSsThreads) void bucket_start_kernel(const int32_t*
       const uint32_t above = (uint32_t)readlane((int)b[j - 1], kWave - 1);
       const uint32_t prev = lane > 0 ? left : above;
       const uint32_t first = p == 0 ? 0u : prev + 1u;
-      const uint32_t gap = p < b1 ? b[j] + 1u - first : 0u;  // entries [first, first + gap) start here
+      // Entries [first, first + gap) start here; none after a bucket above.
+      const uint32_t gap = p < b1 && b[j] >= first ? b[j] + 1u - first : 0u;
       nwide += p < b1 && p >= kSsWide && b[j - 1] == b[j] ? 1 : 0;
       if (gap <= 8u) {
         for (uint32_t k = 0; k < gap; ++k) start[first + k] = (int32_t)p;
@@ -243,22 +252,27 @@ __global__ __launch_bounds__(kSsThreads) void bucket_start_kernel(const int32_t*
         const uint32_t f = (uint32_t)readlane((int)first, l), g = (uint32_t)readlane((int)gap, l);
         const int32_t at = (int32_t)(w + (j - 1) * kWave) + l;
         if (g > kSsLongGap) {
+          int q = 0;
           if (lane == 0) {
-            const int q = atomicAdd(&s_gaps, 1);
-            s_first[q] = f;
-            s_last[q] = f + g;
-            s_at[q] = at;
+            q = atomicAdd(&s_gaps, 1);
+            if (q < kSsLongGaps) {
+              s_first[q] = f;
+              s_last[q] = f + g;
+              s_at[q] = at;
+            }
           }
-        } else {
-          for (uint32_t k = lane; k < g; k += kWave) start[f + k] = at;
+          // Rises of a sorted haystack have room for all of theirs.
+          if (__builtin_amdgcn_readfirstlane(q) < kSsLongGaps) continue;
         }
+        for (uint32_t k = lane; k < g; k += kWave) start[f + k] = at;
       }
     }
   }
   nwide = wave_sum(nwide);
   if (lane == 0 && nwide) atomicAdd(&s_wide, nwide);
   __syncthreads();
-  for (int q = 0; q < s_gaps; ++q) {
+  const int gaps = s_gaps < kSsLongGaps ? s_gaps : kSsLongGaps;
+  for (int q = 0; q < gaps; ++q) {
     for (uint32_t k = s_first[q] + threadIdx.x; k < s_last[q]; k += kSsThreads) start[k] = s_at[q];
   }
   if (threadIdx.x == 0) {

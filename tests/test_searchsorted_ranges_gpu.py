@@ -1,5 +1,6 @@
 """searchsorted at the ends of what its arguments allow (GPU): the longest
-haystacks."""
+haystacks, and haystacks that are not sorted, whose results are unspecified
+but stay in range."""
 import ctypes
 import os
 
@@ -49,3 +50,31 @@ def test_longest_haystacks(lib, ops, dev, n):
     for m in (70_000, v.numel()):
         assert torch.equal(ops.run_searchsorted(hay, v[:m].contiguous()), exp[:m])
         assert torch.equal(_indexed(lib, hay, v[:m].contiguous(), lib.tcs_searchsorted_workspace_bytes(n)), exp[:m])
+
+
+@pytest.mark.parametrize("n", [70_001, (1 << 20) + 3, (1 << 22) + 5])
+@pytest.mark.parametrize("order", ["descending", "shuffled", "zigzag", "beyond_ends", "sorted"])
+def test_unsorted_haystacks_stay_in_range(lib, ops, dev, n, order):
+    """Every answer lies in [0, n] and nothing outside the workspace and the
+    outputs is written, whatever the order of the haystack: by sixteen lanes
+    a needle, by the table (of the least workspace and the preferred one) and
+    by slices; a later search of a sorted haystack is right."""
+    g = torch.Generator(device=dev).manual_seed(n)
+    hay = torch.randint(I32_MIN, I32_MAX, (n,), generator=g, device=dev, dtype=torch.int32).sort().values
+    good = hay.clone()
+    if order == "descending":
+        hay = hay.flip(0).contiguous()
+    elif order == "shuffled":
+        hay = hay[torch.randperm(n, generator=g, device=dev)]
+    elif order == "zigzag":  # falls and rises across the whole table
+        hay[0::2], hay[1::2] = good[: (n + 1) // 2], good[(n + 1) // 2:].flip(0)
+    elif order == "beyond_ends":  # keys outside the first and last element
+        hay[n // 3], hay[n // 2], hay[0], hay[-1] = I32_MIN, I32_MAX, -1000, 1000
+    for m in (1000, 70_000, 600_001, (3 << 20) + 5):
+        v = torch.randint(I32_MIN, I32_MAX, (m,), generator=g, device=dev, dtype=torch.int32)
+        for out in (ops.run_searchsorted(hay, v), _indexed(lib, hay, v, lib.tcs_searchsorted_workspace_bytes(n)),
+                    _indexed(lib, hay, v, lib.tcs_searchsorted_preferred_bytes(n, m))):
+            assert int(out.min()) >= 0 and int(out.max()) <= n
+            if order == "sorted":
+                assert torch.equal(out, torch.searchsorted(hay, v, out_int32=True))
+        assert torch.equal(ops.run_searchsorted(good, v), torch.searchsorted(good, v, out_int32=True))
