@@ -7,11 +7,17 @@ extern "C" {
 
 size_t tcs_scan_workspace_bytes(int64_t n, int S, int tiles_per_wg) {
   if (n <= 0 || S <= 0) return tcs::lookback_ws_bytes(0);
-  // Sized for the smallest tile any dtype uses with these parameters (the
-  // default tile of short inputs is 8K).
+  // Sized for the smallest tile any dtype uses with these parameters: with
+  // the default ones 8192 elements, and kShortTile up to kShortMax.  Never
+  // less for a larger n, so that a workspace of the largest serves them all.
   int64_t tile = tcs::tile_elems_for(S, tiles_per_wg);
   if (tile > 16384) tile = 16384;
-  if (tiles_per_wg <= 0 && tile > 8192) tile = 8192;
+  if (tiles_per_wg <= 0) {
+    if (tile > 8192) tile = 8192;
+    const int64_t ns = n < tcs::kShortMax ? n : tcs::kShortMax;
+    const int64_t few = (ns + tcs::kShortTile - 1) / tcs::kShortTile, many = (n + tile - 1) / tile;
+    return tcs::lookback_ws_bytes((uint64_t)(few > many ? few : many));
+  }
   return tcs::lookback_ws_bytes((uint64_t)((n + tile - 1) / tile));
 }
 
