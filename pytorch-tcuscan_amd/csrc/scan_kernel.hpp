@@ -866,8 +866,8 @@ static int scan_dispatch(const void* x, int x_dtype, void* y, const int8_t* flag
   // The shipped local scan is the faster one measured on MI355X at
   // N = 2^28 with the default tiles: DPP for every dtype (fp16 5.6 vs 3.7
   // TB/s on the matrix units; int8 5.1 vs 4.4).
+  const bool dflt = tiles_per_wg <= 0 && method == TCS_METHOD_AUTO && window == 0;
   if (method == TCS_METHOD_AUTO) method = TCS_METHOD_DPP;
-  const bool dflt = tiles_per_wg <= 0 && method == TCS_METHOD_DPP && window == 0;
   // Default look-back window, measured the same way: 6 for DPP (fp16 265 us
   // at 6 vs 272 at 8, 284 at 16, 420 at 1; bf16 263 vs 270; int8 level from
   // 5 to 8), 32 for the matrix-unit scan.

@@ -52,3 +52,13 @@ def test_larger_scans_keep_their_tiles(lib, dev, n):
     need = lib.tcs_scan_workspace_bytes(n, 128, 0)
     assert need >= lib.tcs_scan_workspace_bytes(SHORT_MAX, 128, 0)
     assert _scan_tiles(lib, x, need) < -(-n // SHORT_TILE)
+
+
+@pytest.mark.parametrize("n", [65_537, 1 << 20])
+def test_a_named_method_is_not_the_short_scan(lib, dev, n):
+    """TCS_METHOD_DPP (1) and TCS_METHOD_MFMA (2) run the pipelined scan with
+    that local scan, whatever the workspace holds."""
+    x = uniform_pm1(n, torch.float16, n).to(dev)
+    need = lib.tcs_scan_workspace_bytes(n, 128, 0)
+    for method in (1, 2):
+        assert _scan_tiles(lib, x, need, method) < -(-n // SHORT_TILE)
