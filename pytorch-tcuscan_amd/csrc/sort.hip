@@ -584,7 +584,11 @@ inline SortLayout sort_layout(int64_t n, int dt) {
   while (L.wide && L.parts < 4 && L.chunk / L.parts > 16384) L.parts *= 2;
   L.tmpv_off = align256((size_t)n * sort_elem_bytes(dt));
   L.counts_off = align256(L.tmpv_off + (size_t)n * 4);
-  L.totals_off = align256(L.counts_off + (size_t)L.chunks * L.parts * 256 * 4);
+  // Room for the most rows of counts up to this many keys: rounding chunks
+  // up to whole units can leave fewer chunks for more keys, and scratch of a
+  // larger n is to serve a smaller one.
+  const int64_t rows = L.wide ? (int64_t)kSortMaxRows : (n + least - 1) / least;
+  L.totals_off = align256(L.counts_off + (size_t)(rows < most || L.wide ? rows : most) * 256 * 4);
   L.scratch = align256(L.totals_off + 256 * 4);
   return L;
 }
