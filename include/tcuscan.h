@@ -424,7 +424,9 @@ int tcs_sort(const void* x, int dtype, const int32_t* idx_in, void* out_x, int32
  * --------------------------------------------------------------------- */
 
 /* Workspace (zeroed once, reusable) and scratch (any contents) of tcs_topk;
- * 0 for an unsupported dtype. */
+ * 0 for an unsupported dtype.  Scratch of larger sizes is taken for smaller
+ * ones; where it is less than this returns for theirs, the selection is by
+ * radix select. */
 size_t tcs_topk_workspace_bytes(int64_t n, int64_t k, int dtype);
 size_t tcs_topk_scratch_bytes(int64_t n, int64_t k, int dtype);
 

@@ -1218,15 +1218,20 @@ inline TopkPath topk_path(const TopkMaxima& m, int64_t n, int64_t k, int key_byt
 
 struct TopkLayout {
   size_t state_off, part_off, psum_off, own_total;
-  size_t cand_i_off, tcnt_off, tstat_off, tlist_off, sort_scratch_off, scratch;
+  size_t cand_i_off, tcnt_off, tstat_off, tlist_off, sort_scratch_off, scratch, least;
   size_t word_off, submax_off, gcomp_off, mstate_off;  // maxima path and rank words
   int groups;
   int64_t chunk;
   TopkMaxima mx;
   TopkPath path;
+  bool words;  // the selected keys are ranked by counting
 };
 
-inline TopkLayout topk_layout(int64_t n, int64_t k, int dt) {
+// Scratch of the select with its keys sorted: it does not fall as n or k
+// grow, and is the least that tcs_topk takes, so that scratch of the largest
+// sizes serves them all.  Where `avail` bytes do not hold the way that the
+// sizes take, the select runs.
+inline TopkLayout topk_layout(int64_t n, int64_t k, int dt, size_t avail = SIZE_MAX) {
   TopkLayout L{};
   const uint64_t tiles = (uint64_t)((n + kTkTileMin - 1) / kTkTileMin);
   int64_t groups = (n + 65535) / 65536;
@@ -1251,12 +1256,18 @@ inline TopkLayout topk_layout(int64_t n, int64_t k, int dt) {
   const int kb = topk_elem_bytes(dt);
   L.mx = topk_maxima(n, k, kb);
   L.path = topk_path(L.mx, n, k, kb);
+  L.words = k <= kTkRankMax;
   L.word_off = align256(L.sort_scratch_off +
                         (L.path == TopkPath::kSort ? sort_first_scratch_bytes(n, dt) : tcs_sort_scratch_bytes(k, dt)));
   L.submax_off = align256(L.word_off + (size_t)kTkCandMax * 8);
   L.gcomp_off = align256(L.submax_off + (size_t)L.mx.subs * 4);
   L.mstate_off = align256(L.gcomp_off + (size_t)L.mx.groups * 8);
   L.scratch = L.mstate_off + 256;
+  L.least = L.sort_scratch_off + tcs_sort_scratch_bytes(k, dt);
+  if (L.scratch > avail) {
+    L.path = TopkPath::kSelect;
+    L.words = false;
+  }
   return L;
 }
 
@@ -1344,7 +1355,7 @@ static int topk_run(const void* x, int64_t n, int64_t k, bool largest, void* out
                     size_t ws_bytes, void* scratch, size_t scratch_bytes, hipStream_t st) {
   using KT = SortKey<DT>;
   using Raw = typename KT::Raw;
-  const TopkLayout L = topk_layout(n, k, DT);
+  const TopkLayout L = topk_layout(n, k, DT, scratch_bytes);
   char* w = static_cast<char*>(ws);
   char* sc = static_cast<char*>(scratch);
   if (L.path == TopkPath::kSort)
@@ -1353,7 +1364,7 @@ static int topk_run(const void* x, int64_t n, int64_t k, bool largest, void* out
   const Raw* xr = static_cast<const Raw*>(x);
   constexpr int64_t kTile = TopkGeom<DT>::kTile;
   if (L.chunk % kTile != 0 || L.chunk / kTile > kTkMaxChunkTiles) return TCS_ERR_INVALID_ARG;
-  if (k > kTkRankMax) {
+  if (!L.words) {
     const int rc = topk_select<DT, false>(xr, n, k, flip, L, w, sc, nullptr, st);
     if (rc != TCS_OK) return rc;
     // Largest first (smallest first for !largest), ties in input order.
@@ -1406,7 +1417,7 @@ int tcs_topk(const void* x, int dtype, int64_t n, int64_t k, int largest, void* 
   if (k == 0) return TCS_OK;
   if (!x || !out_vals || !out_idx || !aligned16(x)) return TCS_ERR_INVALID_ARG;
   if (!workspace || workspace_bytes < tcs_topk_workspace_bytes(n, k, dtype)) return TCS_ERR_WORKSPACE;
-  if (!scratch || scratch_bytes < tcs_topk_scratch_bytes(n, k, dtype)) return TCS_ERR_WORKSPACE;
+  if (!scratch || scratch_bytes < topk_layout(n, k, dtype).least) return TCS_ERR_WORKSPACE;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool lg = largest != 0;
   switch (dtype) {

@@ -51,3 +51,28 @@ def test_sort_in_the_scratch_of_a_larger_one(lib, dev, dtype):
                             ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
         ref = torch.sort(x, stable=True)
         assert torch.equal(y, ref.values) and torch.equal(idx.long(), ref.indices)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.int8, torch.int32], ids=str)
+def test_topk_in_the_scratch_of_a_larger_one(lib, dev, dtype):
+    """The scratch and workspace of the largest of several calls serve them
+    all, whichever way each size takes by itself."""
+    code = {torch.float16: 0, torch.int8: 3, torch.int32: 5}[dtype]
+    top, kmax = (1 << 23) + 5, 3000
+    scratch = torch.full((lib.tcs_topk_scratch_bytes(top, kmax, code),), -1, dtype=torch.int8, device=dev)
+    ns = (top, 4_300_001, 1 << 21, 1 << 18, 5000)
+    ws = torch.zeros(max(lib.tcs_topk_workspace_bytes(n, kmax, code) for n in ns), dtype=torch.uint8, device=dev)
+    g = torch.Generator(device=dev).manual_seed(2)
+    for n in ns:
+        x = torch.randint(-128 if code == 3 else -30000, 128 if code == 3 else 30000, (n,), generator=g,
+                          device=dev).to(dtype)
+        ref = torch.sort(x, descending=True, stable=True)
+        for k in (1, 300, kmax):
+            y, idx = torch.empty(k, dtype=dtype, device=dev), torch.empty(k, dtype=torch.int32, device=dev)
+            assert lib.tcs_topk(ctypes.c_void_p(x.data_ptr()), code, ctypes.c_int64(n), ctypes.c_int64(k), 1,
+                                ctypes.c_void_p(y.data_ptr()), ctypes.c_void_p(idx.data_ptr()),
+                                ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(ws.numel()),
+                                ctypes.c_void_p(scratch.data_ptr()), ctypes.c_size_t(scratch.numel()),
+                                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+            assert torch.equal(y, ref.values[:k]) and torch.equal(idx.long(), ref.indices[:k]), (n, k)
