@@ -1036,9 +1036,13 @@ __global__ __launch_bounds__(kTkBoundThreads) void topk_bound_kernel(const typen
 
 // Appends the keys above T, or equal to T in a sub-chunk up to P, as rank
 // words.  A wave looks at kTkGatherSubs sub-chunk maxima and reads the
-// sub-chunks that reach the bound; a workgroup's words meet in LDS and take
-// their place in cand_w with one atomic.  state[0] counts them all, stored
-// or not.
+// sub-chunks that reach the bound, one after the other.  Those may lie
+// together, at the front where keys repeat, so the ones a wave and a
+// workgroup look at lie apart (2^25 random int8 keys, k = 2048: 37 us with
+// consecutive ones, 6 so; and 2^28 fp16 keys of four values, k = 4096, gave
+// one workgroup more words than its list holds, 800 us with the select behind
+// it, 146 so).  A workgroup's words meet in LDS and take their place in cand_w
+// with one atomic.  state[0] counts them all, stored or not.
 constexpr int kTkGatherThreads = 512, kTkGatherSubs = 32;
 template <int DT, int U>
 __global__ __launch_bounds__(kTkGatherThreads) void topk_gather_kernel(
@@ -1055,8 +1059,10 @@ __global__ __launch_bounds__(kTkGatherThreads) void topk_gather_kernel(
   if (tid == 0) s_n = 0;
   const uint32_t T = state[1], P = state[2];
   __syncthreads();
-  const uint32_t first = (blockIdx.x * (kTkGatherThreads / kWave) + wid) * kTkGatherSubs;
-  const uint32_t s = first + lane;
+  // The wave's sub-chunks: first, first + step, ...; consecutive ones belong
+  // to different workgroups.
+  const uint32_t first = wid * gridDim.x + blockIdx.x, step = gridDim.x * (kTkGatherThreads / kWave);
+  const uint32_t s = first + lane * step;
   const bool look = lane < kTkGatherSubs && s < subs;
   const uint32_t m = look ? submax[s] : 0u;
   uint64_t active = __ballot(look && (m > T || (m == T && s <= P)));
@@ -1064,7 +1070,7 @@ __global__ __launch_bounds__(kTkGatherThreads) void topk_gather_kernel(
   while (active != 0 && __hip_atomic_load(&s_n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= kList) {
     const int l = __builtin_ctzll(active);
     active &= active - 1;
-    const uint32_t sub = first + l;
+    const uint32_t sub = first + l * step;
     const int64_t b = (int64_t)sub * SUB + lane * V;
     const uint32_t least = sub <= P ? T : T + 1;  // T + 1 wraps only if nothing is above T
     const bool none = sub > P && T == 0xffffffffu;
