@@ -78,6 +78,10 @@ inline int64_t topk_tile(int key_bytes) { return (int64_t)kTkNW * (key_bytes <= 
 // The kernels of the radix select take `gate`: null, or the candidate count
 // of the maxima path, which has succeeded when the count fits.
 constexpr uint32_t kTkCandMax = 8192;  // 64 KiB of LDS
+// Words of the maxima path's state: candidates, the bound's T and P, arrivals
+// and digit counts of the gated launches.
+constexpr int kTkArrived = 8, kTkBins = 64, kTkStateWords = kTkBins + 256;
+constexpr uint32_t kTkGatedGroups = 256;
 __device__ __forceinline__ bool topk_done(const uint32_t* gate) { return gate && *gate <= kTkCandMax; }
 
 // Behind a gate the last workgroup of a launch also runs the small step that
@@ -112,22 +116,13 @@ __device__ __forceinline__ void topk_leave(uint64_t* p, uint64_t v, bool shared)
 
 // Picks digit r of the k-th largest key: the bin b where the count of keys
 // in bins >= b first reaches the number still to take.  One workgroup of NT
-// threads.
-template <int NT, bool SHARED>
-__device__ __forceinline__ void topk_pick(const uint64_t* partial, int groups, int r, int first, int64_t k,
-                                          uint64_t* state) {
+// threads; count(d, q, nq) is thread q's share of digit d's keys, of nq threads
+// a digit.
+template <int NT, class F>
+__device__ __forceinline__ void topk_pick(F count, int r, int first, int64_t k, uint64_t* state) {
   constexpr int NQ = NT / 256;
   const int tid = threadIdx.x, d = tid & 255, q = tid >> 8;
-  uint32_t s = 0;
-  int g = q;
-  for (; g + 7 * NQ < groups; g += 8 * NQ) {  // eight loads in flight
-    uint64_t v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = topk_read<SHARED>(&partial[(size_t)(g + NQ * u) * 256 + d]);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += (uint32_t)v[u];
-  }
-  for (; g < groups; g += NQ) s += (uint32_t)topk_read<SHARED>(&partial[(size_t)g * 256 + d]);
+  const uint32_t s = count(d, q, NQ);
   __shared__ uint32_t sr[NQ][256];
   __shared__ uint32_t ws[4];
   __shared__ uint64_t s_state[2];
@@ -178,6 +173,7 @@ __global__ __launch_bounds__(kTkThreads) void topk_hist_kernel(const typename So
                                                                uint8_t* __restrict__ tlist,
                                                                const uint32_t* __restrict__ gate,
                                                                uint32_t* __restrict__ arrived,
+                                                               uint32_t* __restrict__ bins,
                                                                const uint32_t* __restrict__ submax, int sub_shift) {
   if (topk_done(gate)) return;
   using KT = SortKey<DT>;
@@ -206,8 +202,6 @@ __global__ __launch_bounds__(kTkThreads) void topk_hist_kernel(const typename So
   __syncthreads();
   const int hs = 8 * (r + 1);  // bits above digit r
   const uint32_t want = hs >= KT::kBits ? 0u : (uint32_t)(state[0] >> hs);
-  const int64_t c0 = (int64_t)blockIdx.x * chunk;
-  const int64_t c1 = c0 + chunk < n ? c0 + chunk : n;
   auto count = [&](const Raw (&v)[V]) {
 #pragma unroll
     for (int i = 0; i < V; ++i) {
@@ -253,53 +247,65 @@ __global__ __launch_bounds__(kTkThreads) void topk_hist_kernel(const typename So
     if (above != 0) atomicAdd(&s_am[lt], above << 16);
     if (subm != 0) atomicOr(&s_sub[lt], subm);
   };
-  int64_t b0 = c0 + (int64_t)tid * V;
-  const int64_t full_end = c0 + ((c1 - c0) / (U * STEP)) * (U * STEP);  // steps [c0, full_end) are whole
-  // Behind a gate a wave leaves out the steps whose sub-chunks all lie below
-  // the bound: no key there is selected, and the digits chosen count only
-  // keys at or above the k-th.  2^28 sorted fp16 keys (few sub-chunks hold
-  // them all): 615 us without, 378 with it and with groups
-  // of sub-chunks that lie apart.
+  // Whole steps of this workgroup: step0, step0 + stride, ..., nst of them,
+  // and a last one that is not whole where `end` cuts it.  Without a gate a
+  // range of its own.  Behind one, steps that lie apart: a wave leaves out
+  // those whose sub-chunks all lie below the bound (no key there is selected,
+  // and the digits chosen count only keys at or above the k-th), and the
+  // rest may lie together.
+  constexpr int64_t SPAN = U * STEP;
+  const int64_t step0 = gate ? (int64_t)blockIdx.x * SPAN : (int64_t)blockIdx.x * chunk;
+  const int64_t stride = gate ? (int64_t)gridDim.x * SPAN : SPAN;
+  const int64_t end = gate || step0 + chunk > n ? n : step0 + chunk;
+  const int nst = end - step0 >= SPAN ? (int)((end - step0 - SPAN) / stride) + 1 : 0;
   const uint32_t bound = gate ? gate[1] : 0u;
   const int64_t wave0 = (int64_t)__builtin_amdgcn_readfirstlane(wid) * (kWave * V);
-  auto below = [&](int64_t step0) {
-    uint32_t m = 0;
+  for (int j0 = 0; j0 < nst; j0 += kWave) {
+    uint64_t todo = nst - j0 < kWave ? (1ull << (nst - j0)) - 1ull : ~0ull;
+    if (gate) {
+      // Lane l looks at step j0 + l.
+      const int j = j0 + (int)__lane_id();
+      uint32_t m = 0;
+      if (j < nst) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t q = submax[(step0 + u * STEP + wave0) >> sub_shift];
-      m = m > q ? m : q;
+        for (int u = 0; u < U; ++u) {
+          const uint32_t q = submax[(step0 + j * stride + u * STEP + wave0) >> sub_shift];
+          m = m > q ? m : q;
+        }
+      }
+      todo &= __ballot(m >= bound);
     }
-    return m < bound;
-  };
-  int64_t step0 = c0;
-  bool next_below = gate && c0 < full_end && below(c0);
-  for (; b0 < full_end; b0 += U * STEP) {
-    const bool skip = next_below;
-    step0 += U * STEP;
-    if (gate && step0 < full_end) next_below = below(step0);
-    if (skip) continue;
-    Raw v[U][V];
+    while (todo != 0) {
+      // In a vector register: for a uniform tile the compiler would join the
+      // lanes' LDS adds one lane at a time.
+      int j = j0 + __builtin_ctzll(todo);
+      asm volatile("" : "+v"(j));
+      todo &= todo - 1;
+      const int64_t b0 = step0 + j * stride + (int64_t)tid * V;
+      Raw v[U][V];
 #pragma unroll
-    for (int u = 0; u < U; ++u) load_items<Raw, V, true>(x, b0 + u * STEP, c1, v[u]);
-    if constexpr (FUSE) {
-      // Chunks are whole tiles and one step is one tile.
-      count_record(v, (int)((b0 - c0) / TILE), (b0 - c0) % TILE, [](int, int) { return true; });
-    } else {
+      for (int u = 0; u < U; ++u) load_items<Raw, V, true>(x, b0 + u * STEP, end, v[u]);
+      if constexpr (FUSE) {
+        count_record(v, j, (int64_t)tid * V, [](int, int) { return true; });
+      } else {
 #pragma unroll
-      for (int u = 0; u < U; ++u) count(v[u]);
+        for (int u = 0; u < U; ++u) count(v[u]);
+      }
     }
   }
-  for (; b0 < c1; b0 += STEP) {
+  const int64_t last = step0 + nst * stride;
+  int tail = nst;
+  asm volatile("" : "+v"(tail));
+  for (int64_t b0 = last + (int64_t)tid * V; b0 < end; b0 += STEP) {
     Raw v[1][V];
-    load_items<Raw, V, false>(x, b0, c1, v[0]);
+    load_items<Raw, V, false>(x, b0, end, v[0]);
     if constexpr (FUSE) {
-      // [full_end, c1) is less than one tile: the chunk's last.
-      count_record(v, (int)((full_end - c0) / TILE), b0 - full_end, [&](int, int i) { return b0 + i < c1; });
+      count_record(v, tail, b0 - last, [&](int, int i) { return b0 + i < end; });
     } else {
 #pragma unroll
       for (int i = 0; i < V; ++i) {
         const uint32_t k = KT::key(v[0][i]) ^ flip;
-        const bool match = b0 + i < c1 && (hs >= KT::kBits || (k >> hs) == want);
+        const bool match = b0 + i < end && (hs >= KT::kBits || (k >> hs) == want);
         if (match) atomicAdd(&h[hc][(k >> (8 * r)) & 0xffu], 1u);
       }
     }
@@ -309,20 +315,33 @@ __global__ __launch_bounds__(kTkThreads) void topk_hist_kernel(const typename So
     uint32_t s = 0;
 #pragma unroll
     for (int w = 0; w < NH; ++w) s += h[w][e];
-    topk_leave(&partial[(size_t)blockIdx.x * 256 + e], s, gate != nullptr);
+    if (!gate) {
+      partial[(size_t)blockIdx.x * 256 + e] = s;
+    } else if (s != 0) {
+      __hip_atomic_fetch_add(&bins[e], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
   if constexpr (FUSE) {
-    const int64_t t0 = c0 / TILE;
-    const int ntl = c1 > c0 ? (int)((c1 - c0 + TILE - 1) / TILE) : 0;
+    const int64_t tile0 = step0 / TILE, apart = stride / TILE;
+    const int ntl = end > step0 ? (int)((end - step0 + stride - 1) / stride) : 0;
     for (int e = tid; e < ntl; e += kTkThreads) {
       const uint32_t am = s_am[e];
-      tstat[t0 + e] = ((uint64_t)(am >> 16) << 32) | (s_sub[e] << 16) | (am & 0xffffu);
+      tstat[tile0 + e * apart] = ((uint64_t)(am >> 16) << 32) | (s_sub[e] << 16) | (am & 0xffffu);
     }
     for (int e = tid; e < ntl * kTkListMax; e += kTkThreads)
-      tlist[t0 * kTkListMax + e] = s_list[e / kTkListMax][e % kTkListMax];
+      tlist[(tile0 + e / kTkListMax * apart) * kTkListMax + e % kTkListMax] = s_list[e / kTkListMax][e % kTkListMax];
   }
-  // Behind a gate the last workgroup picks the digit.
-  if (gate && topk_last_arrival(arrived)) topk_pick<kTkThreads, true>(partial, gridDim.x, r, hs >= KT::kBits, k_all, state);
+  // Behind a gate the last workgroup picks the digit and leaves the bins zero
+  // for the next launch.
+  if (gate && topk_last_arrival(arrived)) {
+    auto sum = [&](int d, int q, int) {
+      if (q != 0) return 0u;
+      const uint32_t c = __hip_atomic_load(&bins[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&bins[d], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return c;
+    };
+    topk_pick<kTkThreads>(sum, r, hs >= KT::kBits, k_all, state);
+  }
 }
 
 // First level of the digit-count sum: workgroup q adds the partials of
@@ -350,7 +369,20 @@ __global__ __launch_bounds__(256) void topk_sum_kernel(const uint64_t* __restric
 __global__ __launch_bounds__(kTkPickThreads) void topk_pick_kernel(const uint64_t* __restrict__ partial,
                                                                    int groups, int r, int first, int64_t k,
                                                                    uint64_t* __restrict__ state) {
-  topk_pick<kTkPickThreads, false>(partial, groups, r, first, k, state);
+  auto count = [&](int d, int q, int nq) {
+    uint32_t s = 0;
+    int g = q;
+    for (; g + 7 * nq < groups; g += 8 * nq) {  // eight loads in flight
+      uint64_t v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = partial[(size_t)(g + nq * u) * 256 + d];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += (uint32_t)v[u];
+    }
+    for (; g < groups; g += nq) s += (uint32_t)partial[(size_t)g * 256 + d];
+    return s;
+  };
+  topk_pick<kTkPickThreads>(count, r, first, k, state);
 }
 
 // ---------------------------------------------------------------------------
@@ -455,33 +487,47 @@ __device__ __forceinline__ void topk_tilescan(uint64_t* tcnt, uint32_t tiles) {
   if (tid == 0) tcnt[tiles] = (uint64_t)carry;
 }
 
-// tcnt[tile] = (keys above T) << 32 | (keys equal to T) in the tile.
+// tcnt[tile] = (keys above T) << 32 | (keys equal to T) in the tile.  Behind
+// a gate, tiles whose sub-chunks all lie below the bound are not read.
 template <int DT>
 __global__ __launch_bounds__(kTkNW * kWave) void topk_tilecount_kernel(
     const typename SortKey<DT>::Raw* __restrict__ x, int64_t n, uint32_t flip,
-    const uint64_t* __restrict__ state, uint64_t* tcnt, const uint32_t* __restrict__ gate,
-    uint32_t* __restrict__ arrived) {
+    const uint64_t* __restrict__ state, uint64_t* tcnt, uint32_t tiles, const uint32_t* __restrict__ gate,
+    uint32_t* __restrict__ arrived, const uint32_t* __restrict__ submax, int sub_shift) {
   constexpr int J = TopkGeom<DT>::J, NW = kTkNW;
+  constexpr int64_t TILE = TopkGeom<DT>::kTile;
   if (topk_done(gate)) return;
   __shared__ int s_w[NW];
   const int lane = __lane_id(), wid = threadIdx.x / kWave;
-  Packed<typename SortKey<DT>::Raw, kTkG> xv[J];
-  uint32_t gtb[J], eqb[J];
-  topk_classify_any<DT>(x, n, flip, (uint32_t)state[0], blockIdx.x, wid, lane, xv, gtb, eqb);
-  int c = 0;
+  const uint32_t bound = gate ? gate[1] : 0u;
+  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    if (gate) {
+      const int64_t p = (int64_t)tile * TILE + ((int64_t)lane << sub_shift);
+      const bool in = ((int64_t)lane << sub_shift) < TILE && p < n;
+      if (__ballot(in && submax[in ? p >> sub_shift : 0] >= bound) == 0) {
+        if (threadIdx.x == 0) topk_leave(&tcnt[tile], 0, true);
+        continue;
+      }
+    }
+    Packed<typename SortKey<DT>::Raw, kTkG> xv[J];
+    uint32_t gtb[J], eqb[J];
+    topk_classify_any<DT>(x, n, flip, (uint32_t)state[0], tile, wid, lane, xv, gtb, eqb);
+    int c = 0;
 #pragma unroll
-  for (int j = 0; j < J; ++j) c += (__builtin_popcount(gtb[j]) << 16) | __builtin_popcount(eqb[j]);
-  c = wave_sum(c);
-  if (lane == 0) s_w[wid] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int t = 0;
+    for (int j = 0; j < J; ++j) c += (__builtin_popcount(gtb[j]) << 16) | __builtin_popcount(eqb[j]);
+    c = wave_sum(c);
+    __syncthreads();  // s_w of the tile before has been read
+    if (lane == 0) s_w[wid] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int t = 0;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) t += s_w[w];
-    topk_leave(&tcnt[blockIdx.x], ((uint64_t)((uint32_t)t >> 16) << 32) | ((uint32_t)t & 0xffffu), gate != nullptr);
+      for (int w = 0; w < NW; ++w) t += s_w[w];
+      topk_leave(&tcnt[tile], ((uint64_t)((uint32_t)t >> 16) << 32) | ((uint32_t)t & 0xffffu), gate != nullptr);
+    }
   }
   // Behind a gate the last workgroup scans the counts.
-  if (gate && topk_last_arrival(arrived)) topk_tilescan<kTkNW * kWave, true>(tcnt, gridDim.x);
+  if (gate && topk_last_arrival(arrived)) topk_tilescan<kTkNW * kWave, true>(tcnt, tiles);
 }
 
 // tcnt[tile] as topk_tilecount_kernel writes it, from the record of the
@@ -489,8 +535,10 @@ __global__ __launch_bounds__(kTkNW * kWave) void topk_tilecount_kernel(
 // T's plus the recorded matching keys whose low byte is above T's, keys
 // equal to T the recorded ones with T's low byte.  A tile with more matching
 // keys than were recorded is counted from its keys.  One wave per tile.
-template <int DT>
-__global__ __launch_bounds__(256) void topk_tilefix_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
+// Workgroups of 256 threads spread the tiles that are read; behind a gate few
+// are, and 1024 threads mean few arrivals and a quick scan.
+template <int DT, int NT>
+__global__ __launch_bounds__(NT) void topk_tilefix_kernel(const typename SortKey<DT>::Raw* __restrict__ x,
                                                            int64_t n, uint32_t flip,
                                                            const uint64_t* __restrict__ state,
                                                            const uint64_t* __restrict__ tstat,
@@ -504,7 +552,7 @@ __global__ __launch_bounds__(256) void topk_tilefix_kernel(const typename SortKe
   constexpr int64_t TILE = TopkGeom<DT>::kTile;
   constexpr int V = 16 / (int)sizeof(Raw);
   const int lane = __lane_id();
-  const uint32_t tile = blockIdx.x * (256 / kWave) + threadIdx.x / kWave;
+  const uint32_t tile = blockIdx.x * (NT / kWave) + threadIdx.x / kWave;
   if (tile < tiles) {
     const uint32_t T = (uint32_t)state[0];
     const uint64_t rec = tstat[tile];
@@ -519,16 +567,29 @@ __global__ __launch_bounds__(256) void topk_tilefix_kernel(const typename SortKe
       const int64_t t0 = (int64_t)tile * TILE;
       const int64_t t1 = t0 + TILE < n ? t0 + TILE : n;
       uint32_t gl = 0, el = 0;
-      for (int64_t b = t0 + (int64_t)lane * V; b < t1; b += (int64_t)kWave * V) {
-        Raw v[V];
-        load_items<Raw, V>(x, b, t1, v);
-  #pragma unroll
+      auto add = [&](const auto& v, int64_t b) {
+#pragma unroll
         for (int i = 0; i < V; ++i) {
           const uint32_t kk = KT::key(v[i]) ^ flip;
           const bool ok = b + i < t1;
           gl += ok && kk > T ? 1u : 0u;
           el += ok && kk == T ? 1u : 0u;
         }
+      };
+      // Four loads in flight: a wave reads the tile by itself.
+      constexpr int F = 4;
+      int64_t b = t0 + (int64_t)lane * V;
+      for (; t0 + TILE <= n && b < t1; b += F * kWave * V) {
+        Raw v[F][V];
+#pragma unroll
+        for (int f = 0; f < F; ++f) load_items<Raw, V, true>(x, b + f * (kWave * V), t1, v[f]);
+#pragma unroll
+        for (int f = 0; f < F; ++f) add(v[f], b + f * (kWave * V));
+      }
+      for (; b < t1; b += (int64_t)kWave * V) {
+        Raw v[V];
+        load_items<Raw, V>(x, b, t1, v);
+        add(v, b);
       }
       g = (uint32_t)wave_sum((int)gl);
       e = (uint32_t)wave_sum((int)el);
@@ -536,7 +597,7 @@ __global__ __launch_bounds__(256) void topk_tilefix_kernel(const typename SortKe
     if (lane == 0) topk_leave(&tcnt[tile], ((uint64_t)g << 32) | e, gate != nullptr);
   }
   // Behind a gate the last workgroup scans the counts.
-  if (gate && topk_last_arrival(arrived)) topk_tilescan<256, true>(tcnt, tiles);
+  if (gate && topk_last_arrival(arrived)) topk_tilescan<NT, true>(tcnt, tiles);
 }
 
 __global__ __launch_bounds__(kTkScanThreads) void topk_tilescan_kernel(uint64_t* __restrict__ tcnt,
@@ -775,8 +836,12 @@ __global__ __launch_bounds__(kTkMaxThreads) void topk_max_kernel(const typename 
   constexpr int V = TopkSub<DT, U>::V;
   constexpr int64_t SUB = TopkSub<DT, U>::kKeys;
   const int lane = __lane_id();
-  // Candidates, counted by the gather kernel, and the gated arrivals.
-  if (blockIdx.x == 0 && threadIdx.x == 0) state[0] = state[8] = 0;
+  // Candidates, counted by the gather kernel, and the gated launches' words.
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) state[0] = state[kTkArrived] = 0;
+    static_assert(kTkMaxThreads == 256, "one bin a thread");
+    state[kTkBins + threadIdx.x] = 0;
+  }
   const uint32_t g = blockIdx.x * (kTkMaxThreads / kWave) + threadIdx.x / kWave;
   if (g >= groups) return;
   uint32_t mine = 0, best = 0, at = g;
@@ -1268,7 +1333,7 @@ inline TopkLayout topk_layout(int64_t n, int64_t k, int dt, size_t avail = SIZE_
   L.submax_off = align256(L.word_off + (size_t)kTkCandMax * 8);
   L.gcomp_off = align256(L.submax_off + (size_t)L.mx.subs * 4);
   L.mstate_off = align256(L.gcomp_off + (size_t)L.mx.groups * 8);
-  L.scratch = L.mstate_off + 256;
+  L.scratch = L.mstate_off + kTkStateWords * sizeof(uint32_t);
   L.least = L.sort_scratch_off + tcs_sort_scratch_bytes(k, dt);
   if (L.scratch > avail) {
     L.path = TopkPath::kSelect;
@@ -1288,8 +1353,10 @@ static int topk_select(const typename SortKey<DT>::Raw* xr, int64_t n, int64_t k
   auto* state = reinterpret_cast<uint64_t*>(w + L.state_off);
   auto* partial = reinterpret_cast<uint64_t*>(w + L.part_off);
   auto* psum = reinterpret_cast<uint64_t*>(w + L.psum_off);
-  // Arrivals of the gated launches, zeroed with the gate by the maxima pass.
-  uint32_t* arrived = gate ? gate + 8 : nullptr;
+  // Arrivals and digit counts of the gated launches, zeroed with the gate by
+  // the maxima pass.
+  uint32_t* arrived = gate ? gate + kTkArrived : nullptr;
+  uint32_t* bins = gate ? gate + kTkBins : nullptr;
   const auto* submax = reinterpret_cast<const uint32_t*>(sc + L.submax_off);
   const int sub_shift = __builtin_ctz(L.mx.U * kWave * (16 / (int)sizeof(Raw)));
   const int sum_per = (L.groups + kTkSumGroups - 1) / kTkSumGroups;
@@ -1301,13 +1368,17 @@ static int topk_select(const typename SortKey<DT>::Raw* xr, int64_t n, int64_t k
   auto* tstat = reinterpret_cast<uint64_t*>(sc + L.tstat_off);
   auto* tlist = reinterpret_cast<uint8_t*>(sc + L.tlist_off);
   constexpr bool kFuse = P > 1;  // keys of one byte: the tile counts read the keys
+  // Few arrivals behind a gate, and at most kTkMaxChunkTiles tiles a workgroup.
+  const uint32_t most = (tiles + kTkMaxChunkTiles - 1) / kTkMaxChunkTiles;
+  const uint32_t few = most > kTkGatedGroups ? most : kTkGatedGroups;
+  const uint32_t groups = gate && few < (uint32_t)L.groups ? few : (uint32_t)L.groups;
   for (int r = P - 1; r >= 0; --r) {
     if (kFuse && r == 0) {
-      hipLaunchKernelGGL((topk_hist_kernel<DT, kFuse>), dim3(L.groups), dim3(kTkThreads), 0, st, xr, n, L.chunk,
-                         flip, r, k, state, partial, tstat, tlist, gate, arrived, submax, sub_shift);
+      hipLaunchKernelGGL((topk_hist_kernel<DT, kFuse>), dim3(groups), dim3(kTkThreads), 0, st, xr, n, L.chunk,
+                         flip, r, k, state, partial, tstat, tlist, gate, arrived, bins, submax, sub_shift);
     } else {
-      hipLaunchKernelGGL((topk_hist_kernel<DT, false>), dim3(L.groups), dim3(kTkThreads), 0, st, xr, n, L.chunk,
-                         flip, r, k, state, partial, nullptr, nullptr, gate, arrived, submax, sub_shift);
+      hipLaunchKernelGGL((topk_hist_kernel<DT, false>), dim3(groups), dim3(kTkThreads), 0, st, xr, n, L.chunk,
+                         flip, r, k, state, partial, nullptr, nullptr, gate, arrived, bins, submax, sub_shift);
     }
     TCS_CHECK_LAUNCH();
     if (!gate) {
@@ -1319,11 +1390,17 @@ static int topk_select(const typename SortKey<DT>::Raw* xr, int64_t n, int64_t k
     }
   }
   if constexpr (kFuse) {
-    hipLaunchKernelGGL((topk_tilefix_kernel<DT>), dim3((tiles + 3) / 4), dim3(256), 0, st, xr, n, flip, state, tstat,
-                       tlist, tcnt, tiles, gate, arrived);
+    if (gate) {
+      hipLaunchKernelGGL((topk_tilefix_kernel<DT, 1024>), dim3((tiles + 15) / 16), dim3(1024), 0, st, xr, n, flip, state,
+                         tstat, tlist, tcnt, tiles, gate, arrived);
+    } else {
+      hipLaunchKernelGGL((topk_tilefix_kernel<DT, 256>), dim3((tiles + 3) / 4), dim3(256), 0, st, xr, n, flip, state,
+                         tstat, tlist, tcnt, tiles, gate, arrived);
+    }
   } else {
-    hipLaunchKernelGGL((topk_tilecount_kernel<DT>), dim3(tiles), dim3(kTkNW * kWave), 0, st, xr, n, flip, state,
-                       tcnt, gate, arrived);
+    const uint32_t grid = gate && tiles > kTkGatedGroups ? kTkGatedGroups : tiles;
+    hipLaunchKernelGGL((topk_tilecount_kernel<DT>), dim3(grid), dim3(kTkNW * kWave), 0, st, xr, n, flip, state, tcnt,
+                       tiles, gate, arrived, submax, sub_shift);
   }
   TCS_CHECK_LAUNCH();
   if (!gate) {
