@@ -562,14 +562,13 @@ inline int sort_passes(int dt) {
 
 inline int sort_elem_bytes(int dt) { return dt == TCS_I8 ? 1 : (sort_passes(dt) == 2 ? 2 : 4); }
 
-// Above this many keys the scatter workgroups take 16 waves, and 16384 or
+// Above kSortWideMin keys the scatter workgroups take 16 waves, and 16384 or
 // 32768 keys a tile (the LDS of a whole compute unit), one workgroup on each:
 // a tile's runs are then twice or four times as long, and fewer of the lines
 // that the 256 runs write are left partial between tiles.  Below it 8-wave
 // workgroups with 4096-key tiles, two to a compute unit, divide the keys more
 // evenly (fp16 keys, 4e6: 46 against 53 us, 5e6: 56 against 61, 8e6: 73
 // either way; int32, 4e6: 101 against 106, 8e6: 176 against 161).
-constexpr int64_t kSortWideMin = (int64_t)6 << 20;
 inline SortLayout sort_layout(int64_t n, int dt) {
   SortLayout L{};
   L.wide = n > kSortWideMin;

@@ -330,7 +330,8 @@ int seg_scan_flags_cfg(const void* x, int x_dtype, const int8_t* flags, void* y,
                        void* stream);
 
 // The first k of the stable sort of x (sort.hip), with scratch of
-// sort_first_scratch_bytes.
+// sort_first_scratch_bytes; k < n up to kSortWideMin keys only.
+constexpr int64_t kSortWideMin = (int64_t)6 << 20;
 int sort_first(const void* x, int dtype, void* out_x, int32_t* out_idx, int64_t n, int64_t k, bool descending,
                void* scratch, hipStream_t st);
 size_t sort_first_scratch_bytes(int64_t n, int dtype);

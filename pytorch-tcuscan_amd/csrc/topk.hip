@@ -1253,8 +1253,15 @@ inline int topk_elem_bytes(int dt) {
   }
 }
 
-// Sub-chunks of one vector (U = 1) up to 2^17 of them, of four above; groups
-// of `per` sub-chunks, 4096 of them or as many as leave the bound tight.
+// Sub-chunks of one vector (U = 1) up to 2^17 of them, of four above; 4096
+// groups (enough waves for the read) or four times the winners, which leave
+// the bound tight, and more where a group would take over 64 sub-chunks.
+// Fewer, of equal size, where those are enough for the winners (the bound
+// looks at every group: 9e6 fp32 keys, k = 3000, 67 us with 11719 groups, 78
+// with 16384).  Otherwise groups differ by one sub-chunk, as many at every
+// size: just above a multiple of them equal ones would be half as many, too
+// few for the bound (9e6 fp16 keys, k = 3000: 58 us, 88 by the select).
+constexpr int64_t kTkGroupsPerK = 3;
 struct TopkMaxima {
   int U, per;
   uint32_t subs, groups;
@@ -1265,11 +1272,12 @@ inline TopkMaxima topk_maxima(int64_t n, int64_t k, int key_bytes) {
   const int64_t vec = kWave * (16 / key_bytes);
   m.U = n > vec << 17 ? 4 : 1;
   m.subs = (uint32_t)((n + m.U * vec - 1) / (m.U * vec));
-  int64_t most = 4096;  // enough waves for the read, four times the winners
-  while (most < 4 * k && most < kTkMaxGroupsM) most *= 2;
-  m.per = (int)((m.subs + most - 1) / most);
-  if (m.per < 1) m.per = 1;
-  m.groups = (m.subs + m.per - 1) / m.per;
+  int64_t most = 4096;
+  while (most < kTkMaxGroupsM && (most < 4 * k || m.subs > most * kWave)) most *= 2;
+  m.groups = m.subs < most ? m.subs : (uint32_t)most;
+  m.per = m.groups > 0 ? (int)((m.subs + m.groups - 1) / m.groups) : 1;
+  const int64_t even = (m.subs + m.per - 1) / m.per;
+  if (even >= kTkGroupsPerK * k) m.groups = (uint32_t)even;
   return m;
 }
 
@@ -1277,14 +1285,14 @@ enum class TopkPath { kSort, kMaxima, kSelect };
 
 // The sort while its passes cost less than the maxima path's launches; the
 // maxima path where it has groups enough for its bound to be tight (three
-// times as many as winners: about 1.2 k candidates); the sort again up to
-// 2^21 or 2^22 more keys than that; the radix select beyond.  fp16, k = 300:
-// 2^21 keys 31 us sorted, 30 by maxima; k = 3000, 4e6 keys: 45 us sorted, the
-// select 114; fp32, k = 300: 5e5 keys 51 us sorted, 1e6 by maxima 44.
+// times as many as winners: about 1.2 k candidates); where it has not, the
+// sort up to kSortWideMin 16-bit keys, and the radix select beyond.  fp16, k =
+// 300: 2^21 keys 31 us sorted, 30 by maxima; k = 3000, 4e6 keys: 45 us sorted,
+// the select 114; fp32, k = 300: 5e5 keys 51 us sorted, 1e6 by maxima 44.
 inline TopkPath topk_path(const TopkMaxima& m, int64_t n, int64_t k, int key_bytes) {
   if (n <= (key_bytes <= 2 ? (int64_t)1 << 21 : (int64_t)1 << 18)) return TopkPath::kSort;
-  if (k <= kTkRankMax && (int64_t)m.groups >= 3 * k && m.per <= kWave) return TopkPath::kMaxima;
-  return n <= (key_bytes <= 2 ? (int64_t)6 << 20 : (int64_t)3 << 20) ? TopkPath::kSort : TopkPath::kSelect;
+  if (k <= kTkRankMax && (int64_t)m.groups >= kTkGroupsPerK * k && m.per <= kWave) return TopkPath::kMaxima;
+  return n <= (key_bytes <= 2 ? kSortWideMin : kSortWideMin / 2) ? TopkPath::kSort : TopkPath::kSelect;
 }
 
 struct TopkLayout {
