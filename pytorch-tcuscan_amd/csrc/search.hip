@@ -76,6 +76,7 @@ __device__ __forceinline__ int32_t lower_bound_in(const int32_t* __restrict__ so
 // samples.  2^24 needles into 2^14 elements: 40.7 us (4.1e11 needles a
 // second; bound by the steps' LDS reads), 187 with one needle a thread at a
 // time and a sorted array of samples.
+template <int U>
 __device__ __forceinline__ void search_staged(int32_t* s_tree, const int32_t* __restrict__ sorted, int32_t len,
                                               const int32_t* __restrict__ values, int32_t* __restrict__ out,
                                               int64_t nv) {
@@ -91,13 +92,13 @@ __device__ __forceinline__ void search_staged(int32_t* s_tree, const int32_t* __
   const int32_t first = sorted[0];
   __syncthreads();
   const int64_t stride = (int64_t)gridDim.x * kSsThreads;
-  for (int64_t i = (int64_t)blockIdx.x * kSsThreads + threadIdx.x; i < nv; i += kSsU * stride) {
-    int32_t key[kSsU], c[kSsU];
+  for (int64_t i = (int64_t)blockIdx.x * kSsThreads + threadIdx.x; i < nv; i += U * stride) {
+    int32_t key[U], c[U];
 #pragma unroll
-    for (int u = 0; u < kSsU; ++u) key[u] = values[i + u * stride < nv ? i + u * stride : nv - 1];
-    tree_count<kSsU>(s_tree, log, key, c);
+    for (int u = 0; u < U; ++u) key[u] = values[i + u * stride < nv ? i + u * stride : nv - 1];
+    tree_count<U>(s_tree, log, key, c);
 #pragma unroll
-    for (int u = 0; u < kSsU; ++u) {
+    for (int u = 0; u < U; ++u) {
       c[u] += first < key[u] ? 1 : 0;
       int32_t lo = c[u];
       if (B > 1 && lo > 0) {
@@ -111,11 +112,13 @@ __device__ __forceinline__ void search_staged(int32_t* s_tree, const int32_t* __
   }
 }
 
+// U needles of a thread in flight.
+template <int U>
 __global__ __launch_bounds__(kSsThreads) void searchsorted_kernel(const int32_t* __restrict__ sorted, int32_t len,
                                                                   const int32_t* __restrict__ values,
                                                                   int32_t* __restrict__ out, int64_t nv) {
   __shared__ int32_t s_tree[kSsNodes];
-  search_staged(s_tree, sorted, len, values, out, nv);
+  search_staged<U>(s_tree, sorted, len, values, out, nv);
 }
 
 // ---------------------------------------------------------------------------
@@ -363,7 +366,7 @@ __global__ __launch_bounds__(kSsThreads) void searchsorted_indexed_kernel(const 
   const int64_t first = (int64_t)blockIdx.x * kSsThreads + threadIdx.x;
   if (bucket_clustered(wide, len, m, s_tree)) {
     __syncthreads();  // the sum has been read
-    search_staged(s_tree, sorted, len, values, out, nv);
+    search_staged<kSsU>(s_tree, sorted, len, values, out, nv);
     return;
   }
   for (int64_t i = first; i < nv; i += stride * kSsU) {
@@ -760,13 +763,16 @@ int tcs_searchsorted(const int32_t* sorted, int64_t sorted_len, const int32_t* v
   }
   // A workgroup for each CU first, then kSsU needles a thread before more of
   // them stage the samples (2^20 needles into 2^14: 16.4 us with one needle a
-  // thread, 7.4 with four).
+  // thread, 7.4 with four).  While no thread has more than one needle, one in
+  // flight: the steps of three copies of it would be LDS reads as well (2^18
+  // needles into 2^14: 7.1 us with four, 5.9 with one; 2^19 7.1 and 7.9).
   const uint64_t cap = searchsorted_grid();
   const uint64_t rows = (uint64_t)((num_values + kSsThreads - 1) / kSsThreads);
   const uint64_t few = rows < cap / 4 ? rows : cap / 4, need = (rows + kSsU - 1) / kSsU;
   const uint32_t blocks = (uint32_t)(need < few ? few : (need < cap ? need : cap));
-  hipLaunchKernelGGL(searchsorted_kernel, dim3(blocks), dim3(kSsThreads), 0, static_cast<hipStream_t>(stream),
-                     sorted, (int32_t)sorted_len, values, out, num_values);
+  hipLaunchKernelGGL(blocks == rows ? searchsorted_kernel<1> : searchsorted_kernel<kSsU>, dim3(blocks),
+                     dim3(kSsThreads), 0, static_cast<hipStream_t>(stream), sorted, (int32_t)sorted_len, values, out,
+                     num_values);
   TCS_CHECK_LAUNCH();
   return TCS_OK;
 }

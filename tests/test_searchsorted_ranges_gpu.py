@@ -78,3 +78,15 @@ def test_unsorted_haystacks_stay_in_range(lib, ops, dev, n, order):
             if order == "sorted":
                 assert torch.equal(out, torch.searchsorted(hay, v, out_int32=True))
         assert torch.equal(ops.run_searchsorted(good, v), torch.searchsorted(good, v, out_int32=True))
+
+
+@pytest.mark.parametrize("n", [1, 2, 100, 16384, 16385, 65536])
+@pytest.mark.parametrize("m", [(1 << 16) + 1, 1 << 18, (1 << 18) + 1])
+def test_one_needle_a_thread(ops, dev, n, m):
+    """The sampled search with one needle a thread, up to 2^18 of them, and
+    with four above."""
+    g = torch.Generator(device=dev).manual_seed(n)
+    hay = torch.randint(I32_MIN, I32_MAX, (n,), generator=g, device=dev, dtype=torch.int32).sort().values
+    v = torch.randint(I32_MIN, I32_MAX, (m,), generator=g, device=dev, dtype=torch.int32)
+    v[: m // 2] = hay[torch.randint(0, n, (m // 2,), generator=g, device=dev)]
+    assert torch.equal(ops.run_searchsorted(hay, v), torch.searchsorted(hay, v, out_int32=True))
