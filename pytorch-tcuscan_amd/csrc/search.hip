@@ -733,15 +733,22 @@ static bool searchsorted_few(int64_t len, int64_t nv) {
   return nv <= (mid ? (int64_t)1 << 15 : (int64_t)1 << 16);
 }
 
-// Four workgroups per CU of the current device (two are resident at a
-// time with 64 KiB of LDS each; the second pair evens out the tail).
-static uint32_t searchsorted_grid() {
+// Workgroups for `rows` rows of kSsThreads needles: one for each CU of the
+// current device first, then kSsU needles a thread before more of them, up to
+// the two a CU that are resident with 64 KiB of LDS each, since every workgroup
+// of the sampled search stages the samples (2^20 needles into 2^14 elements:
+// 16.4 us with one needle a thread, 7.4 with four; 2^20 into 2^20 clustered
+// elements, by the table's sampled search: 99 and 49; 2^24 into 2^18: 297 us
+// with four workgroups a CU, 283 with two).
+static uint32_t searchsorted_grid(uint64_t rows) {
   static std::atomic<int> cached[kMaxCachedDevices];
-  return (uint32_t)device_cached(cached, [](int dev) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
-    return 4 * cus;
+  const uint64_t cus = (uint64_t)device_cached(cached, [](int dev) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+    return n;
   });
+  const uint64_t few = rows < cus ? rows : cus, need = (rows + kSsU - 1) / kSsU;
+  return (uint32_t)(need < few ? few : (need < 2 * cus ? need : 2 * cus));
 }
 
 }  // namespace tcs
@@ -761,15 +768,11 @@ int tcs_searchsorted(const int32_t* sorted, int64_t sorted_len, const int32_t* v
     TCS_CHECK_LAUNCH();
     return TCS_OK;
   }
-  // A workgroup for each CU first, then kSsU needles a thread before more of
-  // them stage the samples (2^20 needles into 2^14: 16.4 us with one needle a
-  // thread, 7.4 with four).  While no thread has more than one needle, one in
-  // flight: the steps of three copies of it would be LDS reads as well (2^18
-  // needles into 2^14: 7.1 us with four, 5.9 with one; 2^19 7.1 and 7.9).
-  const uint64_t cap = searchsorted_grid();
+  // While no thread has more than one needle, one in flight: the steps of
+  // three copies of it would be LDS reads as well (2^18 needles into 2^14: 7.1
+  // us with four, 5.9 with one; 2^19 7.1 and 7.9).
   const uint64_t rows = (uint64_t)((num_values + kSsThreads - 1) / kSsThreads);
-  const uint64_t few = rows < cap / 4 ? rows : cap / 4, need = (rows + kSsU - 1) / kSsU;
-  const uint32_t blocks = (uint32_t)(need < few ? few : (need < cap ? need : cap));
+  const uint32_t blocks = searchsorted_grid(rows);
   hipLaunchKernelGGL(blocks == rows ? searchsorted_kernel<1> : searchsorted_kernel<kSsU>, dim3(blocks),
                      dim3(kSsThreads), 0, static_cast<hipStream_t>(stream), sorted, (int32_t)sorted_len, values, out,
                      num_values);
@@ -861,9 +864,8 @@ int tcs_searchsorted_indexed(const int32_t* sorted, int64_t sorted_len, const in
   hipLaunchKernelGGL(bucket_start_kernel, dim3(kSsBuildBlocks), dim3(kSsThreads), 0, st, sorted, len, per_block, bits,
                      wide, start);
   TCS_CHECK_LAUNCH();
-  const uint64_t cap = searchsorted_grid();
-  const uint64_t need = (uint64_t)((num_values + kSsThreads - 1) / kSsThreads);
-  hipLaunchKernelGGL(searchsorted_indexed_kernel, dim3((uint32_t)(need < cap ? need : cap)), dim3(kSsThreads), 0, st,
+  hipLaunchKernelGGL(searchsorted_indexed_kernel,
+                     dim3(searchsorted_grid((uint64_t)((num_values + kSsThreads - 1) / kSsThreads))), dim3(kSsThreads), 0, st,
                      sorted, len, bits, wide, start, values, out, num_values);
   TCS_CHECK_LAUNCH();
   return TCS_OK;
