@@ -467,8 +467,8 @@ size_t tcs_searchsorted_workspace_bytes(int64_t sorted_len);
 /* Workspace bytes with which it is fastest for num_values needles: 512 counts
  * and a table of 2^b + 1 int32, b = clamp(floor(log2(len)) - 2, 10, 22) (at
  * most 16 MiB + 2052 bytes); at most 43 MiB where the needles are many
- * (below).  Any size
- * from the least up is taken. */
+ * (below); the least where it takes no workspace.  Any size from the least up
+ * is taken. */
 size_t tcs_searchsorted_preferred_bytes(int64_t sorted_len, int64_t num_values);
 
 /* tcs_searchsorted with a bucket index built in `workspace` first (no host
@@ -477,9 +477,10 @@ size_t tcs_searchsorted_preferred_bytes(int64_t sorted_len, int64_t num_values);
  * bucket is found once, and each needle then searches only its bucket
  * (4 to 8 elements when the keys spread over their range and the workspace
  * is the preferred one; clustered keys fall back to the sampled search of
- * tcs_searchsorted, and a haystack of at most 16384 elements is searched
- * whole in LDS).  Many needles (above 2^19 to 3 * 2^20, the more the shorter
- * the haystack) are instead grouped by slices of the haystack, in batches
+ * tcs_searchsorted, which few needles, short haystacks and very long ones
+ * take at once).  Many needles (above 2^19 to 3 * 2^20, the more the shorter
+ * the haystack; above one for 256 elements from 2^25 elements on)
+ * are instead grouped by slices of the haystack, in batches
  * that the workspace holds, with `out` as scratch.  Results identical to
  * tcs_searchsorted.  `workspace` is scratch that this call overwrites
  * from its first byte (any contents before, nothing kept after): it must

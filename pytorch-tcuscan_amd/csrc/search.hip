@@ -682,9 +682,13 @@ __global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8)))
 // sweep; 2^18 elements: 2^22 needles 46 and 47, 2^23 83 and 69; 2^20 elements:
 // 2^21 needles 35 and 44, 2^22 60 and 48; 2^21: 2^20 32 and 34, 2^21 52 and
 // 44; 2^22 and above: 2^19 27 and 27, 2^20 41 and 33).
+// From kSwLongLen elements on the sampled search is taken up to one needle for
+// kSwLongShare elements (searchsorted_sampled), and the slices beyond.
 constexpr int64_t kSwMinLen = (int64_t)1 << 16;
+constexpr int64_t kSwLongLen = (int64_t)1 << 25, kSwLongShare = 256;
 static int64_t sweep_min_needles(int64_t len) {
   if (len <= (int64_t)1 << 20) return (int64_t)3 << 20;
+  if (len > kSwLongLen) return len / kSwLongShare;
   return len <= (int64_t)1 << 21 ? (int64_t)1 << 20 : (int64_t)1 << 19;
 }
 
@@ -724,13 +728,28 @@ static int64_t sweep_tiles(int64_t len, int64_t nv, size_t bytes) {
 }
 
 // Whether the needles are too few to pay for staging samples in every
-// workgroup, or for a table (us, sixteen lanes and the other way; 2^16
-// needles into 2^16 elements: 7.4 and 9.1 sampled, 2^17 needles 12.2 and 9.2;
-// 2^16 into 2^20 11.4 and 11.2 with a table, into 2^22 18.9 and 16.1, into
-// 2^24 28.1 and 31, 2^15 into 2^22 10.8 and 15).
+// workgroup, or for a table.  us, sixteen lanes and the other way: 2^16 needles
+// into 2^16 elements 7.4 and 9.1 sampled, 2^17 needles 12.2 and 9.2; 2^16 into
+// 2^18 9.9 and 10.0 by a table, 8.7 and 17.2 where the elements are clustered;
+// into 2^21 16.9 and 13.1, clustered 12.9 and 33; into 2^24 28 and 30.  A
+// needle's fifteen lines a step are the more, the less of the haystack the
+// caches hold: 2^15 into 5e7 elements 26.6 and 30.8 sampled, 2^16 49 and 31; 2^15
+// into 2e8 42 and 32.
 static bool searchsorted_few(int64_t len, int64_t nv) {
-  const bool mid = len > ((int64_t)1 << 18) && len <= ((int64_t)1 << 22);
-  return nv <= (mid ? (int64_t)1 << 15 : (int64_t)1 << 16);
+  const int64_t k = (int64_t)1 << 13;
+  return nv <= (len <= (int64_t)1 << 24 ? 8 * k : len <= (int64_t)1 << 26 ? 5 * k : len <= (int64_t)1 << 27 ? 4 * k : 2 * k);
+}
+
+// Whether the sampled search is taken where there is a workspace too: few
+// needles into a haystack not much longer than the samples (2^17 into 65537
+// elements 7.3 us, 9.2 by a table), and haystacks that cost more to read, for
+// a table or by slices, than their needles to search (us, sampled, by a
+// table, by slices; 2^18 needles into 5e7 elements 61, 75, 58, clustered 51, 121,
+// 50; 2^18 into 1.3e8 70, 195, 136; 2^19 into 2e8 135, 307, 181, 2^20 239, 337,
+// 198).
+static bool searchsorted_sampled(int64_t len, int64_t nv) {
+  if (len <= kSsNodes || (len <= (int64_t)3 << 15 && nv <= (int64_t)1 << 17)) return true;
+  return len > kSwLongLen && nv <= len / kSwLongShare;
 }
 
 // Workgroups for `rows` rows of kSsThreads needles: one for each CU of the
@@ -803,6 +822,7 @@ size_t tcs_searchsorted_preferred_bytes(int64_t sorted_len, int64_t num_values) 
   if (sorted_len <= 0) return 0;
   const int64_t nt = sweep_tiles(sorted_len, num_values, SIZE_MAX);
   const size_t least = tcs_searchsorted_workspace_bytes(sorted_len);
+  if (searchsorted_few(sorted_len, num_values) || searchsorted_sampled(sorted_len, num_values)) return least;
   if (nt > 0) {
     const size_t sweep = sweep_layout(sorted_len, nt).end;
     return sweep > least ? sweep : least;
@@ -843,8 +863,7 @@ int tcs_searchsorted_indexed(const int32_t* sorted, int64_t sorted_len, const in
   if (!values || !out || (sorted_len > 0 && !sorted)) return TCS_ERR_INVALID_ARG;
   if (sorted_len == 0) return tcs_searchsorted(sorted, sorted_len, values, out, num_values, stream);
   if (!workspace || workspace_bytes < tcs_searchsorted_workspace_bytes(sorted_len)) return TCS_ERR_WORKSPACE;
-  // A haystack that fits in LDS needs no table.
-  if (sorted_len <= kSsNodes || searchsorted_few(sorted_len, num_values))
+  if (searchsorted_few(sorted_len, num_values) || searchsorted_sampled(sorted_len, num_values))
     return tcs_searchsorted(sorted, sorted_len, values, out, num_values, stream);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t nt = sweep_tiles(sorted_len, num_values, workspace_bytes);
