@@ -76,10 +76,13 @@ __device__ __forceinline__ int32_t lower_bound_in(const int32_t* __restrict__ so
 // samples.  2^24 needles into 2^14 elements: 40.7 us (4.1e11 needles a
 // second; bound by the steps' LDS reads), 187 with one needle a thread at a
 // time and a sorted array of samples.
-template <int U>
+//
+// narrow(key, lo, hi) may move the ends of the window [lo, hi] that the answer
+// lies in closer together.
+template <int U, class F>
 __device__ __forceinline__ void search_staged(int32_t* s_tree, const int32_t* __restrict__ sorted, int32_t len,
                                               const int32_t* __restrict__ values, int32_t* __restrict__ out,
-                                              int64_t nv) {
+                                              int64_t nv, F narrow) {
   if (len == 0) {
     for (int64_t i = (int64_t)blockIdx.x * kSsThreads + threadIdx.x; i < nv; i += (int64_t)gridDim.x * kSsThreads)
       out[i] = 0;
@@ -103,9 +106,10 @@ __device__ __forceinline__ void search_staged(int32_t* s_tree, const int32_t* __
       int32_t lo = c[u];
       if (B > 1 && lo > 0) {
         // sorted[(c - 1) B] < key <= sorted[c B].
-        const int64_t hi = (int64_t)c[u] * B < len ? (int64_t)c[u] * B : len;
+        int32_t hi = (int64_t)c[u] * B < len ? c[u] * B : len;
         lo = (c[u] - 1) * B + 1;
-        lo = lower_bound_in(sorted, lo, (int32_t)hi - lo, key[u]);
+        narrow(key[u], lo, hi);
+        lo = lower_bound_in(sorted, lo, hi - lo, key[u]);
       }
       if (i + u * stride < nv) out[i + u * stride] = lo;
     }
@@ -118,7 +122,7 @@ __global__ __launch_bounds__(kSsThreads) void searchsorted_kernel(const int32_t*
                                                                   const int32_t* __restrict__ values,
                                                                   int32_t* __restrict__ out, int64_t nv) {
   __shared__ int32_t s_tree[kSsNodes];
-  search_staged<U>(s_tree, sorted, len, values, out, nv);
+  search_staged<U>(s_tree, sorted, len, values, out, nv, [](int32_t, int32_t&, int32_t&) {});
 }
 
 // ---------------------------------------------------------------------------
@@ -169,6 +173,12 @@ __global__ __launch_bounds__(kSfThreads) void searchsorted_few_kernel(const int3
 // ---------------------------------------------------------------------------
 constexpr int kSsBuildBlocks = 512;  // build workgroups: one count word each, before the table
 constexpr int32_t kSsWide = 64;
+// From this length on the sampled search that the table falls back to also
+// looks its window up in the table: between two samples lie 512 elements and
+// more, in a bucket often fewer (2^24 needles into 2^24 clustered elements with
+// the least workspace: 1524 us by samples alone, 626 so, 644 by a search of
+// every bucket of up to 2048; 2^19 with the preferred one 108, 73, 133).
+constexpr int32_t kSsNarrowLen = 1 << 22;
 constexpr int kSsLongGaps = 256;     // table gaps above kSsLongGap: at most 2^22 / kSsLongGap in all
 constexpr uint32_t kSsLongGap = 16384;
 
@@ -279,7 +289,7 @@ __global__ __launch_bounds__(kSsThreads) void bucket_start_kernel(const int32_t*
     for (uint32_t k = s_first[q] + threadIdx.x; k < s_last[q]; k += kSsThreads) start[k] = s_at[q];
   }
   if (threadIdx.x == 0) {
-    wide[blockIdx.x] = s_wide;
+    if (wide) wide[blockIdx.x] = s_wide;
     if (blockIdx.x == 0) start[m.used] = len;
   }
 }
@@ -364,9 +374,19 @@ __global__ __launch_bounds__(kSsThreads) void searchsorted_indexed_kernel(const 
   const BucketMap m = bucket_map(sorted, len, bits);
   const int64_t stride = (int64_t)gridDim.x * kSsThreads;
   const int64_t first = (int64_t)blockIdx.x * kSsThreads + threadIdx.x;
-  if (bucket_clustered(wide, len, m, s_tree)) {
+  if (!wide || bucket_clustered(wide, len, m, s_tree)) {
     __syncthreads();  // the sum has been read
-    search_staged<kSsU>(s_tree, sorted, len, values, out, nv);
+    if (len < kSsNarrowLen) {
+      search_staged<kSsU>(s_tree, sorted, len, values, out, nv, [](int32_t, int32_t&, int32_t&) {});
+    } else {
+      search_staged<kSsU>(s_tree, sorted, len, values, out, nv, [&](int32_t key, int32_t& lo, int32_t& hi) {
+        const uint32_t o = order_key(key);
+        if (o < m.umin || o > m.umax) return;
+        const i32x2u se = *reinterpret_cast<const i32x2u*>(start + ((o - m.umin) >> m.shift));
+        lo = lo > se[0] ? lo : se[0];
+        hi = hi < se[1] ? hi : se[1];
+      });
+    }
     return;
   }
   for (int64_t i = first; i < nv; i += stride * kSsU) {
@@ -759,7 +779,9 @@ static bool searchsorted_sampled(int64_t len, int64_t nv) {
 // 16.4 us with one needle a thread, 7.4 with four; 2^20 into 2^20 clustered
 // elements, by the table's sampled search: 99 and 49; 2^24 into 2^18: 297 us
 // with four workgroups a CU, 283 with two).
-static uint32_t searchsorted_grid(uint64_t rows) {
+// The sampled search of many needles with reads past the samples takes four a
+// CU, which even out the tail (2^24 into 16385 elements: 60 us with two, 56).
+static uint32_t searchsorted_grid(uint64_t rows, bool reads) {
   static std::atomic<int> cached[kMaxCachedDevices];
   const uint64_t cus = (uint64_t)device_cached(cached, [](int dev) {
     int n = 0;
@@ -767,7 +789,8 @@ static uint32_t searchsorted_grid(uint64_t rows) {
     return n;
   });
   const uint64_t few = rows < cus ? rows : cus, need = (rows + kSsU - 1) / kSsU;
-  return (uint32_t)(need < few ? few : (need < 2 * cus ? need : 2 * cus));
+  const uint64_t cap = reads && need >= 16 * cus ? 4 * cus : 2 * cus;
+  return (uint32_t)(need < few ? few : (need < cap ? need : cap));
 }
 
 }  // namespace tcs
@@ -791,7 +814,7 @@ int tcs_searchsorted(const int32_t* sorted, int64_t sorted_len, const int32_t* v
   // three copies of it would be LDS reads as well (2^18 needles into 2^14: 7.1
   // us with four, 5.9 with one; 2^19 7.1 and 7.9).
   const uint64_t rows = (uint64_t)((num_values + kSsThreads - 1) / kSsThreads);
-  const uint32_t blocks = searchsorted_grid(rows);
+  const uint32_t blocks = searchsorted_grid(rows, sorted_len > kSsNodes);
   hipLaunchKernelGGL(blocks == rows ? searchsorted_kernel<1> : searchsorted_kernel<kSsU>, dim3(blocks),
                      dim3(kSsThreads), 0, static_cast<hipStream_t>(stream), sorted, (int32_t)sorted_len, values, out,
                      num_values);
@@ -874,17 +897,24 @@ int tcs_searchsorted_indexed(const int32_t* sorted, int64_t sorted_len, const in
     }
     return TCS_OK;
   }
-  const int64_t entries = (int64_t)(workspace_bytes / sizeof(int32_t)) - kSsBuildBlocks - 1;
-  const int bits = clamp_int(bucket_bits(sorted_len), 1, floor_log2(entries));
-  auto* wide = static_cast<int32_t*>(workspace);
-  int32_t* start = wide + kSsBuildBlocks;
+  // The counts before the table; where they would halve it (the least
+  // workspace) and buckets are wide by then, the table alone, every needle
+  // by samples and table (2^24 needles into 2^26 elements: 3307 us with the
+  // counts, 1703 without; into 2^24, of 32 a bucket: 1023 and 1056).
+  const int64_t entries = (int64_t)(workspace_bytes / sizeof(int32_t)) - 1;
+  const int most = clamp_int(bucket_bits(sorted_len), 1, floor_log2(entries));
+  const int counted = clamp_int(most, 1, floor_log2(entries - kSsBuildBlocks));
+  const bool alone = counted < most && sorted_len >= kSsNarrowLen && (sorted_len >> counted) > kSsWide / 2;
+  const int bits = alone ? most : counted;
+  auto* wide = alone ? nullptr : static_cast<int32_t*>(workspace);
+  int32_t* start = static_cast<int32_t*>(workspace) + (alone ? 0 : kSsBuildBlocks);
   const int32_t len = (int32_t)sorted_len;
   const int64_t per_block = (sorted_len + kSsBuildBlocks - 1) / kSsBuildBlocks;
   hipLaunchKernelGGL(bucket_start_kernel, dim3(kSsBuildBlocks), dim3(kSsThreads), 0, st, sorted, len, per_block, bits,
                      wide, start);
   TCS_CHECK_LAUNCH();
   hipLaunchKernelGGL(searchsorted_indexed_kernel,
-                     dim3(searchsorted_grid((uint64_t)((num_values + kSsThreads - 1) / kSsThreads))), dim3(kSsThreads), 0, st,
+                     dim3(searchsorted_grid((uint64_t)((num_values + kSsThreads - 1) / kSsThreads), false)), dim3(kSsThreads), 0, st,
                      sorted, len, bits, wide, start, values, out, num_values);
   TCS_CHECK_LAUNCH();
   return TCS_OK;

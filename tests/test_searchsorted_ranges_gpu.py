@@ -90,3 +90,23 @@ def test_one_needle_a_thread(ops, dev, n, m):
     v = torch.randint(I32_MIN, I32_MAX, (m,), generator=g, device=dev, dtype=torch.int32)
     v[: m // 2] = hay[torch.randint(0, n, (m // 2,), generator=g, device=dev)]
     assert torch.equal(ops.run_searchsorted(hay, v), torch.searchsorted(hay, v, out_int32=True))
+
+
+@pytest.mark.parametrize("n", [1 << 22, (1 << 22) - 1, (1 << 24) + 1, (1 << 25) + 5])
+@pytest.mark.parametrize("kind", ["uniform", "clustered", "two_runs"])
+def test_least_workspace_of_long_haystacks(lib, dev, n, kind):
+    """The table in the least workspace: wide buckets, searched by samples and
+    table together from 2^22 elements on, without the counts above 2^24."""
+    g = torch.Generator(device=dev).manual_seed(n)
+    hay = torch.randint(I32_MIN, I32_MAX, (n,), generator=g, device=dev, dtype=torch.int32)
+    if kind == "clustered":
+        hay = (hay.double() / 2**31).pow(9).mul(2**31).int()
+    elif kind == "two_runs":
+        hay = torch.where(hay < 0, -5, 2**30).int()
+        hay[:3] = torch.tensor([I32_MIN, 7, I32_MAX], dtype=torch.int32)
+    hay = hay.sort().values
+    v = torch.randint(I32_MIN, I32_MAX, (300_001,), generator=g, device=dev, dtype=torch.int32)
+    v[:100_000] = hay[torch.randint(0, n, (100_000,), generator=g, device=dev)]
+    v[-6:] = torch.tensor([I32_MIN, I32_MAX, -5, -4, 2**30, 2**30 + 1], dtype=torch.int32)
+    got = _indexed(lib, hay, v, lib.tcs_searchsorted_workspace_bytes(n))
+    assert torch.equal(got, torch.searchsorted(hay, v, out_int32=True))
