@@ -414,6 +414,10 @@ __global__ __launch_bounds__(kSsThreads) void searchsorted_indexed_kernel(const 
 //            many need, searches them in LDS and writes the answers in their
 //            place;
 //   unsplit: a tile's answers back to the needles' order.
+// A tile whose needles are all in one slice (needles in order, few values) is
+// answered by the split, its groups empty (2^24 needles in order into 2^20
+// elements: 163 us through all four kernels, 100 so, 144 by a table of the
+// bounds).
 // All memory is read and written in runs of a group (64 bytes for 2^24
 // elements) or longer, where a search per needle reads a line of the haystack
 // and one of a table for each.  Slices hold equal numbers of elements and
@@ -425,7 +429,17 @@ __global__ __launch_bounds__(kSsThreads) void searchsorted_indexed_kernel(const 
 // ---------------------------------------------------------------------------
 constexpr int kSwThreads = kSsThreads, kSwRows = 16, kSwTile = kSwThreads * kSwRows;
 constexpr int kSwSlices = 1024, kSwSamples = kSsNodes;
-constexpr int kSwShare = 20480;  // most needles of a share
+// Most needles of a share (us with 10240, 20480 and 40960 at most: 2^24 random
+// needles into 2^24 elements 179, 162, 162, clustered ones 173, 166, 173, into 2^22
+// 142, 130, 125; 2^23 into 98304 79, 72, 75); and where there are few slices, of a slice with few
+// needles left (the split has answered the rest), which would keep one
+// compute unit busy and the others waiting (2^22 needles in order into 98305
+// elements: sweep 15.7 us, 8.8 so).
+constexpr int kSwShare = 20480, kSwFewSlices = 16, kSwFewNeedles = 65536, kSwFewShare = 4096;
+__host__ __device__ constexpr int32_t sweep_shares(int32_t needles, int nb) {
+  const int32_t share = nb <= kSwFewSlices && needles <= kSwFewNeedles ? kSwFewShare : kSwShare;
+  return (needles + share - 1) / share;
+}
 
 // Inclusive maximum scan over a wave's lanes of values >= 0.
 __device__ __forceinline__ int32_t wave_incl_max(int32_t v) {
@@ -456,13 +470,25 @@ __device__ __forceinline__ int32_t sw_block_scan(int32_t v, int32_t* s_w, int32_
   return before;
 }
 
+// The lower bound of a key of the slice from element e0 that c samples lie
+// below: with B = 1, no more than the samples (c is 0 in slice 0 only),
+// otherwise between samples c - 1 and c.
+__device__ __forceinline__ int32_t slice_answer(const int32_t* __restrict__ sorted, int32_t len, int32_t B, int64_t e0,
+                                                int32_t c, int32_t key) {
+  if (B == 1 || c == 0) return (int32_t)e0 + c;
+  const int64_t l = e0 + (int64_t)(c - 1) * B + 1;
+  const int64_t hi = l + B - 1 < len ? l + B - 1 : len;
+  return lower_bound_in(sorted, (int32_t)l, (int32_t)(hi - l), key);
+}
+
 __global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8))) void searchsorted_split_kernel(
     const int32_t* __restrict__ sorted, int64_t slice, int nb, int log, const int32_t* values, int32_t* out,
-    int64_t nv, uint16_t* __restrict__ pos, uint16_t* __restrict__ start) {
-  __shared__ int32_t s_key[kSwTile];
+    int64_t nv, uint16_t* __restrict__ pos, uint16_t* __restrict__ start, int32_t len, int32_t B) {
+  __shared__ int32_t s_key[kSwTile];  // or the samples of the one slice that all needles are in
   __shared__ int32_t s_tree[kSwSlices];
   __shared__ int32_t s_cnt[kSwSlices + 1];
   __shared__ int32_t s_w[kSwThreads / kWave];
+  __shared__ int32_t s_one;
   const int tid = threadIdx.x;
   stage_tree(s_tree, log, sorted + slice, slice, nb - 1);
   const int64_t t0 = (int64_t)blockIdx.x * kSwTile;
@@ -471,7 +497,10 @@ __global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8)))
   out += t0;
   pos += t0;
   s_cnt[tid] = 0;
-  if (tid == 0) s_cnt[kSwSlices] = 0;
+  if (tid == 0) {
+    s_cnt[kSwSlices] = 0;
+    s_one = -1;
+  }
   int32_t key[kSwRows], br[kSwRows];  // slice << 16 | rank in it (in no particular order)
 #pragma unroll
   for (int i = 0; i < kSwRows; ++i) {
@@ -490,13 +519,46 @@ __global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8)))
     for (int u = 0; u < 4; ++u) {
       // Rows past the end count in a word of their own.
       const int32_t b = (i + u) * kSwThreads + again < tvalid ? c4[u] : kSwSlices;
-      br[i + u] = b << 16 | atomicAdd(&s_cnt[b], 1);
+      // A wave whose needles are in one slice (needles in order) counts them
+      // with one add: 64 to one word follow one another.
+      const int32_t b0 = __builtin_amdgcn_readfirstlane(b);
+      if (__ballot(b != b0) == 0) {
+        int32_t at = 0;
+        if (__lane_id() == 0) at = atomicAdd(&s_cnt[b0], kWave);
+        br[i + u] = b << 16 | (__builtin_amdgcn_readfirstlane(at) + (int32_t)__lane_id());
+      } else {
+        br[i + u] = b << 16 | atomicAdd(&s_cnt[b], 1);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
   int32_t all;
+  if (s_cnt[tid] == tvalid) s_one = tid;
   const int32_t first = sw_block_scan(s_cnt[tid], s_w, &all);
+  if (s_one >= 0) {
+    // All needles in one slice (needles in order, or few values): answered
+    // here, the slice's samples in the place of the needles.  The tile's groups
+    // are empty, starting at its end, which unsplit knows it by.
+    if (tid < nb) start[(int64_t)blockIdx.x * nb + tid] = (uint16_t)tvalid;
+    const int64_t e0 = (int64_t)s_one * slice, rest = (len - e0 + B - 1) / B;
+    stage_tree(s_key, kSsLog, sorted + e0 + B, B, (int32_t)(rest < kSwSamples ? rest : kSwSamples) - 1);
+    const int32_t least = sorted[e0];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSwRows; i += 4) {
+      const int32_t k4[4] = {key[i], key[i + 1], key[i + 2], key[i + 3]};
+      int32_t c4[4];
+      tree_count<4>(s_key, kSsLog, k4, c4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int32_t lo = slice_answer(sorted, len, B, e0, c4[u] + (least < k4[u] ? 1 : 0), k4[u]);
+        const int p = (i + u) * kSwThreads + tid;
+        if (p < tvalid) out[p] = lo;
+      }
+    }
+    return;
+  }
   s_cnt[tid] = first;
   if (tid == 0) s_cnt[kSwSlices] = tvalid;
   if (tid < nb) start[(int64_t)blockIdx.x * nb + tid] = (uint16_t)first;
@@ -554,7 +616,7 @@ __global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8)))
   const int tid = threadIdx.x, lane = __lane_id(), wid = tid / kWave;
   if (tid == 0) s_shares = 0;
   const int32_t tot = tid < nb ? total[tid] : 0;
-  const int32_t shares = (tot + kSwShare - 1) / kSwShare;
+  const int32_t shares = sweep_shares(tot, nb);
   int32_t all;
   const int32_t before = sw_block_scan(shares, s_w, &all);
   const int32_t me = (int32_t)blockIdx.x - before;
@@ -653,14 +715,7 @@ __global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8)))
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       c[u] += first < key[u] ? 1 : 0;  // samples below the needle
-      // Elements below it: B = 1, no more than the samples (c is 0 in slice 0
-      // only); otherwise between samples c - 1 and c.
-      int32_t lo = (int32_t)e0 + c[u];
-      if (B > 1 && c[u] > 0) {
-        const int64_t l = e0 + (int64_t)(c[u] - 1) * B + 1;
-        const int64_t hi = l + B - 1 < len ? l + B - 1 : len;
-        lo = lower_bound_in(sorted, (int32_t)l, (int32_t)(hi - l), key[u]);
-      }
+      const int32_t lo = slice_answer(sorted, len, B, e0, c[u], key[u]);
       if (at[u] >= 0) out[at[u]] = lo;
       if (more) {
         at[u] = nat[u];
@@ -671,11 +726,12 @@ __global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8)))
 }
 
 __global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8))) void searchsorted_unsplit_kernel(
-    const uint16_t* __restrict__ pos, int32_t* __restrict__ out, int64_t nv) {
+    const uint16_t* __restrict__ pos, const uint16_t* __restrict__ start, int nb, int32_t* __restrict__ out, int64_t nv) {
   __shared__ int32_t s_r[kSwTile];
   const int tid = threadIdx.x;
   const int64_t t0 = (int64_t)blockIdx.x * kSwTile;
   const int tvalid = t0 + kSwTile <= nv ? kSwTile : (int)(nv - t0);
+  if (start[(int64_t)blockIdx.x * nb] != 0) return;  // the split has answered the tile
   int32_t r[kSwRows];
   uint32_t q[kSwRows];
 #pragma unroll
@@ -699,14 +755,16 @@ __global__ __launch_bounds__(kSwThreads) __attribute__((amdgpu_waves_per_eu(8)))
 
 // The sweep from these sizes on; below, its four launches and the slices read
 // by workgroups with few needles cost more than a table does (us, table and
-// sweep; 2^18 elements: 2^22 needles 46 and 47, 2^23 83 and 69; 2^20 elements:
-// 2^21 needles 35 and 44, 2^22 60 and 48; 2^21: 2^20 32 and 34, 2^21 52 and
-// 44; 2^22 and above: 2^19 27 and 27, 2^20 41 and 33).
+// sweep; 65537 elements: 2^22 needles 41 and 50, in order 16 and 37, 2^24 143 and
+// 131; 2^18: 2^22 needles 46 and 47, 2^23 83 and 69; 2^20: 2^21 needles 35 and 44,
+// 2^22 60 and 48; 2^21: 2^20 32 and 34, 2^21 52 and 44; 2^22 and above: 2^19 27 and
+// 27, 2^20 41 and 33).
 // From kSwLongLen elements on the sampled search is taken up to one needle for
 // kSwLongShare elements (searchsorted_sampled), and the slices beyond.
 constexpr int64_t kSwMinLen = (int64_t)1 << 16;
 constexpr int64_t kSwLongLen = (int64_t)1 << 25, kSwLongShare = 256;
 static int64_t sweep_min_needles(int64_t len) {
+  if (len <= (int64_t)3 << 15) return (int64_t)6 << 20;
   if (len <= (int64_t)1 << 20) return (int64_t)3 << 20;
   if (len > kSwLongLen) return len / kSwLongShare;
   return len <= (int64_t)1 << 21 ? (int64_t)1 << 20 : (int64_t)1 << 19;
@@ -864,16 +922,19 @@ static int sweep_batch(const int32_t* sorted, int64_t len, const int32_t* values
   auto* start = reinterpret_cast<uint16_t*>(w + l.start);
   auto* pos = reinterpret_cast<uint16_t*>(w + l.pos);
   hipLaunchKernelGGL(searchsorted_split_kernel, dim3((uint32_t)nt), dim3(kSwThreads), 0, st, sorted,
-                     (int64_t)kSwSamples * l.B, l.nb, l.log, values, out, nv, pos, start);
+                     (int64_t)kSwSamples * l.B, l.nb, l.log, values, out, nv, pos, start, (int32_t)len, l.B);
   TCS_CHECK_LAUNCH();
   hipLaunchKernelGGL(searchsorted_columns_kernel, dim3(l.nb), dim3(kSwThreads), 0, st, start, l.nb, (int)nt, nv, groups,
                      total);
   TCS_CHECK_LAUNCH();
-  // At most one share more than full ones for each slice.
-  hipLaunchKernelGGL(searchsorted_sweep_kernel, dim3((uint32_t)(l.nb + nv / kSwShare)), dim3(kSwThreads), 0, st, sorted,
+  // At most one share more than full ones for each slice, and those of a slice
+  // with few needles.
+  const int64_t more = l.nb <= kSwFewSlices ? kSwFewNeedles / kSwFewShare : 1;
+  hipLaunchKernelGGL(searchsorted_sweep_kernel, dim3((uint32_t)(l.nb * more + nv / kSwShare)), dim3(kSwThreads), 0, st, sorted,
                      (int32_t)len, l.B, l.nb, (int)nt, groups, total, out);
   TCS_CHECK_LAUNCH();
-  hipLaunchKernelGGL(searchsorted_unsplit_kernel, dim3((uint32_t)nt), dim3(kSwThreads), 0, st, pos, out, nv);
+  hipLaunchKernelGGL(searchsorted_unsplit_kernel, dim3((uint32_t)nt), dim3(kSwThreads), 0, st, pos, start, l.nb,
+                     out, nv);
   TCS_CHECK_LAUNCH();
   return TCS_OK;
 }

@@ -110,3 +110,29 @@ def test_least_workspace_of_long_haystacks(lib, dev, n, kind):
     v[-6:] = torch.tensor([I32_MIN, I32_MAX, -5, -4, 2**30, 2**30 + 1], dtype=torch.int32)
     got = _indexed(lib, hay, v, lib.tcs_searchsorted_workspace_bytes(n))
     assert torch.equal(got, torch.searchsorted(hay, v, out_int32=True))
+
+
+@pytest.mark.parametrize("n,m", [((1 << 16) + 1, (6 << 20) + 1), ((7 << 14) + 1, (3 << 20) + 1), ((7 << 14) + 16384, (1 << 24) + 16385),
+                                 ((1 << 22) + 3, (1 << 20) + 16383), ((1 << 25) + 16386, 700_001)])
+@pytest.mark.parametrize("needles", ["ordered", "one", "one_but_a_few", "above", "below", "two_halves"])
+def test_tiles_of_one_slice(ops, dev, n, m, needles):
+    """Tiles whose needles all lie in one slice, which are answered without the
+    sweep, beside tiles that are not, and a last tile of one needle and of
+    one less than a tile; in place too."""
+    g = torch.Generator(device=dev).manual_seed(n + m)
+    hay = torch.randint(I32_MIN, I32_MAX, (n,), generator=g, device=dev, dtype=torch.int32).sort().values
+    v = torch.randint(I32_MIN, I32_MAX, (m,), generator=g, device=dev, dtype=torch.int32)
+    if needles == "ordered":
+        v = v.sort().values
+    elif needles in ("one", "one_but_a_few"):
+        v[:] = hay[n // 2]
+        if needles == "one_but_a_few":
+            v[::100_003] = hay[n // 5]
+    elif needles == "above":
+        hay, v = hay // 2, torch.full_like(v, I32_MAX)
+    elif needles == "below":
+        hay, v = hay // 2, torch.full_like(v, I32_MIN)
+    else:
+        v[: m // 2] = hay[n // 3]
+    exp = torch.searchsorted(hay, v, out_int32=True)
+    assert torch.equal(ops.run_searchsorted(hay, v), exp)
