@@ -202,7 +202,7 @@ __device__ __forceinline__ BucketMap bucket_map(const int32_t* __restrict__ sort
 }
 
 // The table in one pass over the haystack: element i starts the buckets after
-// its predecessor's up to its own (2^24 elements 24 us; a search per entry took
+// its predecessor's up to its own (2^24 elements 25 us; a search per entry took
 // 86).  A wave takes 256 consecutive elements at a time, four rows of 64, so an element's predecessor is the lane's below
 // (or the last lane's of the row before) and the element 64 places back the
 // lane's own of the row before.  Few buckets start at one element as a rule;
@@ -252,8 +252,9 @@ __global__ __launch_bounds__(kSsThreads) void bucket_start_kernel(const int32_t*
       const uint32_t above = (uint32_t)readlane((int)b[j - 1], kWave - 1);
       const uint32_t prev = lane > 0 ? left : above;
       const uint32_t first = p == 0 ? 0u : prev + 1u;
-      // Entries [first, first + gap) start here; none after a bucket above.
-      const uint32_t gap = p < b1 && b[j] >= first ? b[j] + 1u - first : 0u;
+      // Entries [first, first + gap) start here; below zero after a bucket
+      // above, which the comparisons take for a long gap.
+      const uint32_t gap = p < b1 ? b[j] + 1u - first : 0u;
       nwide += p < b1 && p >= kSsWide && b[j - 1] == b[j] ? 1 : 0;
       if (gap <= 8u) {
         for (uint32_t k = 0; k < gap; ++k) start[first + k] = (int32_t)p;
@@ -263,6 +264,7 @@ __global__ __launch_bounds__(kSsThreads) void bucket_start_kernel(const int32_t*
         const int l = __builtin_ctzll(more);
         more &= more - 1;
         const uint32_t f = (uint32_t)readlane((int)first, l), g = (uint32_t)readlane((int)gap, l);
+        if ((int32_t)g <= 0) continue;  // buckets are at most 2^22
         const int32_t at = (int32_t)(w + (j - 1) * kWave) + l;
         if (g > kSsLongGap) {
           int q = 0;
@@ -819,14 +821,14 @@ static bool searchsorted_few(int64_t len, int64_t nv) {
 }
 
 // Whether the sampled search is taken where there is a workspace too: few
-// needles into a haystack not much longer than the samples (2^17 into 65537
-// elements 7.3 us, 9.2 by a table), and haystacks that cost more to read, for
+// needles into a haystack not much longer than the samples (2^18 into 65537
+// elements 8.4 us, 9.6 by a table), and haystacks that cost more to read, for
 // a table or by slices, than their needles to search (us, sampled, by a
 // table, by slices; 2^18 needles into 5e7 elements 61, 75, 58, clustered 51, 121,
 // 50; 2^18 into 1.3e8 70, 195, 136; 2^19 into 2e8 135, 307, 181, 2^20 239, 337,
 // 198).
 static bool searchsorted_sampled(int64_t len, int64_t nv) {
-  if (len <= kSsNodes || (len <= (int64_t)3 << 15 && nv <= (int64_t)1 << 17)) return true;
+  if (len <= kSsNodes || (len <= (int64_t)3 << 15 && nv <= (int64_t)1 << 18)) return true;
   return len > kSwLongLen && nv <= len / kSwLongShare;
 }
 
