@@ -591,7 +591,7 @@ __global__ __launch_bounds__(kSegNW * kWave) void seg_reduce_kernel(
 // row inside the tile is stored, a row cut by the tile's ends is added to
 // (the row pass has zeroed it): integer additions, so any order gives the
 // same sum.  No tile waits for another.  2^26 values in rows
-// of 64: 20 us (3.8 TB/s); the segmented reduction below, bound by its 20
+// of 64: 20 us (3.8 TB/s); the segmented reduction above, bound by its 20
 // instructions a value, took 60.
 constexpr int kSegI8Threads = 512, kSegI8J = 2;
 constexpr int64_t kSegI8Tile = (int64_t)kSegI8Threads * kSegI8J * 16;
@@ -625,8 +625,8 @@ __global__ __launch_bounds__(kSegI8Threads) void seg_sum_i8_kernel(const int8_t*
   if (r_hi > R - 1) r_hi = R - 1;
   // The first rows' ends, before the prefixes are ready.
   const int64_t first = r_lo + tid;
-  int64_t e = first <= r_hi ? row_end(ends, first, n_ends, nnz) : 0;
-  int64_t b = first <= r_hi ? row_end(ends, first - 1, n_ends, nnz) : 0;
+  const int64_t e = first <= r_hi ? row_end(ends, first, n_ends, nnz) : 0;
+  const int64_t b = first <= r_hi ? row_end(ends, first - 1, n_ends, nnz) : 0;
 
 #pragma unroll
   for (int j = 0; j < J; ++j) {
@@ -662,18 +662,41 @@ __global__ __launch_bounds__(kSegI8Threads) void seg_sum_i8_kernel(const int8_t*
     }
     return sum;
   };
-  for (int64_t r = first; r <= r_hi; r += kSegI8Threads) {
-    if (r != first) {
-      e = row_end(ends, r, n_ends, nnz);
-      b = row_end(ends, r - 1, n_ends, nnz);
-    }
+  auto add = [&](int64_t r, int64_t b, int64_t e) {
     const int64_t from = b > t0 ? b : t0, to = e < t1 ? e : t1;
-    if (from >= to) continue;  // empty (zeroed by the row pass), or not in this tile
+    if (from >= to) return;  // empty (zeroed by the row pass), or not in this tile
     const int part = prefix(to) - prefix(from);
     if (b >= t0 && e <= t1) {
       y[r] = part;
     } else {
       atomicAdd(&y[r], part);
+    }
+  };
+  if (first <= r_hi) add(first, b, e);
+  // More rows than threads.  Many (empty ones) four rows' ends in flight (2^22
+  // rows over 100001 values, nearly all empty: 728 us with one, 305 so).
+  if (r_hi - r_lo < 4 * kSegI8Threads) {
+    for (int64_t r = first + kSegI8Threads; r <= r_hi; r += kSegI8Threads)
+      add(r, row_end(ends, r - 1, n_ends, nnz), row_end(ends, r, n_ends, nnz));
+    return;
+  }
+  if (n_ends == 0) return;  // all rows but the first are empty
+  constexpr int U = 4;
+  for (int64_t r = first + kSegI8Threads; r <= r_hi; r += U * kSegI8Threads) {
+    IdxT bu[U], eu[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // Only loads here, of rows that exist: rows from n_ends on end at nnz.
+      const int64_t q = r + u * kSegI8Threads;
+      bu[u] = ends[q - 1 < n_ends ? q - 1 : n_ends - 1];
+      eu[u] = ends[q < n_ends ? q : n_ends - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t q = r + u * kSegI8Threads;
+      const int64_t bq = q - 1 < n_ends && (int64_t)bu[u] < nnz ? (int64_t)bu[u] : nnz;
+      const int64_t eq = q < n_ends && (int64_t)eu[u] < nnz ? (int64_t)eu[u] : nnz;
+      if (q <= r_hi && bq != eq) add(q, bq, eq);
     }
   }
 }
