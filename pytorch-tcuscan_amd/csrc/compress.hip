@@ -514,7 +514,7 @@ __global__ __launch_bounds__(BLOCK) void count_mask_chunks_kernel(const int8_t* 
   constexpr int kPerWave = kChunksPerBlock / kWaves;  // 8 or 2
   constexpr int kBatch = kPerWave < 4 ? kPerWave : 4;
   const int64_t b0 = (int64_t)blockIdx.x * kCountChunk;
-  uint32_t mine = 0;  // lane i keeps the count of chunk wid + 4i
+  uint32_t mine = 0;  // lane i keeps the count of chunk wid + BLOCK / 64 * i
   uint32_t tot = 0;
 #pragma unroll
   for (int i0 = 0; i0 < kPerWave; i0 += kBatch) {
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(BLOCK) void count_keep_chunks_kernel(const XT* __re
   constexpr int kBatch = 2;
   constexpr int kItems = (int)(kChunk / kWave);  // 32 per lane
   const int64_t b0 = (int64_t)blockIdx.x * kCountChunk;
-  uint32_t mine = 0;  // lane i keeps the count of chunk wid + 4i
+  uint32_t mine = 0;  // lane i keeps the count of chunk wid + BLOCK / 64 * i
   uint32_t tot = 0;
 #pragma unroll
   for (int i0 = 0; i0 < kPerWave; i0 += kBatch) {

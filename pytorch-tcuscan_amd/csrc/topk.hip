@@ -16,10 +16,10 @@
 // counting.  If they do not fit (the largest keys lie together), the radix
 // select below runs instead, over the sub-chunks that reach the bound: its
 // kernels are launched behind this path and leave at once when it has
-// succeeded, so nothing waits for the host.  2^28 fp16 normals, k = 2048: 125
-// us, of which the read takes 86, the select's two reads and eleven launches
-// 278; sorted keys, which give too many candidates, 378 against 429 (2^25 of
-// them 138 against 115).
+// succeeded, so nothing waits for the host.  2^28 fp16 normals, k = 2048: 124
+// us, of which the read takes 82, the select's two reads and eleven launches
+// 278; sorted keys, which give too many candidates, 183 against 429 (2^25 of
+// them 89 against 116; fp32 112 against 157).
 //
 // Otherwise radix select: the k-th largest order key T is found one 8-bit
 // digit at a time, from the top: a histogram of digit r over the keys whose
@@ -69,8 +69,8 @@ constexpr int kTkListMax = 16;
 // (their record's mask bits): a selected key is above or matches the
 // higher digits.
 constexpr int64_t kTkSubChunk = 2048;
-// Tiles per histogram chunk: chunks are whole tiles, at most
-// ceil(n / kTkMaxGroups) <= 2^21 keys for n < 2^31, so 256 of 8192.
+// Tiles of a histogram workgroup, in a chunk of whole tiles or (behind a gate)
+// apart: at most ceil(n / kTkMaxGroups) <= 2^21 keys for n < 2^31, so 256 of 8192.
 constexpr int kTkMaxChunkTiles = 256;
 
 inline int64_t topk_tile(int key_bytes) { return (int64_t)kTkNW * (key_bytes <= 2 ? 4 : 2) * kWave * kTkG; }
@@ -81,6 +81,10 @@ constexpr uint32_t kTkCandMax = 8192;  // 64 KiB of LDS
 // Words of the maxima path's state: candidates, the bound's T and P, arrivals
 // and digit counts of the gated launches.
 constexpr int kTkArrived = 8, kTkBins = 64, kTkStateWords = kTkBins + 256;
+// Workgroups of a gated launch: one a CU, so that few arrive at one word (2^25
+// sorted fp32 keys, k = 2048: 112 us with 256, 118 with 512 or 1024; the select
+// before it, with a range of keys a workgroup and every workgroup's digit counts
+// read by the last, 225).
 constexpr uint32_t kTkGatedGroups = 256;
 __device__ __forceinline__ bool topk_done(const uint32_t* gate) { return gate && *gate <= kTkCandMax; }
 
@@ -803,7 +807,7 @@ __global__ __launch_bounds__(256) void topk_pivot_kernel(const uint16_t* __restr
 // sub-chunk's largest order key, gcomp[g] = the group's largest << 32 |
 // ~(its first sub-chunk that holds it).  Reads at the streaming rate: seven
 // packed instructions map two 16-bit keys and one takes their maximum (2^28
-// fp16 keys 94 us, 5.7 TB/s; with plain loads 106).
+// fp16 keys 82 us, 6.5 TB/s; plain loads measured 12 us slower).
 // ---------------------------------------------------------------------------
 constexpr int kTkMaxThreads = 256;
 
