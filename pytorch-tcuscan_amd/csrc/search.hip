@@ -424,8 +424,9 @@ __global__ __launch_bounds__(kSsThreads) void searchsorted_indexed_kernel(const 
 // elements) or longer, where a search per needle reads a line of the haystack
 // and one of a table for each.  Slices hold equal numbers of elements and
 // shares equal numbers of needles, whatever the keys.  2^24 needles into 2^24
-// elements: 161 us (split 51, columns 12, sweep 83, unsplit 27 alone; a table
-// searched by groups of 8192 needles 551).  Split and unsplit run at 3.1 and 5.9
+// elements: 162 us, 172 on inputs that change from call to call (split 47,
+// columns 11, sweep 77, unsplit 27 alone; a table searched by groups of 8192
+// needles 551).  Split and unsplit run at 3.1 and 5.9
 // TB/s; the sweep is bound by its vector instructions (112 a row of 64
 // needles, 70% busy) and by the tree's LDS reads (50% busy).
 // ---------------------------------------------------------------------------
