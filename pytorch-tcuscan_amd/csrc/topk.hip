@@ -1264,7 +1264,9 @@ inline int topk_elem_bytes(int dt) {
 // looks at every group: 9e6 fp32 keys, k = 3000, 67 us with 11719 groups, 78
 // with 16384).  Otherwise groups differ by one sub-chunk, as many at every
 // size: just above a multiple of them equal ones would be half as many, too
-// few for the bound (9e6 fp16 keys, k = 3000: 58 us, 88 by the select).
+// few for the bound (9e6 fp16 keys, k = 3000: 58 us, 88 by the select).  Keys of
+// one byte gain nothing there (k = 2048: 53 us either way) and lose where the
+// winners lie in one region (87, by the select 57).
 constexpr int64_t kTkGroupsPerK = 3;
 struct TopkMaxima {
   int U, per;
@@ -1281,7 +1283,7 @@ inline TopkMaxima topk_maxima(int64_t n, int64_t k, int key_bytes) {
   m.groups = m.subs < most ? m.subs : (uint32_t)most;
   m.per = m.groups > 0 ? (int)((m.subs + m.groups - 1) / m.groups) : 1;
   const int64_t even = (m.subs + m.per - 1) / m.per;
-  if (even >= kTkGroupsPerK * k) m.groups = (uint32_t)even;
+  if (even >= kTkGroupsPerK * k || key_bytes == 1) m.groups = (uint32_t)even;
   return m;
 }
 
